@@ -10,8 +10,8 @@
 //
 // Batched PCG: independent CG recurrences per column (own alpha, beta, convergence flag),
 // FP64 Krylov vectors, flexible beta, the operator's multigrid V-cycle applied to the whole
-// block in FP32.  Column reductions are deterministic: fixed grid, per-block partials, the last
-// block to arrive sums them in a fixed order.
+// block in FP32.  Column reductions are deterministic: fixed grid, per-block partials, summed
+// in a fixed order by a second launch with one block per column.
 #include "sell.h"
 
 namespace mk {
@@ -371,8 +371,8 @@ template void spmm_launch<float>(mk_ctx*, const mk_op*, int, const float*, float
 
 // Per-column partial sums of K quantities of this block (the thread's column is
 // threadIdx.x % MW, blockDim 256, grid <= kBlkParts), stored at
-// partials[(k * 64 + j) * kBlkParts + block].  No fence or ticket: a one-block finishing kernel
-// adds them (colsum_total) after the kernel boundary, in a fixed order.
+// partials[(k * 64 + j) * kBlkParts + block].  No fence or ticket: a finishing kernel with one
+// block per column adds them (colsum_total) after the kernel boundary, in a fixed order.
 template <int K, int MW>
 __device__ __forceinline__ void colsum_write(double (&v)[K], double* partials) {
     __shared__ double sh[K][4][64];
@@ -392,34 +392,30 @@ __device__ __forceinline__ void colsum_write(double (&v)[K], double* partials) {
             partials[(size_t(k) * 64 + t) * kBlkParts + blockIdx.x] = sh[k][0][t] + sh[k][1][t] + sh[k][2][t] + sh[k][3][t];
     }
 }
-// Column totals over nparts blocks (one block of 256 threads): tot[k][j], j < MW, valid in every
-// thread after the call.
-template <int K, int MW>
-__device__ __forceinline__ void colsum_total(const double* __restrict__ partials, int nparts, double (*tot)[64]) {
-    __shared__ double sh[K][4][64];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, j = threadIdx.x % MW;
+// Totals of column j over nparts blocks (one block of 256 threads per column, reading the
+// column's contiguous partials): tot[k], valid in thread 0 after the call.  Fixed order: a
+// thread's partials b, b + 256, ..., then the block's fixed tree.  One block for all columns
+// read the same partials with a stride of kBlkParts: 79 us (one quantity) and 147 us (two) per
+// launch at 64 columns, against 4 us for 64 blocks.
+template <int K>
+__device__ __forceinline__ void colsum_total(const double* __restrict__ partials, int nparts, int j, double (&tot)[K]) {
 #pragma unroll
     for (int k = 0; k < K; k++) {
-        double a = 0.0;
         const double* pk = partials + (size_t(k) * 64 + j) * kBlkParts;
-        for (int b = threadIdx.x / MW; b < nparts; b += 256 / MW) a += pk[b];
-#pragma unroll
-        for (int off = MW; off < 64; off <<= 1) a += __shfl_xor(a, off, 64);
-        if (lane < MW) sh[k][wid][lane] = a;
+        double a = 0.0;
+#pragma unroll 8
+        for (int b = threadIdx.x; b < nparts; b += 256) a += pk[b];
+        tot[k] = a;
     }
-    __syncthreads();
-    if (threadIdx.x < MW) {
-        const int t = threadIdx.x;
-#pragma unroll
-        for (int k = 0; k < K; k++) tot[k][t] = sh[k][0][t] + sh[k][1][t] + sh[k][2][t] + sh[k][3][t];
-    }
-    __syncthreads();
+    block_sum<K>(tot);
 }
 
-__device__ __forceinline__ void bstate_all_done(BState* st, int mw) {
-    int all = 1;
-    for (int j = 0; j < mw; j++) all &= st->done[j];
-    st->all_done = all;
+// Marks column j finished (thread 0 of the column's block, at most once per column and solve);
+// the last of the MW columns raises all_done.
+template <int MW>
+__device__ __forceinline__ void column_done(BState* st, int j) {
+    st->done[j] = 1;
+    if (atomicAdd(&st->ndone, 1) + 1 == MW) st->all_done = 1;
 }
 
 // X = 0 ; R = B ; Rz = ZT(B) (the V-cycle's input copy; none for an FP64 V-cycle) ; bb_j = |B_j|^2
@@ -438,11 +434,11 @@ __global__ void __launch_bounds__(256) bk_init0(size_t len, const double* __rest
 }
 template <int MW>
 __global__ void __launch_bounds__(256) bk_init0_fin(BState* st, const double* __restrict__ partials, int nparts) {
-    __shared__ double tot[1][64];
-    colsum_total<1, MW>(partials, nparts, tot);
-    if (threadIdx.x < MW) {
-        const int j = threadIdx.x;
-        st->bb[j] = tot[0][j];
+    const int j = blockIdx.x;
+    double tot[1];
+    colsum_total<1>(partials, nparts, j, tot);
+    if (threadIdx.x == 0) {
+        st->bb[j] = tot[0];
         st->it[j] = 0;
         st->status[j] = MK_OK;
     }
@@ -463,21 +459,17 @@ __global__ void __launch_bounds__(256) bk_init1(size_t len, const double* __rest
 }
 template <int MW>
 __global__ void __launch_bounds__(256) bk_init1_fin(BState* st, const double* __restrict__ partials, int nparts) {
-    __shared__ double tot[2][64];
-    colsum_total<2, MW>(partials, nparts, tot);
-    {
-        if (threadIdx.x < MW) {
-            const int j = threadIdx.x;
-            const double rz = tot[0][j], rr = tot[1][j];
-            st->rz[j] = rz;
-            st->rr[j] = rr;
-            int d = (rr <= st->tol2 * st->bb[j]) ? 1 : 0;
-            if (!(rz == rz) || !(rr == rr)) { st->status[j] = MK_ERR_NAN; d = 1; }
-            else if (!d && !(rz > 0.0)) { st->status[j] = MK_ERR_NOT_SPD; d = 1; }
-            st->done[j] = d;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) bstate_all_done(st, MW);
+    const int j = blockIdx.x;
+    double tot[2];
+    colsum_total<2>(partials, nparts, j, tot);
+    if (threadIdx.x == 0) {
+        const double rz = tot[0], rr = tot[1];
+        st->rz[j] = rz;
+        st->rr[j] = rr;
+        bool d = rr <= st->tol2 * st->bb[j];
+        if (!(rz == rz) || !(rr == rr)) { st->status[j] = MK_ERR_NAN; d = true; }
+        else if (!d && !(rz > 0.0)) { st->status[j] = MK_ERR_NOT_SPD; d = true; }
+        if (d) column_done<MW>(st, j);
     }
 }
 
@@ -492,17 +484,19 @@ __global__ void __launch_bounds__(256) bk_alpha(size_t len, const double* __rest
 }
 template <int MW>
 __global__ void __launch_bounds__(256) bk_alpha_fin(BState* st, const double* __restrict__ partials, int nparts) {
-    if (st->all_done) return;
-    __shared__ double tot[1][64];
-    colsum_total<1, MW>(partials, nparts, tot);
-    if (threadIdx.x < MW) {
-        const int j = threadIdx.x;
-        const double pq = tot[0][j];
-        if (st->done[j]) { st->alpha[j] = 0.0; }
-        else if (!(pq > 0.0)) {
+    const int j = blockIdx.x;
+    if (st->done[j]) {  // only this block writes done[j]: uniform
+        if (threadIdx.x == 0) st->alpha[j] = 0.0;
+        return;
+    }
+    double tot[1];
+    colsum_total<1>(partials, nparts, j, tot);
+    if (threadIdx.x == 0) {
+        const double pq = tot[0];
+        if (!(pq > 0.0)) {
             st->status[j] = (pq == pq) ? MK_ERR_NOT_SPD : MK_ERR_NAN;
-            st->done[j] = 1;
             st->alpha[j] = 0.0;
+            column_done<MW>(st, j);
         } else {
             st->alpha[j] = st->rz[j] / pq;
         }
@@ -531,22 +525,16 @@ __global__ void __launch_bounds__(256) bk_update(size_t len, double* __restrict_
 }
 template <int MW>
 __global__ void __launch_bounds__(256) bk_update_fin(BState* st, const double* __restrict__ partials, int nparts) {
-    if (st->all_done) return;
-    __shared__ double tot[1][64];
-    colsum_total<1, MW>(partials, nparts, tot);
-    {
-        if (threadIdx.x < MW) {
-            const int j = threadIdx.x;
-            const double rr = tot[0][j];
-            if (!st->done[j]) {
-                st->rr[j] = rr;
-                st->it[j] += 1;
-                if (!(rr == rr)) { st->status[j] = MK_ERR_NAN; st->done[j] = 1; }
-                else if (rr <= st->tol2 * st->bb[j]) st->done[j] = 1;
-            }
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) bstate_all_done(st, MW);
+    const int j = blockIdx.x;
+    if (st->done[j]) return;
+    double tot[1];
+    colsum_total<1>(partials, nparts, j, tot);
+    if (threadIdx.x == 0) {
+        const double rr = tot[0];
+        st->rr[j] = rr;
+        st->it[j] += 1;
+        if (!(rr == rr)) { st->status[j] = MK_ERR_NAN; column_done<MW>(st, j); }
+        else if (rr <= st->tol2 * st->bb[j]) column_done<MW>(st, j);
     }
 }
 
@@ -565,25 +553,19 @@ __global__ void __launch_bounds__(256) bk_beta(size_t len, const double* __restr
 }
 template <int MW>
 __global__ void __launch_bounds__(256) bk_beta_fin(BState* st, const double* __restrict__ partials, int nparts) {
-    if (st->all_done) return;
-    __shared__ double tot[2][64];
-    colsum_total<2, MW>(partials, nparts, tot);
-    {
-        if (threadIdx.x < MW) {
-            const int j = threadIdx.x;
-            if (!st->done[j]) {
-                const double a = tot[0][j];
-                if (!(a > 0.0)) {
-                    st->status[j] = (a == a) ? MK_ERR_NOT_SPD : MK_ERR_NAN;
-                    st->done[j] = 1;
-                } else {
-                    st->beta[j] = (a - tot[1][j]) / st->rz[j];
-                    st->rz[j] = a;
-                }
-            }
+    const int j = blockIdx.x;
+    if (st->done[j]) return;
+    double tot[2];
+    colsum_total<2>(partials, nparts, j, tot);
+    if (threadIdx.x == 0) {
+        const double a = tot[0];
+        if (!(a > 0.0)) {
+            st->status[j] = (a == a) ? MK_ERR_NOT_SPD : MK_ERR_NAN;
+            column_done<MW>(st, j);
+        } else {
+            st->beta[j] = (a - tot[1]) / st->rz[j];
+            st->rz[j] = a;
         }
-        __syncthreads();
-        if (threadIdx.x == 0) bstate_all_done(st, MW);
     }
 }
 
@@ -602,6 +584,7 @@ __global__ void __launch_bounds__(256) bk_pupdate(size_t len, double* __restrict
 __global__ void k_set_bstate(BState* st, double tol2) {
     st->tol2 = tol2;
     st->all_done = 0;
+    st->ndone = 0;
 }
 
 // ZT: the V-cycle's precision (float: FP32 multigrid inside the FP64 recurrences; double: an
@@ -627,12 +610,12 @@ static BlockResult block_pcg_mw(mk_ctx* c, const mk_op* A, Mg* mg, const double*
     // the recurrence residual is driven to half the target so the true residual meets it
     hipLaunchKernelGGL(k_set_bstate, dim3(1), dim3(1), 0, c->stream, st.p, 0.25 * rel_tol * rel_tol);
     hipLaunchKernelGGL((bk_init0<MW, ZT>), dim3(g), dim3(256), 0, c->stream, len, B, X, R.p, rz, part.p);
-    hipLaunchKernelGGL((bk_init0_fin<MW>), dim3(1), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
+    hipLaunchKernelGGL((bk_init0_fin<MW>), dim3(MW), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
     mg_apply_block<ZT>(c, mg, MW, vin, zc, nullptr);
     hipLaunchKernelGGL((bk_init1<MW, ZT>), dim3(g), dim3(256), 0, c->stream, len, (const double*)R.p,
                        (const ZT*)zc, P.p, part.p);
     std::swap(zc, zo);
-    hipLaunchKernelGGL((bk_init1_fin<MW>), dim3(1), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
+    hipLaunchKernelGGL((bk_init1_fin<MW>), dim3(MW), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
     MK_HIP(hipGetLastError());
     BState h{};
     int iters = 0;
@@ -659,14 +642,14 @@ static BlockResult block_pcg_mw(mk_ctx* c, const mk_op* A, Mg* mg, const double*
             spmm_launch<double>(c, A, MW, P.p, Q.p, nullptr, SPMV_PLAIN, &st.p->all_done);
             hipLaunchKernelGGL((bk_alpha<MW>), dim3(g), dim3(256), 0, c->stream, len, (const double*)P.p,
                                (const double*)Q.p, (const BState*)st.p, part.p);
-            hipLaunchKernelGGL((bk_alpha_fin<MW>), dim3(1), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
+            hipLaunchKernelGGL((bk_alpha_fin<MW>), dim3(MW), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
             hipLaunchKernelGGL((bk_update<MW, ZT>), dim3(g), dim3(256), 0, c->stream, len, X, R.p, rz,
                                (const double*)P.p, (const double*)Q.p, (const BState*)st.p, part.p);
-            hipLaunchKernelGGL((bk_update_fin<MW>), dim3(1), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
+            hipLaunchKernelGGL((bk_update_fin<MW>), dim3(MW), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
             mg_apply_block<ZT>(c, mg, MW, vin, zc, &st.p->all_done);
             hipLaunchKernelGGL((bk_beta<MW, ZT>), dim3(g), dim3(256), 0, c->stream, len, (const double*)R.p,
                                (const ZT*)zc, (const ZT*)zo, (const BState*)st.p, part.p);
-            hipLaunchKernelGGL((bk_beta_fin<MW>), dim3(1), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
+            hipLaunchKernelGGL((bk_beta_fin<MW>), dim3(MW), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
             hipLaunchKernelGGL((bk_pupdate<MW, ZT>), dim3(g), dim3(256), 0, c->stream, len, P.p, (const ZT*)zc,
                                (const BState*)st.p);
             std::swap(zc, zo);

@@ -133,7 +133,7 @@ struct Work {
 struct BState {
     double rz[64], rr[64], bb[64], alpha[64], beta[64];
     int done[64], status[64], it[64];
-    int all_done, pad;
+    int all_done, ndone;  // every column finished; columns finished so far
     double tol2;
 };
 struct BlockResult {

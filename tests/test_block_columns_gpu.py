@@ -1,0 +1,45 @@
+"""Block PCG column bookkeeping (mk_spd_solve_many): every block width and the column counts at
+their edges, with columns that are empty, converge at once or break down, each column judged by
+its own residual against the 1e-10 the call promises."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+import metriko_amd as mk
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid(nx, ny, shift):
+    T = lambda n: sp.diags([-np.ones(n - 1), 2.0 * np.ones(n), -np.ones(n - 1)], [-1, 0, 1])  # noqa: E731
+    return (sp.kron(T(ny), sp.identity(nx)) + sp.kron(sp.identity(ny), T(nx)) + shift * sp.identity(nx * ny)).tocsr()
+
+
+@pytest.mark.parametrize("precision", [mk.PREC_MIXED_MG, mk.PREC_FP64])
+@pytest.mark.parametrize("m", [1, 8, 9, 16, 17, 32, 33, 64, 65])
+def test_columns_at_the_block_widths(gpu_ctx, m, precision):
+    A = _grid(83, 61, 1e-3)
+    n = A.shape[0]
+    rng = np.random.default_rng(m)
+    B = rng.standard_normal((n, m))
+    if m > 2:
+        B[:, 1] = 0.0                     # finished before the first iteration
+        B[:, 2] = A @ np.ones(n) * 1e-30  # a tiny column: its own norm is the reference
+    X, st = gpu_ctx.op_real(A).solve_many(B, o=mk.opts(precision=precision))
+    res = np.linalg.norm(A @ X - B, axis=0) / np.maximum(np.linalg.norm(B, axis=0), 1e-300)
+    assert res.max() <= 1e-10 and st["solves"] == m
+    if m > 2:
+        assert np.abs(X[:, 1]).max() == 0.0
+
+
+def test_a_column_with_nan_is_reported(gpu_ctx):
+    A = _grid(40, 37, 1e-3)
+    B = np.random.default_rng(0).standard_normal((A.shape[0], 12))
+    B[5, 7] = np.nan
+    op = gpu_ctx.op_real(A)
+    with pytest.raises(mk.MetrikoError) as ei:
+        op.solve_many(B)
+    assert ei.value.status == 5
+    B[5, 7] = 0.0
+    X, _ = op.solve_many(B)  # the operator is still usable
+    assert np.linalg.norm(A @ X - B) <= 1e-10 * np.linalg.norm(B)
