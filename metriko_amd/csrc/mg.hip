@@ -44,9 +44,7 @@ struct Mg {
     const uint64_t uid = next_uid();  // keys the PCG graphs captured through this hierarchy
     bool cplx = false;
     std::vector<MgLevel> lv;
-    int nc = 0;
-    DevBuf<double> inv64;  // dense coarsest inverse (row-major, complex interleaved)
-    DevBuf<float> inv32;
+    DenseInverse coarse;  // of the coarsest operator
     int deg = 2;
     double setup_ms = 0.0;
     int64_t nnz_total = 0;
@@ -68,6 +66,9 @@ struct MgTune {
     double theta_real = 0.05, theta_cplx = 0.08, lmin_div = 10.0, lmax_fac = 1.2;
     int deg = 2, power = 15, phase_real = 1, coarse_real = 500, coarse_cplx = 400, smooth_long = 1, compat = 1,
         l1 = 1, attach = 1, rr = 0;
+    // Largest level the device solves by its dense inverse (the coarse_ limits above are the host
+    // solve's): see build_impl.
+    int dense_real = 2400, dense_cplx = 2100;
 };
 static const MgTune& tune() {
     static const MgTune t = [] {
@@ -83,6 +84,8 @@ static const MgTune& tune() {
         i("METRIKO_MG_PHASE_REAL", x.phase_real);
         i("METRIKO_MG_COARSE_REAL", x.coarse_real);
         i("METRIKO_MG_COARSE_CPLX", x.coarse_cplx);
+        i("METRIKO_MG_DENSE_REAL", x.dense_real);
+        i("METRIKO_MG_DENSE_CPLX", x.dense_cplx);
         i("METRIKO_MG_SMOOTH_LONG", x.smooth_long);
         i("METRIKO_MG_COMPAT", x.compat);
         i("METRIKO_MG_L1", x.l1);
@@ -578,8 +581,7 @@ struct HostHier {
     std::vector<Csr<T>> A, P, R, RR;
     std::vector<double> lmax;
     std::vector<std::vector<double>> dinv;
-    std::vector<double> inv;  // coarsest dense inverse (row-major, complex interleaved)
-    int nc = 0;
+    std::vector<double> inv;  // coarsest dense inverse (row-major, complex interleaved; host solves only)
     // per level but the coarsest: the coarse unknown that stands for each node's aggregate
     // (the first column of its tentative prolongator row; -1 for an empty row)
     std::vector<std::vector<int>> key;
@@ -614,7 +616,7 @@ std::vector<std::vector<int>> hier_order(const HostHier<T>& H) {
 }
 
 template <typename T>
-HostHier<T> build_host(Csr<T> A, double theta, int coarse_max, const std::vector<T>* B0 = nullptr,
+HostHier<T> build_host(Csr<T> A, double theta, int finest_max, int coarse_max, bool host_inverse, const std::vector<T>* B0 = nullptr,
                        int nb = 0) {
     HostHier<T> H;
     const bool cplx = !std::is_same<T, double>::value;
@@ -654,7 +656,9 @@ HostHier<T> build_host(Csr<T> A, double theta, int coarse_max, const std::vector
             }
         }
         lap("diagonals");
-        const double lmax = tune().lmax_fac * rho_dinv_a(A, ds);
+        bool last = A.nr <= (l == 0 ? finest_max : coarse_max) || l == maxLevels - 1;
+        // the coarsest level is not smoothed: no spectral bound
+        const double lmax = last ? 1.0 : tune().lmax_fac * rho_dinv_a(A, ds);
         lap("spectral bound");
         std::vector<double> di(d.size());
         for (size_t i = 0; i < d.size(); i++) di[i] = ds[i] != 0.0 ? 1.0 / ds[i] : 1.0;
@@ -672,7 +676,6 @@ HostHier<T> build_host(Csr<T> A, double theta, int coarse_max, const std::vector
         }
         int nagg = 0;
         Csr<T> Pt;
-        bool last = A.nr <= coarse_max || l == maxLevels - 1;
         if (!last) {
             std::vector<T> Bc;
             if (nb > 0) Pt = tentative_qr(A, d, theta, B, nb, Bc, nagg);
@@ -694,8 +697,7 @@ HostHier<T> build_host(Csr<T> A, double theta, int coarse_max, const std::vector
         H.lmax.push_back(lmax);
         H.dinv.push_back(std::move(di));
         if (last) {
-            dense_hpd_inverse(A, H.inv, cplx);
-            H.nc = A.nr;
+            if (host_inverse) dense_hpd_inverse(A, H.inv, cplx);
             H.A.push_back(std::move(A));
             break;
         }
@@ -818,10 +820,21 @@ HostHier<T> build_host(Csr<T> A, double theta, int coarse_max, const std::vector
 // smoother's diagonal -- and the finest level's pos[old] = new is returned there; the caller's
 // vectors for this hierarchy are then in that order.  Each renumbered row keeps its entries'
 // order, so every product computes the same numbers as without the renumbering.
+//
+// coarse_max: a level of at most this many unknowns is solved by its dense inverse (DenseInverse)
+// instead of being smoothed and coarsened further, the finest level too (then the hierarchy is that
+// inverse), unless an order is asked for: a one-level hierarchy has none, so the finest level is
+// then taken only up to finest_ordered.  Where the line lies: on small levels a smoothing or transfer
+// kernel takes 4 to 5 us whatever its size, six of them per level and cycle; the inverse's product
+// takes 2.3 us at 1,584 complex unknowns, 4.8 us at 1,498 below a 40,820-face field (its levels of
+// 1,498 and 174 took 29 us) and 18.5 us at 2,059 (68 MB, read from HBM; its levels of 2,059 and 216
+// took 30 us); real: 46 MB at 2,400.  At 4,000 real unknowns a solve of 301,702 x 64 columns became
+// slower (46.0 -> 57.7 ms).
 template <typename T>
-Mg* build_impl(mk_ctx* c, Csr<T>&& A0, const mk_solve_opts& o, double theta, int coarse_max,
+Mg* build_impl(mk_ctx* c, Csr<T>&& A0, const mk_solve_opts& o, double theta, int coarse_max, int finest_ordered,
                const std::vector<T>* nullvec = nullptr, int nnull = 0, std::vector<int>* order_out = nullptr) {
-    HostHier<T> H = build_host<T>(std::move(A0), theta, coarse_max, nullvec, nnull);
+    HostHier<T> H = build_host<T>(std::move(A0), theta, order_out ? finest_ordered : coarse_max, coarse_max, false, nullvec,
+                                  nnull);
     const auto t_up = std::chrono::steady_clock::now();
     // per level but the coarsest: pos (stored index of each unknown) and its inverse
     std::vector<std::vector<int>> pos, inv;
@@ -848,8 +861,11 @@ Mg* build_impl(mk_ctx* c, Csr<T>&& A0, const mk_solve_opts& o, double theta, int
             MgLevel L;
             L.n = H.A[l].nr;
             L.lmax = H.lmax[l];
-            L.A = upload(c, H.A[l], o, I_(l), P_(l));
-            {  // the smoother's inverse diagonal replaces the plain one
+            // the coarsest operator is only needed as its inverse
+            const bool last = l + 1 == H.A.size();
+            if (!last) {
+                L.A = upload(c, H.A[l], o, I_(l), P_(l));
+                // the smoother's inverse diagonal replaces the plain one
                 std::vector<double> dv = H.dinv[l];
                 if (P_(l))
                     for (size_t i = 0; i < dv.size(); i++) dv[size_t(pos[l][i])] = H.dinv[l][i];
@@ -876,16 +892,19 @@ Mg* build_impl(mk_ctx* c, Csr<T>&& A0, const mk_solve_opts& o, double theta, int
             g->lv.push_back(std::move(L));
             if (verbose) std::fprintf(stderr, "[mg]   level %zu uploaded %.0f ms\n", l, since_up());
         }
-        g->nc = H.nc;
-        g->inv64.upload(H.inv.data(), H.inv.size(), c->stream);
-        std::vector<float> inv32(H.inv.begin(), H.inv.end());
-        g->inv32.upload(inv32.data(), inv32.size(), c->stream);
-        MK_HIP(hipStreamSynchronize(c->stream));
-        if (verbose) std::fprintf(stderr, "[mg]   coarsest inverse uploaded %.0f ms\n", since_up());
-        for (auto& L : g->lv) {
+        const Csr<T>& Ac = H.A.back();
+        g->coarse = DenseInverse(c, g->cplx, Ac.nr, Ac.ptr.data(), Ac.col.data(),
+                                 reinterpret_cast<const double*>(Ac.val.data()));
+        if (verbose) std::fprintf(stderr, "[mg]   coarsest inverse %.0f ms\n", since_up());
+        // the finest level works on the caller's b and x, the coarsest needs no other vectors
+        for (size_t l = 0; l < g->lv.size(); l++) {
+            MgLevel& L = g->lv[l];
             const size_t len = size_t(L.n) * (g->cplx ? 2 : 1);
-            L.b64.alloc(len); L.x64.alloc(len); L.r64.alloc(len); L.d64.alloc(len); L.y64.alloc(len);
-            L.b32.alloc(len); L.x32.alloc(len); L.r32.alloc(len); L.d32.alloc(len); L.y32.alloc(len);
+            if (l > 0) { L.b64.alloc(len); L.x64.alloc(len); L.b32.alloc(len); L.x32.alloc(len); }
+            if (l + 1 < g->lv.size()) {
+                L.r64.alloc(len); L.d64.alloc(len); L.y64.alloc(len);
+                L.r32.alloc(len); L.d32.alloc(len); L.y32.alloc(len);
+            }
         }
         MK_LOG("[mg] hierarchy upload %.0f ms\n",
                std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_up).count());
@@ -921,37 +940,6 @@ __global__ void k_cheb_first(int n, const T* __restrict__ dinv, const T* __restr
         else x[i] += d0;
     }
 }
-// x = Inv b (dense n x n, row-major): one wavefront per row, lanes stride the row (coalesced
-// reads of Inv), shuffle reduction; 4 rows per 256-thread block
-template <typename T, bool CPLX>
-__global__ void __launch_bounds__(256) k_dense_gemv(int n, const T* __restrict__ inv, const T* __restrict__ b,
-                                                    T* __restrict__ x, const int* skip) {
-    if (skip && *skip) return;
-    const int i = blockIdx.x * 4 + int(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (i >= n) return;  // uniform inside the wavefront
-    T ar = 0, ai = 0;
-    for (int j = lane; j < n; j += 64) {
-        if constexpr (CPLX) {
-            const T mr = inv[2 * (size_t(i) * n + j)], mi = inv[2 * (size_t(i) * n + j) + 1];
-            const T br = b[2 * j], bi = b[2 * j + 1];
-            ar += mr * br - mi * bi;
-            ai += mr * bi + mi * br;
-        } else {
-            ar += inv[size_t(i) * n + j] * b[j];
-        }
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        ar += __shfl_xor(ar, off, 64);
-        if constexpr (CPLX) ai += __shfl_xor(ai, off, 64);
-    }
-    if (lane == 0) {
-        if constexpr (CPLX) { x[2 * i] = ar; x[2 * i + 1] = ai; }
-        else x[i] = ar;
-    }
-}
-
 inline unsigned nb(size_t n) { return unsigned((n + 255) / 256); }
 
 template <typename T>
@@ -965,7 +953,6 @@ struct Sel<double> {
     static double* r(MgLevel& L) { return L.r64.p; }
     static double* d(MgLevel& L) { return L.d64.p; }
     static double* y(MgLevel& L) { return L.y64.p; }
-    static const double* inv(const Mg* g) { return g->inv64.p; }
     static double bytes(const mk_op* A) { return A->bytes64; }
 };
 template <>
@@ -977,7 +964,6 @@ struct Sel<float> {
     static float* r(MgLevel& L) { return L.r32.p; }
     static float* d(MgLevel& L) { return L.d32.p; }
     static float* y(MgLevel& L) { return L.y32.p; }
-    static const float* inv(const Mg* g) { return g->inv32.p; }
     static double bytes(const mk_op* A) { return A->bytes32; }
 };
 
@@ -1035,12 +1021,7 @@ template <typename T>
 void vcycle(mk_ctx* c, Mg* g, int l, const T* b, T* x, const int* skip) {
     MgLevel& L = g->lv[size_t(l)];
     if (l + 1 == int(g->lv.size())) {
-        if (g->cplx)
-            hipLaunchKernelGGL((k_dense_gemv<T, true>), dim3(unsigned((g->nc + 3) / 4)), dim3(256), 0, c->stream, g->nc,
-                               Sel<T>::inv(g), b, x, skip);
-        else
-            hipLaunchKernelGGL((k_dense_gemv<T, false>), dim3(unsigned((g->nc + 3) / 4)), dim3(256), 0, c->stream, g->nc,
-                               Sel<T>::inv(g), b, x, skip);
+        g->coarse.apply<T>(c, b, x, skip);
         return;
     }
     chebyshev<T>(c, g, L, b, x, true, skip);
@@ -1068,20 +1049,6 @@ __global__ void k_bcheb_first(size_t len, int sh, const T* __restrict__ dinv, co
     if (e >= len) return;
     x[e] = c0 * dinv[e >> sh] * r[e];
 }
-// X = Inv B on the coarsest level, one thread per (row, column)
-template <typename T>
-__global__ void k_bdense(int nc, int sh, const T* __restrict__ inv, const T* __restrict__ b, T* __restrict__ x,
-                         const int* skip) {
-    if (skip && *skip) return;
-    const size_t e = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    const size_t mw = size_t(1) << sh;
-    if (e >= size_t(nc) * mw) return;
-    const size_t i = e >> sh, j = e & (mw - 1);
-    T a = T(0);
-    for (int k = 0; k < nc; k++) a += inv[i * size_t(nc) + k] * b[size_t(k) * mw + j];
-    x[e] = a;
-}
-
 // the block buffers of a level in precision T
 template <typename T>
 struct BlockBufs { T *b, *x, *r, *y; };
@@ -1141,11 +1108,7 @@ template <typename T>
 static void vcycle_block(mk_ctx* c, Mg* g, int l, int mw, int sh, const T* b, T* x, const int* skip) {
     MgLevel& L = g->lv[size_t(l)];
     if (l + 1 == int(g->lv.size())) {
-        const T* inv;
-        if constexpr (std::is_same<T, double>::value) inv = g->inv64.p;
-        else inv = g->inv32.p;
-        hipLaunchKernelGGL((k_bdense<T>), dim3(nb(size_t(g->nc) * mw)), dim3(256), 0, c->stream, g->nc, sh, inv, b, x,
-                           skip);
+        g->coarse.apply_block<T>(c, mw, b, x, skip);
         return;
     }
     const BlockBufs<T> Lb = block_bufs<T>(L);
@@ -1268,7 +1231,7 @@ extern "C" mk_status mk_mg_host_pcg(int n, const int64_t* ptr, const int32_t* co
             for (int64_t k = 0; k < ptr[n]; k++) A.val[k] = cd(val[2 * k], val[2 * k + 1]);
             std::vector<cd> B;
             for (size_t q = 0; q < size_t(n) * size_t(nnull); q++) B.emplace_back(nullvec[2 * q], nullvec[2 * q + 1]);
-            HostHier<cd> H = build_host<cd>(Csr<cd>(A), tune().theta_cplx, tune().coarse_cplx, nnull ? &B : nullptr, nnull);
+            HostHier<cd> H = build_host<cd>(Csr<cd>(A), tune().theta_cplx, tune().coarse_cplx, tune().coarse_cplx, true, nnull ? &B : nullptr, nnull);
             if (levels) *levels = int(H.A.size());
             int it = host_pcg<cd>(A, H, reinterpret_cast<const cd*>(b), reinterpret_cast<cd*>(x), tol, maxit, relres);
             if (iters) *iters = it;
@@ -1280,6 +1243,7 @@ extern "C" mk_status mk_mg_host_pcg(int n, const int64_t* ptr, const int32_t* co
             std::vector<double> B;
             if (nnull > 0) B.assign(nullvec, nullvec + size_t(n) * nnull);
             HostHier<double> H = build_host<double>(Csr<double>(A), tune().theta_real, tune().coarse_real,
+                                                    tune().coarse_real, true,
                                                     nnull ? &B : nullptr, nnull);
             if (levels) *levels = int(H.A.size());
             int it = host_pcg<double>(A, H, b, x, tol, maxit, relres);
@@ -1307,7 +1271,7 @@ Mg* mg_build_real(mk_ctx* c, int n, const int64_t* ptr, const int* col, const do
         A.col[size_t(k)] = col[k];
         A.val[size_t(k)] = val[k];
     }
-    Mg* g = build_impl<double>(c, std::move(A), o, tune().theta_real, tune().coarse_real, nullvec, nnull, order_out);
+    Mg* g = build_impl<double>(c, std::move(A), o, tune().theta_real, tune().dense_real, tune().coarse_real, nullvec, nnull, order_out);
     return g;
 }
 Mg* mg_build_complex(mk_ctx* c, int n, const int64_t* ptr, const int* col, const double* val,
@@ -1321,7 +1285,7 @@ Mg* mg_build_complex(mk_ctx* c, int n, const int64_t* ptr, const int* col, const
         A.col[size_t(k)] = col[k];
         A.val[size_t(k)] = cd(val[2 * k], val[2 * k + 1]);
     }
-    return build_impl<cd>(c, std::move(A), o, tune().theta_cplx, tune().coarse_cplx);
+    return build_impl<cd>(c, std::move(A), o, tune().theta_cplx, tune().dense_cplx, tune().coarse_cplx);
 }
 void mg_apply64(mk_ctx* c, Mg* g, const double* b, double* x, const int* skip) { vcycle<double>(c, g, 0, b, x, skip); }
 void mg_apply32(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip) { vcycle<float>(c, g, 0, b, x, skip); }

@@ -141,6 +141,20 @@ struct BlockResult {
     int iters;        // max over the columns
     double max_rel;   // max relative residual (recurrence) over the columns
 };
+// Dense inverse of a Hermitian positive definite operator (dense.hip): the coarsest multigrid
+// level.  FP64, row-major, leading dimension ld; applied to FP64 or FP32 vectors and blocks.
+struct DenseInverse {
+    int n = 0, ld = 0;
+    bool cplx = false;
+    DevBuf<double> inv;
+    DenseInverse() = default;
+    // from CSR arrays on the host (complex: values interleaved)
+    DenseInverse(mk_ctx* c, bool cplx, int n, const int64_t* ptr, const int* col, const double* val);
+    template <typename T>
+    void apply(mk_ctx* c, const T* b, T* x, const int* skip) const;  // x = A^-1 b
+    template <typename T>
+    void apply_block(mk_ctx* c, int mw, const T* B, T* X, const int* skip) const;  // n x mw row-major
+};
 // multigrid (mg.hip)
 // order_out: store the finest level in the aggregates' locality order and return pos[old] = new
 // there (left empty for a one-level hierarchy); the hierarchy then takes and returns vectors
