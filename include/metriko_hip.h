@@ -53,7 +53,9 @@ typedef struct {
     int precond;        /* MK_PRECOND_*, default AMG */
     double inner_tol;   /* FP32 inner relative tolerance per refinement step, default 1e-5 */
     int max_refine;     /* max refinement steps, default 12 */
-    int check_every;    /* iterations between host convergence checks, default 16 */
+    int check_every;    /* iterations between host convergence checks, default 16 (further apart while the
+                         * residual's decrease says at least two such intervals are left; results do not
+                         * depend on it) */
 } mk_solve_opts;
 
 typedef struct {

@@ -465,7 +465,7 @@ __global__ void __launch_bounds__(256) bk_init1_fin(BState* st, const double* __
     if (threadIdx.x == 0) {
         const double rz = tot[0], rr = tot[1];
         st->rz[j] = rz;
-        st->rr[j] = rr;
+        st->rr[j] = st->rr0[j] = rr;
         bool d = rr <= st->tol2 * st->bb[j];
         if (!(rz == rz) || !(rr == rr)) { st->status[j] = MK_ERR_NAN; d = true; }
         else if (!d && !(rz > 0.0)) { st->status[j] = MK_ERR_NOT_SPD; d = true; }
@@ -617,27 +617,16 @@ static BlockResult block_pcg_mw(mk_ctx* c, const mk_op* A, Mg* mg, const double*
     std::swap(zc, zo);
     hipLaunchKernelGGL((bk_init1_fin<MW>), dim3(MW), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
     MK_HIP(hipGetLastError());
-    BState h{};
+    static_assert(sizeof(BState) <= mk_ctx::kPinBytes, "BState does not fit the readback memory");
+    const BState& h = *static_cast<const BState*>(c->pin);
     int iters = 0;
-    // the batch ends where the slowest running column is predicted to converge
+    // the batch ends where the slowest running column is predicted to converge (see BatchPlanner)
     const int interval = c->time_spmv ? 1 : std::max(1, check_every);
+    int plan = BatchPlanner(interval).first(A->last_block_iters);
     int prev_iters = -1;
     double prev_rr[MW] = {};
     for (;;) {
-        MK_HIP(hipMemcpyAsync(&h, st.p, sizeof(BState), hipMemcpyDeviceToHost, c->stream));
-        MK_HIP(hipStreamSynchronize(c->stream));
-        timing_flush(c);
-        if (h.all_done || iters >= maxiter) break;
-        int plan = 0;
-        for (int j = 0; j < MW && plan < interval; j++) {
-            if (h.done[j]) continue;
-            const double nd = BatchPlanner::need(iters, h.rr[j], prev_iters, prev_rr[j], h.tol2 * h.bb[j]);
-            plan = std::max(plan, BatchPlanner::clamp_need(nd, interval));
-        }
-        if (plan == 0) plan = interval;
-        for (int j = 0; j < MW; j++) prev_rr[j] = h.rr[j];
-        prev_iters = iters;
-        const int batch = std::min(plan, maxiter - iters);
+        const int batch = std::max(0, std::min(plan, maxiter - iters));
         for (int k = 0; k < batch; k++) {
             spmm_launch<double>(c, A, MW, P.p, Q.p, nullptr, SPMV_PLAIN, &st.p->all_done);
             hipLaunchKernelGGL((bk_alpha<MW>), dim3(g), dim3(256), 0, c->stream, len, (const double*)P.p,
@@ -656,6 +645,22 @@ static BlockResult block_pcg_mw(mk_ctx* c, const mk_op* A, Mg* mg, const double*
         }
         iters += batch;
         MK_HIP(hipGetLastError());
+        MK_HIP(hipMemcpyAsync(c->pin, st.p, sizeof(BState), hipMemcpyDeviceToHost, c->stream));
+        MK_HIP(hipStreamSynchronize(c->stream));
+        timing_flush(c);
+        if (h.all_done || iters >= maxiter) break;
+        if (prev_iters < 0) {
+            prev_iters = 0;
+            for (int j = 0; j < MW; j++) prev_rr[j] = h.rr0[j];
+        }
+        plan = 1;
+        for (int j = 0; j < MW; j++) {
+            if (h.done[j]) continue;
+            const double nd = BatchPlanner::need(iters, h.rr[j], prev_iters, prev_rr[j], h.tol2 * h.bb[j]);
+            plan = std::max(plan, interval == 1 ? 1 : BatchPlanner::clamp_need(nd, interval));
+        }
+        for (int j = 0; j < MW; j++) prev_rr[j] = h.rr[j];
+        prev_iters = iters;
     }
     BlockResult res;
     res.status = MK_OK;
@@ -667,6 +672,7 @@ static BlockResult block_pcg_mw(mk_ctx* c, const mk_op* A, Mg* mg, const double*
         if (h.bb[j] > 0.0) res.max_rel = std::max(res.max_rel, std::sqrt(h.rr[j] / h.bb[j]));
     }
     if (res.status == MK_OK && !h.all_done) res.status = MK_ERR_NO_CONVERGENCE;
+    A->last_block_iters = res.iters;
     return res;
 }
 

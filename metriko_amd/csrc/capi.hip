@@ -155,9 +155,10 @@ __global__ void __launch_bounds__(64 * kWinDots) k_window_sum(int nparts, const 
     s = mk::wave_sum(s);
     if (lane == 0) out[k] = s;
 }
-// x = sum_j y_j w_j (complex coefficients y[2j], y[2j+1]).
-__global__ void k_window_combine(int n, int nw, const double* __restrict__ W, const double* __restrict__ y,
-                                 double* __restrict__ x) {
+// x = sum_j y_j w_j (complex coefficients y[2j], y[2j+1], handed over with the launch).
+struct WindowCoef { double y[2 * kWin]; };
+__global__ void k_window_combine(int n, int nw, const double* __restrict__ W, WindowCoef c, double* __restrict__ x) {
+    const double* y = c.y;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     double xr = 0.0, xi = 0.0;
@@ -168,6 +169,20 @@ __global__ void k_window_combine(int n, int nw, const double* __restrict__ W, co
     }
     x[2 * i] = xr;
     x[2 * i + 1] = xi;
+}
+
+// The next iterate u = x / sqrt|s| and its right-hand side b = M u, one pass over x (scaling, two
+// copies and the product with M were four).
+__global__ void k_next_iterate(int n, const double* __restrict__ s, const double* __restrict__ mass,
+                               const double* __restrict__ x, double* __restrict__ u, double* __restrict__ b) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const double f = 1.0 / sqrt(fabs(s[0])), m = mass[i];
+    const double u0 = x[2 * i] * f, u1 = x[2 * i + 1] * f;
+    u[2 * i] = u0;
+    u[2 * i + 1] = u1;
+    b[2 * i] = m * u0;
+    b[2 * i + 1] = m * u1;
 }
 
 }  // namespace
@@ -453,12 +468,17 @@ mk_status mk_init(mk_ctx** out, int device) {
         c->partials.alloc(mk::kMaxParts * mk::kMaxK);
         c->state.alloc(1);
         c->scal.alloc(64);
+        MK_HIP(hipHostMalloc(&c->pin, mk_ctx::kPinBytes, hipHostMallocDefault));
         MK_HIP(hipMemsetAsync(c->scal.p, 0, 64 * sizeof(double), c->stream));
         MK_HIP(hipStreamSynchronize(c->stream));
         const char* t = std::getenv("METRIKO_TIME_SPMV");
         c->time_spmv = t && t[0] == '1';
     });
-    if (s != MK_OK) { delete c; return s; }
+    if (s != MK_OK) {
+        if (c->pin) (void)hipHostFree(c->pin);
+        delete c;
+        return s;
+    }
     *out = c;
     return MK_OK;
 }
@@ -475,6 +495,8 @@ mk_status mk_finalize(mk_ctx* c) {
     c->partials.release();
     c->state.release();
     c->scal.release();
+    if (c->pin) (void)hipHostFree(c->pin);
+    c->pin = nullptr;
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return MK_OK;
@@ -909,40 +931,36 @@ mk_status mk_field_smallest_eig(mk_ctx* c, const mk_op* L, const double* mass, c
         mk::stats_reset(c);
         const int n = L->n;
         const size_t len = size_t(n) * 2;
-        DevBuf<double> dm, du, dx, db, dW, dLW, dpart, dy;
+        DevBuf<double> dm, dx, db, dW, dLu, dpart;
         dm.upload(mass, size_t(n), c->stream);
-        du.upload(u0, len, c->stream);
         dx.alloc(len);
         db.alloc(len);
-        dW.alloc(len * kWin);
-        dLW.alloc(len * kWin);
+        dW.alloc(len * kWin);  // the iterates themselves live in the window, iterate `it` in slot it % kWin
+        dLu.alloc(len);
+        MK_HIP(hipMemcpyAsync(dW.p, u0, len * sizeof(double), hipMemcpyHostToDevice, c->stream));
+        mk::mass_mul(c, n, dm.p, dW.p, db.p);
         const unsigned gw = mk::rgrid(size_t(n));
         dpart.alloc(size_t(gw) * kWinDots + kWinDots);
-        dy.alloc(2 * kWin);
         double* sc = c->scal.p;
         int total_it = 0, total_ref = 0;
         double last_rel = 0.0;
         // Galerkin matrix G = W^H L W of the window (slot order), kept across iterations
         std::vector<std::complex<double>> G(static_cast<size_t>(kWin) * kWin), g(static_cast<size_t>(kWin));
-        double hd[kWinDots], hy[2 * kWin];
+        const double* hd = static_cast<const double*>(c->pin);
         for (int it = 0; it < n_iter; it++) {
-            // b = M u
-            mk::mass_mul(c, n, dm.p, du.p, db.p);
-            // The iterate enters the window (slot s) with L u, then the start is the Galerkin
-            // solution on span(W): x0 = W (W^H L W)^+ W^H b.  With the window {u} alone this is
-            // the Rayleigh-quotient start u (u^H M u) / (u^H L u); the last kWin iterates
-            // span the slowly converging eigen-directions, so x0 starts PCG many digits closer.
+            // The start is the Galerkin solution on span(W), the window with the iterate u (slot
+            // s): x0 = W (W^H L W)^+ W^H b.  With the window {u} alone this is the
+            // Rayleigh-quotient start u (u^H M u) / (u^H L u); the last kWin iterates span the
+            // slowly converging eigen-directions, so x0 starts PCG many digits closer.
             const int s = it % kWin, nw = std::min(it + 1, kWin);
             double* ws = dW.p + len * size_t(s);
-            double* lws = dLW.p + len * size_t(s);
-            MK_HIP(hipMemcpyAsync(ws, du.p, len * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-            mk::spmv64(c, L, du.p, lws, nullptr, mk::SPMV_PLAIN, nullptr, nullptr);
+            mk::spmv64(c, L, ws, dLu.p, nullptr, mk::SPMV_PLAIN, nullptr, nullptr);
             hipLaunchKernelGGL(k_window_dots, dim3(gw), dim3(256), 0, c->stream, n, nw, (const double*)dW.p,
-                               (const double*)lws, (const double*)db.p, dpart.p);
+                               (const double*)dLu.p, (const double*)db.p, dpart.p);
             hipLaunchKernelGGL(k_window_sum, dim3(1), dim3(64 * kWinDots), 0, c->stream, int(gw), (const double*)dpart.p,
                                dpart.p + size_t(gw) * kWinDots);
-            MK_HIP(hipMemcpyAsync(hd, dpart.p + size_t(gw) * kWinDots, sizeof(hd), hipMemcpyDeviceToHost,
-                                  c->stream));
+            MK_HIP(hipMemcpyAsync(c->pin, dpart.p + size_t(gw) * kWinDots, kWinDots * sizeof(double),
+                                  hipMemcpyDeviceToHost, c->stream));
             MK_HIP(hipStreamSynchronize(c->stream));
             for (int j = 0; j < nw; j++) {
                 const std::complex<double> gjs(hd[4 * j], hd[4 * j + 1]);  // w_j^H L w_s
@@ -956,10 +974,10 @@ mk_status mk_field_smallest_eig(mk_ctx* c, const mk_op* L, const double* mass, c
             for (int i = 0; i < nw; i++)
                 for (int j = 0; j < nw; j++) Gn[size_t(i) * nw + j] = G[size_t(i) * kWin + j];
             const std::vector<std::complex<double>> y = mk::herm_pinv_solve(nw, Gn, gn);
-            for (int j = 0; j < nw; j++) { hy[2 * j] = y[size_t(j)].real(); hy[2 * j + 1] = y[size_t(j)].imag(); }
-            MK_HIP(hipMemcpyAsync(dy.p, hy, 2 * size_t(nw) * sizeof(double), hipMemcpyHostToDevice, c->stream));
+            WindowCoef hy{};
+            for (int j = 0; j < nw; j++) { hy.y[2 * j] = y[size_t(j)].real(); hy.y[2 * j + 1] = y[size_t(j)].imag(); }
             hipLaunchKernelGGL(k_window_combine, dim3(nblk(size_t(n))), dim3(256), 0, c->stream, n, nw,
-                               (const double*)dW.p, (const double*)dy.p, dx.p);
+                               (const double*)dW.p, hy, dx.p);
             // Each solve aims at a tenth of the required relative residual (as far as the FP64
             // floor of the true residual allows): the iteration keeps every solve's error in the
             // field, and the parameterization downstream amplifies field error about a
@@ -976,10 +994,12 @@ mk_status mk_field_smallest_eig(mk_ctx* c, const mk_op* L, const double* mass, c
             }
             // s = sqrt(|x^H M x|); x /= s; u = x
             mk::mass_dot(c, n, dm.p, dx.p, sc + 12);
-            mk::scale_dev64(c, len, sc + 12, 1, dx.p);
-            MK_HIP(hipMemcpyAsync(du.p, dx.p, len * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+            double* un = dW.p + len * size_t((it + 1) % kWin);
+            hipLaunchKernelGGL(k_next_iterate, dim3(nblk(size_t(n))), dim3(256), 0, c->stream, n,
+                               (const double*)(sc + 12), (const double*)dm.p, (const double*)dx.p, un, db.p);
         }
-        dx.download(x_out, len, c->stream);
+        MK_HIP(hipMemcpyAsync(x_out, inner == MK_OK ? dW.p + len * size_t(n_iter % kWin) : dx.p, len * sizeof(double), hipMemcpyDeviceToHost,
+                              c->stream));
         MK_HIP(hipStreamSynchronize(c->stream));
         if (st) {
             std::memset(st, 0, sizeof(*st));

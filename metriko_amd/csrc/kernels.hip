@@ -65,24 +65,6 @@ struct FinOut {  // plain total
     static constexpr bool guard = false;
     __device__ static void apply(CgState*, const double* tot, double* out) { out[0] = tot[0]; }
 };
-struct FinCgInit {  // rz, rr of the first residual
-    static constexpr bool guard = false;
-    __device__ static void apply(CgState* st, const double* tot, double*) {
-        st->rz = tot[0];
-        st->rr = tot[1];
-        st->it = 0;
-        st->status = MK_OK;
-        st->done = (tot[1] <= st->tol2 * st->bb) ? 1 : 0;
-        if (!(tot[0] == tot[0]) || !(tot[1] == tot[1])) { st->status = MK_ERR_NAN; st->done = 1; }
-    }
-};
-struct FinCgInitZ {  // as FinCgInit, z from an external preconditioner (must be positive)
-    static constexpr bool guard = false;
-    __device__ static void apply(CgState* st, const double* tot, double* o) {
-        FinCgInit::apply(st, tot, o);
-        if (!st->done && !(tot[0] > 0.0)) { st->status = MK_ERR_NOT_SPD; st->done = 1; }
-    }
-};
 struct FinCgAlpha {  // pq -> alpha
     static constexpr bool guard = true;
     __device__ static void apply(CgState* st, const double* tot, double*) {
@@ -180,9 +162,10 @@ __global__ void __launch_bounds__(256) sell_spmv(SellDev<T> A, const T* __restri
 // element e of a complex vector occupies entries 2e, 2e+1; the Jacobi scaling dinv
 // is per element (real).
 template <typename T, bool CPLX>
-__global__ void __launch_bounds__(256) cg_init(int n, const T* __restrict__ r, const T* __restrict__ dinv,
-                                             T* __restrict__ z, T* __restrict__ p, double* partials) {
-    double rz = 0.0, rr = 0.0;
+__global__ void __launch_bounds__(256) cg_init(int n, const T* __restrict__ r, const T* __restrict__ b,
+                                             const T* __restrict__ dinv, T* __restrict__ z, T* __restrict__ p,
+                                             double* partials) {
+    double rz = 0.0, rr = 0.0, bb = 0.0;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const T d = dinv ? dinv[i] : T(1);
         if constexpr (CPLX) {
@@ -191,15 +174,17 @@ __global__ void __launch_bounds__(256) cg_init(int n, const T* __restrict__ r, c
             z[2 * i] = z0; z[2 * i + 1] = z1; p[2 * i] = z0; p[2 * i + 1] = z1;
             rz += double(r0) * z0 + double(r1) * z1;
             rr += double(r0) * r0 + double(r1) * r1;
+            bb += double(b[2 * i]) * b[2 * i] + double(b[2 * i + 1]) * b[2 * i + 1];
         } else {
             const T r0 = r[i], z0 = d * r0;
             z[i] = z0; p[i] = z0;
             rz += double(r0) * z0;
             rr += double(r0) * r0;
+            bb += double(b[i]) * b[i];
         }
     }
-    double v[2] = {rz, rr};
-    partials_write<2>(v, partials);
+    double v[3] = {rz, rr, bb};
+    partials_write<3>(v, partials);
 }
 
 // q = A p ; pq = p^H q ; alpha = rz / pq
@@ -263,24 +248,45 @@ __global__ void __launch_bounds__(256) cg_update(int n, T* __restrict__ x, T* __
 
 // preconditioned variant (z from an external preconditioner): init, update, beta
 template <typename T, bool CPLX>
-__global__ void __launch_bounds__(256) cg_init_z(int n, const T* __restrict__ r, const T* __restrict__ z,
-                                               T* __restrict__ p, double* partials) {
-    double rz = 0.0, rr = 0.0;
+__global__ void __launch_bounds__(256) cg_init_z(int n, const T* __restrict__ r, const T* __restrict__ b,
+                                               const T* __restrict__ z, T* __restrict__ p, double* partials) {
+    double rz = 0.0, rr = 0.0, bb = 0.0;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         if constexpr (CPLX) {
             const T r0 = r[2 * i], r1 = r[2 * i + 1], z0 = z[2 * i], z1 = z[2 * i + 1];
             p[2 * i] = z0; p[2 * i + 1] = z1;
             rz += double(r0) * z0 + double(r1) * z1;
             rr += double(r0) * r0 + double(r1) * r1;
+            bb += double(b[2 * i]) * b[2 * i] + double(b[2 * i + 1]) * b[2 * i + 1];
         } else {
             const T r0 = r[i], z0 = z[i];
             p[i] = z0;
             rz += double(r0) * z0;
             rr += double(r0) * r0;
+            bb += double(b[i]) * b[i];
         }
     }
-    double v[2] = {rz, rr};
-    partials_write<2>(v, partials);
+    double v[3] = {rz, rr, bb};
+    partials_write<3>(v, partials);
+}
+
+// rz, rr, bb of the first residual -> the state of a new solve (z from an external preconditioner,
+// check_z, must make rz positive)
+__global__ void __launch_bounds__(1024) cg_init_fin(CgState* st, const double* __restrict__ partials, int nparts,
+                                                    double tol2, int check_z) {
+    double tot[3];
+    partials_sum<3>(partials, nparts, tot);
+    if (threadIdx.x == 0) {
+        st->rz = tot[0];
+        st->rr = st->rr0 = tot[1];
+        st->bb = tot[2];
+        st->tol2 = tol2;
+        st->it = 0;
+        st->status = MK_OK;
+        st->done = (tot[1] <= tol2 * tot[2]) ? 1 : 0;
+        if (!(tot[0] == tot[0]) || !(tot[1] == tot[1])) { st->status = MK_ERR_NAN; st->done = 1; }
+        if (check_z && !st->done && !(tot[0] > 0.0)) { st->status = MK_ERR_NOT_SPD; st->done = 1; }
+    }
 }
 
 template <typename T, bool CPLX>
@@ -446,37 +452,38 @@ __global__ void __launch_bounds__(1024) cgm_spmv_fin(CgState* st, const double* 
     }
 }
 
-// p = q = zold = 0 ; rr = r.r ; state for the first iteration
-__global__ void __launch_bounds__(256) cgm_init2(size_t len, const double* __restrict__ r, double* __restrict__ p,
-                                               double* __restrict__ q, double* __restrict__ zold, CgState* st,
-                                               double* partials) {
-    double rr = 0.0;
+// p = q = zold = 0 ; r32 = float(r) ; rr, bb ; state for the first iteration
+__global__ void __launch_bounds__(256) cgm_init(size_t len, const double* __restrict__ r, const double* __restrict__ b,
+                                              float* __restrict__ r32, double* __restrict__ p, double* __restrict__ q,
+                                              double* __restrict__ zold, double* partials) {
+    double rr = 0.0, bb = 0.0;
     for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < len; i += size_t(gridDim.x) * blockDim.x) {
+        const double ri = r[i], bi = b[i];
         p[i] = 0.0;
         q[i] = 0.0;
         zold[i] = 0.0;
-        rr += r[i] * r[i];
+        r32[i] = float(ri);
+        rr += ri * ri;
+        bb += bi * bi;
     }
-    double v[1] = {rr};
-    partials_write<1>(v, partials);
+    double v[2] = {rr, bb};
+    partials_write<2>(v, partials);
 }
-__global__ void __launch_bounds__(1024) cgm_init2_fin(CgState* st, const double* __restrict__ partials, int nparts) {
-    double tot[1];
-    partials_sum<1>(partials, nparts, tot);
+__global__ void __launch_bounds__(1024) cgm_init_fin(CgState* st, const double* __restrict__ partials, int nparts,
+                                                   double tol2) {
+    double tot[2];
+    partials_sum<2>(partials, nparts, tot);
     if (threadIdx.x == 0) {
-        st->rr = tot[0];
+        st->rr = st->rr0 = tot[0];
+        st->bb = tot[1];
+        st->tol2 = tol2;
         st->rz = 1.0;
         st->it = 0;
         st->first = 1;
         st->status = MK_OK;
-        st->done = (tot[0] <= st->tol2 * st->bb) ? 1 : 0;
+        st->done = (tot[0] <= tol2 * tot[1]) ? 1 : 0;
         if (!(tot[0] == tot[0])) { st->status = MK_ERR_NAN; st->done = 1; }
     }
-}
-
-__global__ void k_to32(size_t len, const double* __restrict__ x, float* __restrict__ y) {
-    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < len) y[i] = float(x[i]);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -484,11 +491,6 @@ __global__ void k_to32(size_t len, const double* __restrict__ x, float* __restri
 __global__ void k_axpby(size_t len, double a, const double* x, double b, double* y) {
     const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < len) y[i] = a * x[i] + b * y[i];
-}
-__global__ void k_scale_dev(size_t len, const double* s, int invert_sqrt, double* y) {
-    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    const double f = invert_sqrt ? 1.0 / sqrt(fabs(s[0])) : s[0];
-    if (i < len) y[i] *= f;
 }
 __global__ void k_mass_mul(int n, const double* mass, const double* u, double* b) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -517,15 +519,6 @@ __global__ void k_add_scaled(size_t len, const float* d, const double* s, double
     const double f = sqrt(s[0]);
     if (i < len) x[i] += f * double(d[i]);
 }
-__global__ void k_set_state(CgState* st, double bb, double tol2) {
-    st->bb = bb;
-    st->tol2 = tol2;
-}
-__global__ void k_set_state_dev(CgState* st, const double* bb, double tol2) {
-    st->bb = bb[0];
-    st->tol2 = tol2;
-}
-
 // ---------------------------------------------------------------------------------------
 // host side
 
@@ -1059,10 +1052,6 @@ void axpby64(mk_ctx* c, size_t len, double a, const double* x, double b, double*
     hipLaunchKernelGGL(k_axpby, dim3(blocks_for(len)), dim3(256), 0, c->stream, len, a, x, b, y);
     MK_HIP(hipGetLastError());
 }
-void scale_dev64(mk_ctx* c, size_t len, const double* s_dev, int invert_sqrt, double* y) {
-    hipLaunchKernelGGL(k_scale_dev, dim3(blocks_for(len)), dim3(256), 0, c->stream, len, s_dev, invert_sqrt, y);
-    MK_HIP(hipGetLastError());
-}
 void dot64(mk_ctx* c, size_t len, const double* x, const double* y, double* out_dev) {
     const unsigned g = fgrid(len);
     hipLaunchKernelGGL(k_dot, dim3(g), dim3(256), 0, c->stream, len, x, y, c->partials.p);
@@ -1088,8 +1077,7 @@ void add32to64_scaled(mk_ctx* c, size_t len, const float* d, const double* s_dev
     MK_HIP(hipGetLastError());
 }
 
-// Generic PCG on the device.  r must hold the initial residual b - A x on entry; bb_dev
-// points to ||b||^2 on the device.
+// Generic PCG on the device.
 static inline void mg_apply(mk_ctx* c, Mg* g, const double* b, double* x, const int* skip) { mg_apply64(c, g, b, x, skip); }
 static inline void mg_apply(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip) { mg_apply32(c, g, b, x, skip); }
 
@@ -1178,11 +1166,11 @@ static void run_batch(mk_ctx* c, const mk_op* A_, const Mg* mg, std::vector<uint
     c->graph_replays++;
 }
 
-// m iterations as captured batches: the check interval itself, or power-of-two pieces (a few
+// m iterations as captured batches: whole check intervals, then power-of-two pieces (a few
 // graph sizes per operator, each captured once and replayed by every later solve)
 template <typename F>
 static void run_batches(int m, int interval, F&& batch) {
-    if (m == interval) { batch(m); return; }
+    for (; interval > 0 && m >= interval; m -= interval) batch(interval);
     for (int p = 1 << 30; m > 0; p >>= 1)
         if (p <= m) { batch(p); m -= p; }
 }
@@ -1214,62 +1202,69 @@ static void cg_iter_mg(mk_ctx* c, const mk_op* A, const T* val, Mg* mg, T* x, T*
     hipLaunchKernelGGL(cg_pupdate<T>, dim3(blocks_for(len)), dim3(256), 0, c->stream, len, p, z, (const CgState*)st);
 }
 
-template <typename T>
-static CgResult cg_run(mk_ctx* c, const mk_op* A, const T* val, const T* dinv, T* x, T* r, T* z, T* p, T* q,
-                       const double* bb_dev, double rel_tol, int maxiter, int check_every, double bytes,
-                       Mg* mg = nullptr) {
+// Runs a started solve (its state on the device): launch(m) queues m iterations; resid() queues
+// the true residual of x into the state behind a batch that is expected to be the last, so that a
+// solve that ends where its operator's last one did costs one round trip to the host.
+template <typename L, typename R>
+static CgResult drive(mk_ctx* c, int hint, int maxiter, int check_every, L&& launch, R&& resid) {
+    BatchPlanner plan(c->time_spmv ? 1 : check_every);
+    CgState* h = static_cast<CgState*>(c->pin);
+    static_assert(sizeof(CgState) <= mk_ctx::kPinBytes, "CgState does not fit the readback memory");
+    int launched = 0, batch = plan.first(hint);
+    for (;;) {
+        batch = std::min(batch, maxiter - launched);
+        if (batch > 0) { launch(batch); launched += batch; }
+        const bool checked = plan.last && !c->time_spmv && resid();
+        MK_HIP(hipGetLastError());
+        MK_HIP(hipMemcpyAsync(h, c->state.p, sizeof(CgState), hipMemcpyDeviceToHost, c->stream));
+        MK_HIP(hipStreamSynchronize(c->stream));
+        timing_flush(c);
+        if (h->done || h->it >= maxiter) {
+            CgResult res{h->status, h->it, h->rr, h->bb, checked ? h->true_rr : -1.0};
+            if (res.status == MK_OK && !h->done) res.status = MK_ERR_NO_CONVERGENCE;
+            return res;
+        }
+        batch = plan.next(h->it, h->rr, h->rr0, h->tol2 * h->bb);
+    }
+}
+
+// PCG on r (the initial residual); b for its norm.  resid as in drive().
+template <typename T, typename R>
+static CgResult cg_run(mk_ctx* c, const mk_op* A, const T* val, const T* dinv, const T* b, T* x, T* r, T* z, T* p, T* q,
+                       double rel_tol, int hint, int maxiter, int check_every, double bytes, Mg* mg, R&& resid) {
     const int n = A->n;
     const size_t len = size_t(n) * (A->cplx ? 2 : 1);
     const unsigned g = blocks_for(n);
     MK_CHECK(g <= kMaxParts, MK_ERR_ARG, "operator too large for the reduction buffer");
     CgState* st = c->state.p;
-    hipLaunchKernelGGL(k_set_state_dev, dim3(1), dim3(1), 0, c->stream, st, bb_dev, rel_tol * rel_tol);
     const unsigned gn = fgrid(size_t(n));
     if (mg) {
         mg_apply(c, mg, r, z, nullptr);
         if (A->cplx)
-            hipLaunchKernelGGL((cg_init_z<T, true>), dim3(gn), dim3(256), 0, c->stream, n, r, z, p, c->partials.p);
+            hipLaunchKernelGGL((cg_init_z<T, true>), dim3(gn), dim3(256), 0, c->stream, n, r, b, z, p, c->partials.p);
         else
-            hipLaunchKernelGGL((cg_init_z<T, false>), dim3(gn), dim3(256), 0, c->stream, n, r, z, p, c->partials.p);
-        finish<2, FinCgInitZ>(c, gn);
+            hipLaunchKernelGGL((cg_init_z<T, false>), dim3(gn), dim3(256), 0, c->stream, n, r, b, z, p, c->partials.p);
     } else {
         if (A->cplx)
-            hipLaunchKernelGGL((cg_init<T, true>), dim3(gn), dim3(256), 0, c->stream, n, r, dinv, z, p, c->partials.p);
+            hipLaunchKernelGGL((cg_init<T, true>), dim3(gn), dim3(256), 0, c->stream, n, r, b, dinv, z, p,
+                               c->partials.p);
         else
-            hipLaunchKernelGGL((cg_init<T, false>), dim3(gn), dim3(256), 0, c->stream, n, r, dinv, z, p, c->partials.p);
-        finish<2, FinCgInit>(c, gn);
+            hipLaunchKernelGGL((cg_init<T, false>), dim3(gn), dim3(256), 0, c->stream, n, r, b, dinv, z, p,
+                               c->partials.p);
     }
+    hipLaunchKernelGGL(cg_init_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)c->partials.p, int(gn),
+                       rel_tol * rel_tol, mg ? 1 : 0);
     MK_HIP(hipGetLastError());
-    if (mg) {
-        CgState h{};
-        BatchPlanner plan(c->time_spmv ? 1 : check_every);
-        for (;;) {
-            MK_HIP(hipMemcpyAsync(&h, st, sizeof(CgState), hipMemcpyDeviceToHost, c->stream));
-            MK_HIP(hipStreamSynchronize(c->stream));
-            timing_flush(c);
-            if (h.done || h.it >= maxiter) break;
-            const int batch = std::min(plan.next(h.it, h.rr, h.tol2 * h.bb), maxiter - h.it);
-            run_batches(batch, check_every, [&](int b) {
+    if (mg)
+        return drive(c, hint, maxiter, check_every, [&](int batch) {
+            run_batches(batch, check_every, [&](int m) {
                 run_batch(c, A, mg, {uintptr_t(sizeof(T)), uintptr_t(val), uintptr_t(x), uintptr_t(r),
                                      uintptr_t(z), uintptr_t(p), uintptr_t(q)},
-                          b, true, [&] { cg_iter_mg<T>(c, A, val, mg, x, r, z, p, q, bytes); });
+                          m, true, [&] { cg_iter_mg<T>(c, A, val, mg, x, r, z, p, q, bytes); });
             });
-            MK_HIP(hipGetLastError());
-        }
-        CgResult res{h.status, h.it, h.rr, h.bb};
-        if (res.status == MK_OK && !h.done) res.status = MK_ERR_NO_CONVERGENCE;
-        return res;
-    }
-    CgState h{};
-    int launched = 0;
-    BatchPlanner plan(c->time_spmv ? 1 : check_every);
-    for (;;) {
-        MK_HIP(hipMemcpyAsync(&h, st, sizeof(CgState), hipMemcpyDeviceToHost, c->stream));
-        MK_HIP(hipStreamSynchronize(c->stream));
-        timing_flush(c);
-        if (h.done || h.it >= maxiter) break;
-        const int batch = std::min(plan.next(h.it, h.rr, h.tol2 * h.bb), maxiter - h.it);
-        for (int b = 0; b < batch; b++) {
+        }, resid);
+    return drive(c, hint, maxiter, check_every, [&](int batch) {
+        for (int k = 0; k < batch; k++) {
             launch_cg_spmv<T>(c, A, val, p, q, bytes);
             if (A->cplx)
                 hipLaunchKernelGGL((cg_update<T, true>), dim3(gn), dim3(256), 0, c->stream, n, x, r, z, p, q, dinv,
@@ -1280,63 +1275,56 @@ static CgResult cg_run(mk_ctx* c, const mk_op* A, const T* val, const T* dinv, T
             finish<2, FinCgUpdate>(c, gn);
             hipLaunchKernelGGL(cg_pupdate<T>, dim3(blocks_for(len)), dim3(256), 0, c->stream, len, p, z,
                                (const CgState*)st);
-            launched++;
         }
-        MK_HIP(hipGetLastError());
-    }
-    CgResult res{h.status, h.it, h.rr, h.bb};
-    if (res.status == MK_OK && !h.done) res.status = MK_ERR_NO_CONVERGENCE;
-    return res;
+    }, resid);
 }
 
-CgResult cg64(mk_ctx* c, const mk_op* A, const double* b, double* x, double rel_tol, int maxiter, bool jacobi,
-              int check_every, bool x_is_zero, Mg* mg) {
+// ||b - A x||^2 into the CG state, for drive()
+static auto true_residual(mk_ctx* c, const mk_op* A, const double* b, const double* x) {
+    return [=] {
+        work(c).t.ensure(size_t(A->n) * (A->cplx ? 2 : 1));
+        spmv64(c, A, x, work(c).t.p, b, SPMV_RESID, &c->state.p->true_rr, nullptr);
+        return true;
+    };
+}
+
+CgResult cg64(mk_ctx* c, const mk_op* A, const double* b, double* x, double rel_tol, int hint, int maxiter, bool jacobi,
+              int check_every, Mg* mg) {
     Work& w = work(c);
     const size_t len = size_t(A->n) * (A->cplx ? 2 : 1);
     w.r.ensure(len); w.z.ensure(len); w.p.ensure(len); w.q.ensure(len);
-    double* bb = c->scal.p + 0;
-    double* rr0 = c->scal.p + 1;
-    dot64(c, len, b, b, bb);
-    if (x_is_zero) MK_HIP(hipMemcpyAsync(w.r.p, b, len * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-    else spmv64(c, A, x, w.r.p, b, SPMV_RESID, rr0, nullptr);
-    return cg_run<double>(c, A, A->val64.p, jacobi ? A->dinv64.p : nullptr, x, w.r.p, w.z.p, w.p.p, w.q.p, bb,
-                          rel_tol, maxiter, check_every, A->bytes64, mg);
+    spmv64(c, A, x, w.r.p, b, SPMV_RESID_NORED, nullptr, nullptr);
+    return cg_run<double>(c, A, A->val64.p, jacobi ? A->dinv64.p : nullptr, b, x, w.r.p, w.z.p, w.p.p, w.q.p, rel_tol,
+                          hint, maxiter, check_every, A->bytes64, mg, true_residual(c, A, b, x));
 }
 
+// x = A^-1 b from zero in FP32
 CgResult cg32(mk_ctx* c, const mk_op* A, const float* b, float* x, double rel_tol, int maxiter, bool jacobi,
               int check_every, Mg* mg) {
     Work& w = work(c);
     const size_t len = size_t(A->n) * (A->cplx ? 2 : 1);
     w.r32.ensure(len); w.z32.ensure(len); w.p32.ensure(len); w.q32.ensure(len);
-    // x = 0, r = b, ||b|| = 1 by construction of the caller (b normalised)
     MK_HIP(hipMemsetAsync(x, 0, len * sizeof(float), c->stream));
     MK_HIP(hipMemcpyAsync(w.r32.p, b, len * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
-    double one = 1.0;
-    MK_HIP(hipMemcpyAsync(c->scal.p + 2, &one, sizeof(double), hipMemcpyHostToDevice, c->stream));
-    return cg_run<float>(c, A, A->val32.p, jacobi ? A->dinv32.p : nullptr, x, w.r32.p, w.z32.p, w.p32.p, w.q32.p,
-                         c->scal.p + 2, rel_tol, maxiter, check_every, A->bytes32, mg);
+    return cg_run<float>(c, A, A->val32.p, jacobi ? A->dinv32.p : nullptr, b, x, w.r32.p, w.z32.p, w.p32.p, w.q32.p,
+                         rel_tol, 0, maxiter, check_every, A->bytes32, mg, [] { return false; });
 }
 
 // FP64 flexible PCG whose multigrid V-cycle runs in FP32 (vectors converted at its ends).
-CgResult cg64_mg32(mk_ctx* c, const mk_op* A, const double* b, double* x, double rel_tol, int maxiter,
+CgResult cg64_mg32(mk_ctx* c, const mk_op* A, const double* b, double* x, double rel_tol, int hint, int maxiter,
                    int check_every, Mg* mg) {
     Work& w = work(c);
     const size_t len = size_t(A->n) * (A->cplx ? 2 : 1);
     w.r.ensure(len); w.z.ensure(len); w.p.ensure(len); w.q.ensure(len);
     w.r32.ensure(len); w.z32.ensure(len);
-    const unsigned g = blocks_for(len);
-    MK_CHECK(g <= kMaxParts, MK_ERR_ARG, "operator too large for the reduction buffer");
-    double* bb = c->scal.p + 0;
-    double* rr0 = c->scal.p + 1;
-    dot64(c, len, b, b, bb);
-    spmv64(c, A, x, w.r.p, b, SPMV_RESID, rr0, nullptr);
+    MK_CHECK(blocks_for(len) <= kMaxParts, MK_ERR_ARG, "operator too large for the reduction buffer");
+    spmv64(c, A, x, w.r.p, b, SPMV_RESID_NORED, nullptr, nullptr);
     CgState* st = c->state.p;
-    hipLaunchKernelGGL(k_set_state_dev, dim3(1), dim3(1), 0, c->stream, st, (const double*)bb, rel_tol * rel_tol);
-    hipLaunchKernelGGL(k_to32, dim3(g), dim3(256), 0, c->stream, len, (const double*)w.r.p, w.r32.p);
     const unsigned gl = fgrid(len);
-    hipLaunchKernelGGL(cgm_init2, dim3(gl), dim3(256), 0, c->stream, len, (const double*)w.r.p, w.p.p, w.q.p,
-                       w.z.p, st, c->partials.p);
-    hipLaunchKernelGGL(cgm_init2_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)c->partials.p, int(gl));
+    hipLaunchKernelGGL(cgm_init, dim3(gl), dim3(256), 0, c->stream, len, (const double*)w.r.p, b, w.r32.p, w.p.p, w.q.p,
+                       w.z.p, c->partials.p);
+    hipLaunchKernelGGL(cgm_init_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)c->partials.p, int(gl),
+                       rel_tol * rel_tol);
     mg_apply32(c, mg, w.r32.p, w.z32.p, &st->done);
     MK_HIP(hipGetLastError());
     unsigned gs = 0;
@@ -1362,25 +1350,14 @@ CgResult cg64_mg32(mk_ctx* c, const mk_op* A, const double* b, double* x, double
         hipLaunchKernelGGL(cgm_update_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)c->partials.p, int(gl));
         mg_apply32(c, mg, w.r32.p, w.z32.p, &st->done);
     };
-    CgState h{};
-    BatchPlanner plan(c->time_spmv ? 1 : check_every);
-    for (;;) {
-        MK_HIP(hipMemcpyAsync(&h, st, sizeof(CgState), hipMemcpyDeviceToHost, c->stream));
-        MK_HIP(hipStreamSynchronize(c->stream));
-        timing_flush(c);
-        if (h.done || h.it >= maxiter) break;
-        const int batch = std::min(plan.next(h.it, h.rr, h.tol2 * h.bb), maxiter - h.it);
-        run_batches(batch, check_every, [&](int b) {
+    return drive(c, hint, maxiter, check_every, [&](int batch) {
+        run_batches(batch, check_every, [&](int m) {
             run_batch(c, A, mg, {uintptr_t(4), uintptr_t(A->val64.p), uintptr_t(x), uintptr_t(w.r.p),
                                  uintptr_t(w.r32.p), uintptr_t(w.z32.p), uintptr_t(w.z.p), uintptr_t(w.p.p),
                                  uintptr_t(w.q.p)},
-                      b, true, iteration);
+                      m, true, iteration);
         });
-        MK_HIP(hipGetLastError());
-    }
-    CgResult res{h.status, h.it, h.rr, h.bb};
-    if (res.status == MK_OK && !h.done) res.status = MK_ERR_NO_CONVERGENCE;
-    return res;
+    }, true_residual(c, A, b, x));
 }
 
 // Iterative refinement: FP64 residual r = b - A x, FP32 PCG correction on r/||r||.
@@ -1401,24 +1378,26 @@ SolveResult solve_spd(mk_ctx* c, const mk_op* A, const double* b, double* x, con
         // the recurrences can drift from the true residual: it is recomputed in FP64 and the
         // solve restarts from x (at most twice) while it is above the tolerance
         for (int attempt = 0;; attempt++) {
-            const CgResult cr = mg32 ? cg64_mg32(c, A, b, x, goal, o.maxiter - res.iters, o.check_every, mg)
-                                     : cg64(c, A, b, x, goal, o.maxiter - res.iters, jac, o.check_every, false, mg);
+            const int hint = attempt == 0 ? A->last_iters : 0;
+            const CgResult cr = mg32 ? cg64_mg32(c, A, b, x, goal, hint, o.maxiter - res.iters, o.check_every, mg)
+                                     : cg64(c, A, b, x, goal, hint, o.maxiter - res.iters, jac, o.check_every, mg);
             res.iters += cr.iters;
-            Work& w = work(c);
-            double h[2];
-            w.t.ensure(len);
-            spmv64(c, A, x, w.t.p, b, SPMV_RESID, c->scal.p + 3, nullptr);
-            MK_HIP(hipMemcpyAsync(h, c->scal.p, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-            double rr;
-            MK_HIP(hipMemcpyAsync(&rr, c->scal.p + 3, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-            MK_HIP(hipStreamSynchronize(c->stream));
-            res.rel_residual = h[0] > 0 ? std::sqrt(rr / h[0]) : std::sqrt(rr);
+            double rr = cr.true_rr;
+            if (!(rr >= 0.0)) {
+                true_residual(c, A, b, x)();
+                double* h = static_cast<double*>(c->pin);
+                MK_HIP(hipMemcpyAsync(h, &c->state.p->true_rr, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+                MK_HIP(hipStreamSynchronize(c->stream));
+                rr = *h;
+            }
+            res.rel_residual = cr.bb > 0 ? std::sqrt(rr / cr.bb) : std::sqrt(rr);
             res.status = cr.status;
             if (res.status == MK_ERR_NO_CONVERGENCE && res.rel_residual <= o.tol) res.status = MK_OK;
             if (!(res.status == MK_OK && res.rel_residual > o.tol && attempt < 2 && res.iters < o.maxiter))
                 break;
             res.refinements++;
         }
+        A->last_iters = res.iters;
         if (res.status == MK_OK && res.rel_residual > o.tol) res.status = MK_ERR_NO_CONVERGENCE;
         return res;
     }

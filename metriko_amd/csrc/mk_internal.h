@@ -89,19 +89,26 @@ struct CgState {
     int status;     // MK_OK / MK_ERR_NOT_SPD / MK_ERR_NAN
     int it;         // iterations taken
     int first;      // 1 until the first beta of the fused FP32-multigrid iteration
+    double rr0;     // ||r||^2 at the start
+    double true_rr; // ||b - A x||^2 recomputed behind a batch that is expected to converge
 };
 
 // Iterations to launch before the next host convergence check.  Iterations launched past
-// convergence return at once, but each still costs its few dozen launches (about a third of
-// a multigrid PCG iteration), so after the first check interval the count is predicted: the
-// residual's geometric decrease per iteration since the previous check, extrapolated to the
-// target (rounded up), within [1, interval].  An iteration stops where it would stop with
-// any batching, so results do not depend on the prediction.  The solvers use interval 1 in
-// kernel-timing mode, so the per-kernel averages hold no launch past convergence.
+// convergence return at once, but each still costs its launches (about a third of a multigrid
+// PCG iteration on a large system, more than half on a small one), and every check costs a
+// round trip to the host of about 20 us.  The first batch takes as many iterations as the
+// operator's last solve needed (kFirst without one), at most the interval; after that the count is
+// predicted: the residual's geometric decrease per iteration since the previous check,
+// extrapolated to the target (rounded up).  While it says two intervals or more, half of it is
+// launched (up to kAhead intervals).  An iteration stops where it would stop with any batching, so
+// results do not depend on the prediction.  The solvers use interval 1 in kernel-timing mode, so
+// the per-kernel averages hold no launch past convergence.
 struct BatchPlanner {
+    static constexpr int kFirst = 4, kAhead = 8;
     int interval;
     int prev_it = -1;
     double prev_rr = 0.0;
+    bool last = false;  // the planned batch is expected to converge
     explicit BatchPlanner(int iv) : interval(iv > 0 ? iv : 1) {}
     // iterations needed from rr to reach target at the rate seen since (prev_it, prev_rr); 0 =
     // no prediction
@@ -112,14 +119,23 @@ struct BatchPlanner {
         return std::log(target / rr) / rate;
     }
     static int clamp_need(double nd, int interval) {
-        if (!(nd > 0.0) || nd >= double(interval)) return interval;
-        return std::max(1, int(std::ceil(nd)));
+        if (!(nd > 0.0)) return interval;
+        if (nd >= 2.0 * interval) return int(std::min(0.5 * nd, double(kAhead) * interval));
+        return nd >= double(interval) ? interval : std::max(1, int(std::ceil(nd)));
     }
-    int next(int it, double rr, double target) {
-        const int b = clamp_need(need(it, rr, prev_it, prev_rr, target), interval);
+    // hint: iterations of the operator's last solve (0: none)
+    int first(int hint) {
+        last = hint > 0 && hint <= interval;
+        return std::min(interval, hint > 0 ? hint : kFirst);
+    }
+    // rr0: the residual before the first iteration (what the first check compares with)
+    int next(int it, double rr, double rr0, double target) {
+        if (prev_it < 0) { prev_it = 0; prev_rr = rr0; }
+        const double nd = need(it, rr, prev_it, prev_rr, target);
         prev_it = it;
         prev_rr = rr;
-        return b;
+        last = nd > 0.0 && nd <= double(interval);
+        return interval == 1 ? 1 : clamp_need(nd, interval);
     }
 };
 
@@ -131,7 +147,7 @@ struct Work {
 
 // batched (multi-right-hand-side) solves (block.hip): up to 64 columns, row-major blocks
 struct BState {
-    double rz[64], rr[64], bb[64], alpha[64], beta[64];
+    double rz[64], rr[64], rr0[64], bb[64], alpha[64], beta[64];
     int done[64], status[64], it[64];
     int all_done, ndone;  // every column finished; columns finished so far
     double tol2;
@@ -205,6 +221,8 @@ struct mk_ctx {
     mk::DevBuf<double> partials;
     mk::DevBuf<mk::CgState> state;
     mk::DevBuf<double> scal;   // general device scalars
+    void* pin = nullptr;       // page-locked host memory the solvers' states are read back into
+    static constexpr size_t kPinBytes = 8192;
     // SpMV timing (events around each SpMV launch when enabled), attributed per
     // "operator label:kernel:precision" key
     bool time_spmv = false;
@@ -243,6 +261,9 @@ struct mk_op {
         double spmv_bytes = 0.0;
     };
     std::vector<Graph> graphs;
+    // iterations of the last solve / block solve: how many the next one launches before it first
+    // looks (BatchPlanner); nothing else depends on them
+    mutable int last_iters = 0, last_block_iters = 0;
     ~mk_op() {
         for (auto& g : graphs) if (g.exec) (void)hipGraphExecDestroy(g.exec);
         if (mg) mk::mg_free(mg);
@@ -347,20 +368,15 @@ void reduce_partials(mk_ctx* c, const double* partials, int np, int K, double* o
 
 // vector kernels (len = number of scalar entries; complex vectors count 2 per element)
 void axpby64(mk_ctx* c, size_t len, double a, const double* x, double b, double* y);  // y = a x + b y
-void scale_dev64(mk_ctx* c, size_t len, const double* s_dev, int invert_sqrt, double* y);
 void dot64(mk_ctx* c, size_t len, const double* x, const double* y, double* out_dev);  // real dot of interleaved
 void mass_mul(mk_ctx* c, int n, const double* mass, const double* u, double* b);      // complex b = M u
 void mass_dot(mk_ctx* c, int n, const double* mass, const double* x, double* out_dev); // x^H M x
 void cvt64to32_scaled(mk_ctx* c, size_t len, const double* x, const double* s_dev, float* y); // y = x / sqrt(s)
 void add32to64_scaled(mk_ctx* c, size_t len, const float* d, const double* s_dev, double* x);  // x += sqrt(s) d
 
-// CG on the device: solves A x = b for FP64 (x,b device) -- returns status, iterations
-struct CgResult { int status; int iters; double rr; double bb; };
-CgResult cg64(mk_ctx* c, const mk_op* A, const double* b, double* x, double rel_tol, int maxiter, bool jacobi,
-              int check_every, bool x_is_zero, Mg* mg = nullptr);
-CgResult cg32(mk_ctx* c, const mk_op* A, const float* b, float* x, double rel_tol, int maxiter, bool jacobi,
-              int check_every, Mg* mg = nullptr);
-
+// A PCG run on the device: status, iterations, ||r||^2, ||b||^2.
+// true_rr: ||b - A x||^2 recomputed after the last iteration; negative: not computed
+struct CgResult { int status; int iters; double rr; double bb; double true_rr = -1.0; };
 // refinement driver: x (device FP64) warm start, b device FP64; pre overrides A's own multigrid.
 // target (when below o.tol): the relative residual the iteration aims at; the result only has
 // to meet o.tol, so a target under the FP64 floor of the true residual costs no restarts.
