@@ -406,32 +406,42 @@ struct Fp32Gather {
         else { xr = double(z[c]); xi = 0.0; }
     }
 };
+// the row's own entries of z, p and q, loaded while its gathers are in flight
 template <bool CPLX>
-__global__ void __launch_bounds__(256) cgm_spmv(SellDev<double> A, const float* __restrict__ z32,
-                                              double* __restrict__ p, double* __restrict__ q,
+struct CgmOperands {
+    static constexpr int W = CPLX ? 2 : 1;
+    const float* __restrict__ z32;
+    const double* __restrict__ p;
+    const double* __restrict__ q;
+    double zv[W], pv[W], qv[W];
+    __device__ __forceinline__ void operator()(int row) {
+#pragma unroll
+        for (int k = 0; k < W; k++) {
+            zv[k] = double(z32[W * row + k]);
+            pv[k] = p[W * row + k];
+            qv[k] = q[W * row + k];
+        }
+    }
+};
+template <bool CPLX>
+__global__ void __launch_bounds__(256) cgm_spmv(SellDev<double> A, const float* __restrict__ z32, double* p, double* q,
                                               double* __restrict__ zold, CgState* st, double* partials) {
     if (st->done) return;
+    constexpr int W = CPLX ? 2 : 1;
     const double beta = st->beta;
     double contrib = 0.0;
     for (int vb = blockIdx.x; vb < A.nvb; vb += gridDim.x) {
         int row = 0;
-        double ar, ai;
-        if (!spmv_row_g<double, CPLX>(A, Fp32Gather<CPLX>{z32}, vb, row, ar, ai)) continue;
-        if constexpr (CPLX) {
-            const double z0 = double(z32[2 * row]), z1 = double(z32[2 * row + 1]);
-            const double p0 = z0 + beta * p[2 * row], p1 = z1 + beta * p[2 * row + 1];
-            const double q0 = ar + beta * q[2 * row], q1 = ai + beta * q[2 * row + 1];
-            p[2 * row] = p0; p[2 * row + 1] = p1;
-            q[2 * row] = q0; q[2 * row + 1] = q1;
-            zold[2 * row] = z0; zold[2 * row + 1] = z1;
-            contrib += p0 * q0 + p1 * q1;
-        } else {
-            const double z0 = double(z32[row]);
-            const double p0 = z0 + beta * p[row], q0 = ar + beta * q[row];
-            p[row] = p0;
-            q[row] = q0;
-            zold[row] = z0;
-            contrib += p0 * q0;
+        double a[2];
+        CgmOperands<CPLX> o{z32, p, q};
+        if (!spmv_row_gp<double, CPLX>(A, Fp32Gather<CPLX>{z32}, vb, row, a[0], a[1], o)) continue;
+#pragma unroll
+        for (int k = 0; k < W; k++) {
+            const double pk = o.zv[k] + beta * o.pv[k], qk = a[k] + beta * o.qv[k];
+            p[W * row + k] = pk;
+            q[W * row + k] = qk;
+            zold[W * row + k] = o.zv[k];
+            contrib += pk * qk;
         }
     }
     double v[1] = {contrib};

@@ -137,13 +137,82 @@ struct NoPrefetch {
     __device__ __forceinline__ void operator()(int) {}
 };
 
+// Entry e of a value array (complex: both parts in one load; the arrays are the library's own
+// allocations, so pairs are aligned).
+template <typename T, bool CPLX>
+struct MatVal {
+    T r, i;
+    __device__ __forceinline__ void load(const T* __restrict__ v, int64_t e) {
+        if constexpr (!CPLX) { r = v[e]; i = T(0); }
+        else if constexpr (sizeof(T) == 8) { const double2 t = reinterpret_cast<const double2*>(v)[e]; r = t.x; i = t.y; }
+        else { const float2 t = reinterpret_cast<const float2*>(v)[e]; r = t.x; i = t.y; }
+    }
+    __device__ __forceinline__ void fma(T xr, T xi, T& ar, T& ai) const {
+        if constexpr (CPLX) { ar += r * xr - i * xi; ai += r * xi + i * xr; }
+        else { ar += r * xr; }
+    }
+};
+
+// One SELL row: every column index first (w <= kSellMaxLen), then the gathers.  w and the slice's
+// base are the wavefront's, STRIDE (the slice height) a constant where it is 64, so an entry is one
+// load with an immediate offset and the width test a scalar branch.
+template <typename T, bool CPLX, typename G>
+__device__ __forceinline__ void sell_row(const int* __restrict__ col, const T* __restrict__ val, int lane, int stride,
+                                         int w, const G& g, T& ar, T& ai) {
+    int ci[kSellMaxLen];
+#pragma unroll
+    for (int j = 0; j < kSellMaxLen; j++)
+        if (j < w) ci[j] = col[j * stride + lane];
+#pragma unroll
+    for (int j = 0; j < kSellMaxLen; j++)
+        if (j < w) {
+            MatVal<T, CPLX> v;
+            v.load(val, j * stride + lane);
+            T xr, xi;
+            g(ci[j], xr, xi);
+            v.fma(xr, xi, ar, ai);
+        }
+}
+
+// A lane's share of a medium row, entries k0 + sub, k0 + sub + L, ...: U at a time, summed in order;
+// past the end the lane's first entry is taken again with a zero value, so there is no branch.
+template <typename T, bool CPLX, int L, typename G>
+__device__ __forceinline__ void mid_row(const int* __restrict__ col, const T* __restrict__ val, int rem, const G& g, T& ar,
+                                        T& ai) {
+    constexpr int U = 4;
+    for (; rem > 0; rem -= U * L, col += U * L, val += U * L * (CPLX ? 2 : 1)) {
+        int c[U];
+        MatVal<T, CPLX> v[U];
+        T xr[U], xi[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int q = u * L < rem ? u * L : 0;
+            c[u] = col[q];
+            v[u].load(val, q);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) g(c[u], xr[u], xi[u]);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (u * L >= rem) { v[u].r = T(0); v[u].i = T(0); xr[u] = T(0); xi[u] = T(0); }
+            v[u].fma(xr[u], xi[u], ar, ai);
+        }
+    }
+}
+
 // Computes one row of A x for virtual block vb (uniform in the block), x given by a gather.
-// Returns true in the thread that owns the result (row, ar, ai).  pre(row) is called as soon
-// as the row is known -- for the SELL rows before their column loads -- so that the caller's
-// row-local operands (right-hand side, diagonal, vectors updated in place) are in flight
-// together with the gathers instead of after them.
+// Returns true in the thread that owns the result (row, ar, ai).  pre(row) is called in that thread
+// as soon as the row is known, before any column is loaded, so that the caller's row-local
+// operands (right-hand side, diagonal, vectors updated in place) are in flight together with the
+// gathers instead of after them.
+//
+// Up to about 100,000 rows these kernels are bound by the instructions a wavefront issues, not by
+// memory: an empty kernel takes 1.6 us, one with four dependent loads 2.2, and with 64-bit vector
+// addresses, a runtime slice height and a divergent test per entry a smoothing step took 4.1 us
+// on 4,900 rows of 5 and, with one column and gather at a time, 6.2 us on 9,683 rows of 12.
 template <typename T, bool CPLX, typename G, typename P>
 __device__ __forceinline__ bool spmv_row_gp(const SellDev<T>& A, const G& g, int vb, int& row, T& ar, T& ai, P& pre) {
+    constexpr int W = CPLX ? 2 : 1;
     ar = 0;
     ai = 0;
     // the long rows' blocks come first: their wavefronts run the longest chains, so they start
@@ -154,62 +223,42 @@ __device__ __forceinline__ bool spmv_row_gp(const SellDev<T>& A, const G& g, int
     }
     if (vb < A.nb_sell) {
         const int r = vb * blockDim.x + threadIdx.x;
-        if (r >= A.n_short) return false;
-        const int s = r / A.C, lane = r - s * A.C;
-        const int64_t base = A.slice_ptr[s] + lane;
+        // the slice is the wavefront's (C is a multiple of 64): its position is a scalar load
+        const int r0 = __builtin_amdgcn_readfirstlane(r);
+        if (r0 >= A.n_short) return false;
+        const int s = A.C == 64 ? r0 >> 6 : r0 / A.C;
+        const int64_t base = A.slice_ptr[s];
         const int w = A.slice_w[s];
+        if (r >= A.n_short) return false;
         row = A.perm ? A.perm[r] : r;
         pre(row);
-        // every column index first (w <= kSellMaxLen), then the gathers: two memory latencies
-        // per row instead of two per entry
-        int ci[kSellMaxLen];
-#pragma unroll
-        for (int j = 0; j < kSellMaxLen; j++)
-            if (j < w) ci[j] = A.col[base + int64_t(j) * A.C];
-#pragma unroll
-        for (int j = 0; j < kSellMaxLen; j++) {
-            if (j < w) {
-                const int64_t e = base + int64_t(j) * A.C;
-                T xr, xi;
-                g(ci[j], xr, xi);
-                if constexpr (CPLX) {
-                    const T vr = A.val[2 * e], vi = A.val[2 * e + 1];
-                    ar += vr * xr - vi * xi;
-                    ai += vr * xi + vi * xr;
-                } else {
-                    ar += A.val[e] * xr;
-                }
-            }
-        }
+        const int* col = A.col + base;
+        const T* val = A.val + base * W;
+        if (A.C == 64) sell_row<T, CPLX>(col, val, r & 63, 64, w, g, ar, ai);
+        else sell_row<T, CPLX>(col, val, r - s * A.C, A.C, w, g, ar, ai);
         return true;
     }
     if (vb < A.nb_sell + A.nb_mid) {  // medium rows: a group of mid_lanes lanes per row
         const int L = A.mid_lanes;
         const int t = (vb - A.nb_sell) * int(blockDim.x) + int(threadIdx.x);
-        const int m = t / L, sub = t - m * L;
+        const int m = L == 4 ? t >> 2 : L == 8 ? t >> 3 : t >> 4, sub = t & (L - 1);
         if (m < A.nmid) {
-            for (int64_t k = A.mid_ptr[m] + sub; k < A.mid_ptr[m + 1]; k += L) {
-                const int c = A.mid_col[k];
-                T xr, xi;
-                g(c, xr, xi);
-                if constexpr (CPLX) {
-                    const T vr = A.mid_val[2 * k], vi = A.mid_val[2 * k + 1];
-                    ar += vr * xr - vi * xi;
-                    ai += vr * xi + vi * xr;
-                } else {
-                    ar += A.mid_val[k] * xr;
-                }
-            }
+            const int64_t k = A.mid_ptr[m] + sub;
+            const int rem = int(A.mid_ptr[m + 1] - k);
+            row = A.mid_rows[m];
+            if (sub == 0) pre(row);
+            const int* col = A.mid_col + k;
+            const T* val = A.mid_val + k * W;
+            if (L == 4) mid_row<T, CPLX, 4>(col, val, rem, g, ar, ai);
+            else if (L == 8) mid_row<T, CPLX, 8>(col, val, rem, g, ar, ai);
+            else mid_row<T, CPLX, 16>(col, val, rem, g, ar, ai);
         }
         // reduce inside the group (every lane takes part; L divides 64)
         for (int off = L >> 1; off > 0; off >>= 1) {
             ar += __shfl_xor(ar, off, 64);
             if constexpr (CPLX) ai += __shfl_xor(ai, off, 64);
         }
-        if (m >= A.nmid || sub != 0) return false;
-        row = A.mid_rows[m];
-        pre(row);
-        return true;
+        return m < A.nmid && sub == 0;
     }
     const int w = (vb - A.nb_sell - A.nb_mid) * int(blockDim.x >> 6) + int(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
@@ -220,14 +269,12 @@ __device__ __forceinline__ bool spmv_row_gp(const SellDev<T>& A, const G& g, int
         constexpr int U = CPLX ? 2 : 8;
         const int64_t kend = A.long_ptr[w + 1];
         int64_t k = A.long_ptr[w] + lane;
+        row = A.long_rows[w];
+        if (lane == 0) pre(row);
         auto add = [&](int64_t q, T xr, T xi) {
-            if constexpr (CPLX) {
-                const T vr = A.long_val[2 * q], vi = A.long_val[2 * q + 1];
-                ar += vr * xr - vi * xi;
-                ai += vr * xi + vi * xr;
-            } else {
-                ar += A.long_val[q] * xr;
-            }
+            MatVal<T, CPLX> v;
+            v.load(A.long_val, q);
+            v.fma(xr, xi, ar, ai);
         };
         for (; k + (U - 1) * 64 < kend; k += U * 64) {
             T xr[U], xi[U];
@@ -243,8 +290,6 @@ __device__ __forceinline__ bool spmv_row_gp(const SellDev<T>& A, const G& g, int
         }
         ar = wave_sum_t(ar);
         if constexpr (CPLX) ai = wave_sum_t(ai);
-        row = A.long_rows[w];
-        if (lane == 0) pre(row);
         return lane == 0;
     }
     return false;
