@@ -1014,21 +1014,23 @@ __global__ void __launch_bounds__(256) sell_spmv2(SellDev<T> A, int m1, const T*
 }
 
 template <typename T>
-void spmv2_launch(mk_ctx* c, const mk_op* A, int m1, const T* u, const T* v, T* y, const int* skip) {
+void spmv2_launch(mk_ctx* c, const mk_op* A, int m1, const T* u, const T* v, T* y, const int* skip, const char* name) {
     unsigned g = 0;
     const T* val;
     if constexpr (std::is_same<T, double>::value) val = A->val64.p;
     else val = A->val32.p;
     const SellDev<T> D = sell_dev<T>(A, val, A->block, &g);
-    SpmvTimer tm(c, sizeof(T) == 8 ? A->bytes64 : A->bytes32, A, "restrict_resid", sizeof(T) == 4);
+    SpmvTimer tm(c, sizeof(T) == 8 ? A->bytes64 : A->bytes32, A, name, sizeof(T) == 4);
     if (A->cplx)
         MK_TLAUNCH(tm, 0, (sell_spmv2<T, true>), dim3(g), dim3(A->block), 0, c->stream, D, m1, u, v, y, skip);
     else
         MK_TLAUNCH(tm, 0, (sell_spmv2<T, false>), dim3(g), dim3(A->block), 0, c->stream, D, m1, u, v, y, skip);
     MK_HIP(hipGetLastError());
 }
-template void spmv2_launch<double>(mk_ctx*, const mk_op*, int, const double*, const double*, double*, const int*);
-template void spmv2_launch<float>(mk_ctx*, const mk_op*, int, const float*, const float*, float*, const int*);
+template void spmv2_launch<double>(mk_ctx*, const mk_op*, int, const double*, const double*, double*, const int*,
+                                   const char*);
+template void spmv2_launch<float>(mk_ctx*, const mk_op*, int, const float*, const float*, float*, const int*,
+                                  const char*);
 
 template <typename T>
 __global__ void k_copy(size_t len, const T* __restrict__ x, T* __restrict__ y, const int* skip) {

@@ -32,6 +32,9 @@ struct MgLevel {
     mk_op* P = nullptr;  // n_l x n_{l+1}
     mk_op* R = nullptr;  // n_{l+1} x n_l
     mk_op* RR = nullptr; // n_{l+1} x 2 n_l: [R | -R A] (restriction of the residual in one product)
+    // the whole level as two products (explicit_level): b_c = W b, x = M [b; x_c]; null: smoothed
+    mk_op* W = nullptr;  // n_{l+1} x n_l
+    mk_op* M = nullptr;  // n_l x (n_l + n_{l+1})
     double lmax = 2.0;
     int n = 0;
     DevBuf<double> b64, x64, r64, d64, y64;  // y: second iterate buffer of the fused smoother
@@ -57,6 +60,8 @@ void mg_free(Mg* g) {
         delete L.P;
         delete L.R;
         delete L.RR;
+        delete L.W;
+        delete L.M;
     }
     delete g;
 }
@@ -69,6 +74,9 @@ struct MgTune {
     // Largest level the device solves by its dense inverse (the coarse_ limits above are the host
     // solve's): see build_impl.
     int dense_real = 2400, dense_cplx = 2100;
+    // Largest level run as two explicit products: rows, and bytes of its FP32 operator M (see
+    // explicit_level)
+    int explicit_rows = 131072, explicit_mb = 64;
 };
 static const MgTune& tune() {
     static const MgTune t = [] {
@@ -86,6 +94,8 @@ static const MgTune& tune() {
         i("METRIKO_MG_COARSE_CPLX", x.coarse_cplx);
         i("METRIKO_MG_DENSE_REAL", x.dense_real);
         i("METRIKO_MG_DENSE_CPLX", x.dense_cplx);
+        i("METRIKO_MG_EXPLICIT", x.explicit_rows);
+        i("METRIKO_MG_EXPLICIT_MB", x.explicit_mb);
         i("METRIKO_MG_SMOOTH_LONG", x.smooth_long);
         i("METRIKO_MG_COMPAT", x.compat);
         i("METRIKO_MG_L1", x.l1);
@@ -579,12 +589,27 @@ mk_op* upload(mk_ctx* c, const Csr<T>& A, const mk_solve_opts& o, const int* rsr
 template <typename T>
 struct HostHier {
     std::vector<Csr<T>> A, P, R, RR;
+    std::vector<uint8_t> any_long;  // per level but the coarsest: it has long rows
     std::vector<double> lmax;
     std::vector<std::vector<double>> dinv;
     std::vector<double> inv;  // coarsest dense inverse (row-major, complex interleaved; host solves only)
     // per level but the coarsest: the coarse unknown that stands for each node's aggregate
     // (the first column of its tentative prolongator row; -1 for an empty row)
     std::vector<std::vector<int>> key;
+};
+
+// Chebyshev(2) coefficients on [lmax / lmin_div, lmax]: first step d_1 = c0 D^-1 r, second step
+// d_2 = a d_1 + s D^-1 r.
+struct Cheb2 {
+    double c0, a, s;
+    explicit Cheb2(double lmax) {
+        const double lmin = lmax / tune().lmin_div, theta = 0.5 * (lmax + lmin), delta = 0.5 * (lmax - lmin),
+                     sigma = theta / delta;
+        const double rho0 = 1.0 / sigma, rho1 = 1.0 / (2.0 * sigma - rho0);
+        c0 = 1.0 / theta;
+        a = rho1 * rho0;
+        s = 2.0 * rho1 / delta;
+    }
 };
 
 // Locality order of every level from the aggregates: the coarsest level keeps its order, and
@@ -616,8 +641,8 @@ std::vector<std::vector<int>> hier_order(const HostHier<T>& H) {
 }
 
 template <typename T>
-HostHier<T> build_host(Csr<T> A, double theta, int finest_max, int coarse_max, bool host_inverse, const std::vector<T>* B0 = nullptr,
-                       int nb = 0) {
+HostHier<T> build_host(Csr<T> A, double theta, int finest_max, int coarse_max, bool host_inverse,
+                       const std::vector<T>* B0 = nullptr, int nb = 0) {
     HostHier<T> H;
     const bool cplx = !std::is_same<T, double>::value;
     std::vector<T> B;
@@ -806,6 +831,7 @@ HostHier<T> build_host(Csr<T> A, double theta, int finest_max, int coarse_max, b
             }
             // exact Hermitian symmetry of the coarse operator
             hermitian_average(Ac);
+            H.any_long.push_back(any_long ? 1 : 0);
             H.A.push_back(std::move(A));
             H.P.push_back(std::move(P));
             H.R.push_back(std::move(R));
@@ -863,7 +889,21 @@ Mg* build_impl(mk_ctx* c, Csr<T>&& A0, const mk_solve_opts& o, double theta, int
             L.lmax = H.lmax[l];
             // the coarsest operator is only needed as its inverse
             const bool last = l + 1 == H.A.size();
-            if (!last) {
+            // small levels without long rows run as two products (long rows, coupled to a whole seam,
+            // would fill them); orders are only asked for on larger operators
+            bool expl = false;
+            if (!last && pos.empty() && H.A[l].nr <= tune().explicit_rows && g->deg == 2 && !H.any_long[l]) {
+                const Cheb2 ch(L.lmax);
+                auto view = [](const Csr<T>& A) {
+                    return HostCsr{A.nr, A.ptr.data(), A.col.data(), reinterpret_cast<const double*>(A.val.data())};
+                };
+                expl = explicit_level(c, g->cplx, view(H.A[l]), view(H.P[l]), view(H.R[l]), H.dinv[l].data(),
+                                      (1.0 + ch.a) * ch.c0 + ch.s, ch.s * ch.c0, double(tune().explicit_mb) * 1048576.0,
+                                      o.block_size, &L.W, &L.M);
+            }
+            // an explicit level of a real hierarchy keeps its smoother too: blocks of right-hand
+            // sides are bound by bytes and use that
+            if (!last && !(expl && g->cplx)) {
                 L.A = upload(c, H.A[l], o, I_(l), P_(l));
                 // the smoother's inverse diagonal replaces the plain one
                 std::vector<double> dv = H.dinv[l];
@@ -875,7 +915,7 @@ Mg* build_impl(mk_ctx* c, Csr<T>&& A0, const mk_solve_opts& o, double theta, int
                 MK_HIP(hipStreamSynchronize(c->stream));
             }
             g->nnz_total += H.A[l].nonZeros();
-            if (l < H.P.size()) {
+            if (l < H.P.size() && !(expl && g->cplx)) {
                 L.P = upload(c, H.P[l], o, I_(l), P_(l + 1));
                 L.R = upload(c, H.R[l], o, I_(l + 1), P_(l));
                 if (l < H.RR.size()) {
@@ -1024,10 +1064,16 @@ void vcycle(mk_ctx* c, Mg* g, int l, const T* b, T* x, const int* skip) {
         g->coarse.apply<T>(c, b, x, skip);
         return;
     }
-    chebyshev<T>(c, g, L, b, x, true, skip);
     MgLevel& Cn = g->lv[size_t(l) + 1];
+    if (L.M) {
+        spmv_launch<T>(c, L.W, Sel<T>::val(L.W), b, Sel<T>::b(Cn), nullptr, SPMV_PLAIN, nullptr, Sel<T>::bytes(L.W), skip);
+        vcycle<T>(c, g, l + 1, Sel<T>::b(Cn), Sel<T>::x(Cn), skip);
+        spmv2_launch<T>(c, L.M, L.n, b, Sel<T>::x(Cn), x, skip, "cheb_level");
+        return;
+    }
+    chebyshev<T>(c, g, L, b, x, true, skip);
     if (L.RR) {  // b_c = [R | -R A] [b; x] = R (b - A x) in one launch
-        spmv2_launch<T>(c, L.RR, L.n, b, x, Sel<T>::b(Cn), skip);
+        spmv2_launch<T>(c, L.RR, L.n, b, x, Sel<T>::b(Cn), skip, "restrict_resid");
     } else {
         T* r = Sel<T>::r(L);
         spmv_launch<T>(c, L.A, Sel<T>::val(L.A), x, r, b, SPMV_RESID_NORED, nullptr, Sel<T>::bytes(L.A), skip);
@@ -1231,7 +1277,8 @@ extern "C" mk_status mk_mg_host_pcg(int n, const int64_t* ptr, const int32_t* co
             for (int64_t k = 0; k < ptr[n]; k++) A.val[k] = cd(val[2 * k], val[2 * k + 1]);
             std::vector<cd> B;
             for (size_t q = 0; q < size_t(n) * size_t(nnull); q++) B.emplace_back(nullvec[2 * q], nullvec[2 * q + 1]);
-            HostHier<cd> H = build_host<cd>(Csr<cd>(A), tune().theta_cplx, tune().coarse_cplx, tune().coarse_cplx, true, nnull ? &B : nullptr, nnull);
+            HostHier<cd> H = build_host<cd>(Csr<cd>(A), tune().theta_cplx, tune().coarse_cplx, tune().coarse_cplx, true,
+                                          nnull ? &B : nullptr, nnull);
             if (levels) *levels = int(H.A.size());
             int it = host_pcg<cd>(A, H, reinterpret_cast<const cd*>(b), reinterpret_cast<cd*>(x), tol, maxit, relres);
             if (iters) *iters = it;
@@ -1318,6 +1365,8 @@ void mg_set_labels(Mg* g, const std::string& base) {
         if (g->lv[l].P) g->lv[l].P->label = s + "_P";
         if (g->lv[l].R) g->lv[l].R->label = s + "_R";
         if (g->lv[l].RR) g->lv[l].RR->label = s + "_RR";
+        if (g->lv[l].M) g->lv[l].M->label = s + "_M";
+        if (g->lv[l].W) g->lv[l].W->label = s + "_W";
     }
 }
 double mg_setup_ms(const Mg* g) { return g->setup_ms; }

@@ -171,6 +171,13 @@ struct DenseInverse {
     template <typename T>
     void apply_block(mk_ctx* c, int mw, const T* B, T* X, const int* skip) const;  // n x mw row-major
 };
+// A host CSR matrix (complex: values interleaved)
+struct HostCsr { int rows; const int64_t* ptr; const int* col; const double* val; };
+// One multigrid level as two products, b_c = W b and x = M [b; x_c] (explicit.hip), for the smoother
+// q = alpha D^-1 - beta D^-1 A D^-1; dinv: the smoother's inverse diagonal.  false (nothing built): a
+// row of the products is too long, or M in FP32 takes more than max_bytes
+bool explicit_level(mk_ctx* c, bool cplx, const HostCsr& A, const HostCsr& P, const HostCsr& R, const double* dinv,
+                    double alpha, double beta, double max_bytes, int block, mk_op** W, mk_op** M);
 // multigrid (mg.hip)
 // order_out: store the finest level in the aggregates' locality order and return pos[old] = new
 // there (left empty for a one-level hierarchy); the hierarchy then takes and returns vectors
@@ -333,9 +340,9 @@ void cheb_launch(mk_ctx* c, const mk_op* A, const T* x_in, T* x_out, const T* b,
 // zero-start Chebyshev steps 1+2 fused: x_out = x1 + d, x1 = c0 D^-1 b, d = a x1 + s D^-1 (b - A x1)
 template <typename T>
 void cheb0_launch(mk_ctx* c, const mk_op* A, const T* b, T* x_out, T* d, T c0, T a, T s, const int* skip);
-// y = M [u; v], columns [0, m1) of M act on u, the rest on v
+// y = M [u; v], columns [0, m1) of M act on u, the rest on v (name: the timing key)
 template <typename T>
-void spmv2_launch(mk_ctx* c, const mk_op* A, int m1, const T* u, const T* v, T* y, const int* skip);
+void spmv2_launch(mk_ctx* c, const mk_op* A, int m1, const T* u, const T* v, T* y, const int* skip, const char* name);
 template <typename T>
 void copy_launch(mk_ctx* c, size_t len, const T* x, T* y, const int* skip);
 template <typename T>

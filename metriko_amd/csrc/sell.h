@@ -241,7 +241,7 @@ __device__ __forceinline__ bool spmv_row_gp(const SellDev<T>& A, const G& g, int
     if (vb < A.nb_sell + A.nb_mid) {  // medium rows: a group of mid_lanes lanes per row
         const int L = A.mid_lanes;
         const int t = (vb - A.nb_sell) * int(blockDim.x) + int(threadIdx.x);
-        const int m = L == 4 ? t >> 2 : L == 8 ? t >> 3 : t >> 4, sub = t & (L - 1);
+        const int m = t >> (31 - __builtin_clz(unsigned(L))), sub = t & (L - 1);
         if (m < A.nmid) {
             const int64_t k = A.mid_ptr[m] + sub;
             const int rem = int(A.mid_ptr[m + 1] - k);
@@ -251,7 +251,9 @@ __device__ __forceinline__ bool spmv_row_gp(const SellDev<T>& A, const G& g, int
             const T* val = A.mid_val + k * W;
             if (L == 4) mid_row<T, CPLX, 4>(col, val, rem, g, ar, ai);
             else if (L == 8) mid_row<T, CPLX, 8>(col, val, rem, g, ar, ai);
-            else mid_row<T, CPLX, 16>(col, val, rem, g, ar, ai);
+            else if (L == 16) mid_row<T, CPLX, 16>(col, val, rem, g, ar, ai);
+            else if (L == 32) mid_row<T, CPLX, 32>(col, val, rem, g, ar, ai);
+            else mid_row<T, CPLX, 64>(col, val, rem, g, ar, ai);
         }
         // reduce inside the group (every lane takes part; L divides 64)
         for (int off = L >> 1; off > 0; off >>= 1) {
