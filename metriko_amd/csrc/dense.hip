@@ -10,6 +10,7 @@
 // an operator of condition 1e7 and more to FP32 can make it indefinite, and the size limit below
 // costs no more in FP64 than a smoothed level does.
 #include "mk_internal.h"
+#include "sell.h"
 
 namespace mk {
 
@@ -213,13 +214,21 @@ __global__ void __launch_bounds__(256) k_gj_update(int ld, int k0, double* __res
 
 // x = Inv b: one wavefront per row, 16 bytes of the row per lane and load (two real columns or a
 // complex one; ld is even, so rows stay aligned), kU loads in flight.
-template <typename T, bool CPLX>
+template <typename T, bool CPLX, bool DOTS>
 __global__ void __launch_bounds__(256) k_dense_gemv(int n, int ld, const double* __restrict__ inv,
-                                                    const T* __restrict__ b, T* __restrict__ x, const int* skip) {
+                                                    const T* __restrict__ b, T* __restrict__ x, const int* skip,
+                                                    const double* __restrict__ r, const double* __restrict__ xold,
+                                                    double* __restrict__ partials) {
     if (skip && *skip) return;
-    const int i = blockIdx.x * 4 + int(threadIdx.x >> 6);
+    const int row_ = blockIdx.x * 4 + int(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    if (i >= n) return;  // uniform inside the wavefront
+    const bool in = row_ < n;  // uniform inside the wavefront
+    if (!DOTS && !in) return;
+    const int i = in ? row_ : n - 1;  // a wavefront past the end only takes part in the dots' reduction
+    // the row's entries of r and xold, in flight with the row
+    double rv[2] = {0.0, 0.0}, ov[2] = {0.0, 0.0};
+    if (DOTS && in && lane == 0)
+        for (int q = 0; q < (CPLX ? 2 : 1); q++) { rv[q] = r[(CPLX ? 2 : 1) * i + q]; ov[q] = xold[(CPLX ? 2 : 1) * i + q]; }
     constexpr int kU = 4;
     const double2* __restrict__ row = reinterpret_cast<const double2*>(inv + size_t(i) * ld * (CPLX ? 2 : 1));
     const int nv = CPLX ? n : (n + 1) / 2;  // 16-byte pieces; an odd n's last one ends in the padding
@@ -249,9 +258,13 @@ __global__ void __launch_bounds__(256) k_dense_gemv(int n, int ld, const double*
         ar += __shfl_xor(ar, off, 64);
         if constexpr (CPLX) ai += __shfl_xor(ai, off, 64);
     }
-    if (lane == 0) {
+    if (lane == 0 && in) {
         if constexpr (CPLX) { x[2 * i] = T(ar); x[2 * i + 1] = T(ai); }
         else x[i] = T(ar);
+    }
+    if constexpr (DOTS) {
+        double d[2] = {rv[0] * double(T(ar)) + rv[1] * double(T(ai)), rv[0] * ov[0] + rv[1] * ov[1]};
+        partials_write<2>(d, partials);
     }
 }
 
@@ -344,13 +357,21 @@ DenseInverse::DenseInverse(mk_ctx* c, bool cplx_, int n_, const int64_t* ptr, co
 }
 
 template <typename T>
-void DenseInverse::apply(mk_ctx* c, const T* b, T* x, const int* skip) const {
-    const dim3 g(unsigned((n + 3) / 4));
-    if (cplx) hipLaunchKernelGGL((k_dense_gemv<T, true>), g, dim3(256), 0, c->stream, n, ld, (const double*)inv.p, b, x, skip);
-    else hipLaunchKernelGGL((k_dense_gemv<T, false>), g, dim3(256), 0, c->stream, n, ld, (const double*)inv.p, b, x, skip);
+unsigned DenseInverse::apply(mk_ctx* c, const T* b, T* x, const int* skip, const double* r, const double* xold,
+                             double* partials) const {
+    const unsigned g = unsigned((n + 3) / 4);
+#define MK_GEMV(CP, DOTS)                                                                                               \
+    hipLaunchKernelGGL((k_dense_gemv<T, CP, DOTS>), dim3(g), dim3(256), 0, c->stream, n, ld, (const double*)inv.p, b, x, skip, \
+                       r, xold, partials)
+    if (cplx) { if (r) MK_GEMV(true, true); else MK_GEMV(true, false); }
+    else { if (r) MK_GEMV(false, true); else MK_GEMV(false, false); }
+#undef MK_GEMV
+    return g;
 }
-template void DenseInverse::apply<float>(mk_ctx*, const float*, float*, const int*) const;
-template void DenseInverse::apply<double>(mk_ctx*, const double*, double*, const int*) const;
+template unsigned DenseInverse::apply<float>(mk_ctx*, const float*, float*, const int*, const double*, const double*,
+                                             double*) const;
+template unsigned DenseInverse::apply<double>(mk_ctx*, const double*, double*, const int*, const double*, const double*,
+                                              double*) const;
 
 template <typename T>
 void DenseInverse::apply_block(mk_ctx* c, int mw, const T* B, T* X, const int* skip) const {

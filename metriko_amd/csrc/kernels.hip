@@ -49,64 +49,17 @@ void timing_flush(mk_ctx* c) {
 
 
 // ---- second launch of the two-launch reductions ---------------------------------------------
-// k_finish<K, F>: one block sums the K partials of the nparts blocks of the previous kernel
-// (fixed order) and thread 0 applies F to the totals; F::guard skips it once the CG state is
-// done (the working kernel then left no partials), skip (if set) does the same.
-template <int K, typename F>
-__global__ void __launch_bounds__(1024) k_finish(CgState* st, const double* __restrict__ partials, int nparts,
-                                                 double* out, const int* skip) {
+// k_finish: one block sums the partials of the nparts blocks of the previous kernel (fixed order).
+__global__ void __launch_bounds__(1024) k_finish(const double* __restrict__ partials, int nparts, double* out,
+                                                 const int* skip) {
     if (skip && *skip) return;
-    if (F::guard && st->done) return;
-    double tot[K];
-    partials_sum<K>(partials, nparts, tot);
-    if (threadIdx.x == 0) F::apply(st, tot, out);
+    double tot[1];
+    partials_sum<1>(partials, nparts, tot);
+    if (threadIdx.x == 0) out[0] = tot[0];
 }
-struct FinOut {  // plain total
-    static constexpr bool guard = false;
-    __device__ static void apply(CgState*, const double* tot, double* out) { out[0] = tot[0]; }
-};
-struct FinCgAlpha {  // pq -> alpha
-    static constexpr bool guard = true;
-    __device__ static void apply(CgState* st, const double* tot, double*) {
-        st->pq = tot[0];
-        if (!(tot[0] > 0.0)) {
-            st->status = (tot[0] == tot[0]) ? MK_ERR_NOT_SPD : MK_ERR_NAN;
-            st->done = 1;
-        } else {
-            st->alpha = st->rz / tot[0];
-        }
-    }
-};
-struct FinCgUpdate {  // rz, rr after the x / r / z update -> beta, convergence
-    static constexpr bool guard = true;
-    __device__ static void apply(CgState* st, const double* tot, double*) {
-        st->beta = tot[0] / st->rz;
-        st->rz = tot[0];
-        st->rr = tot[1];
-        st->it += 1;
-        if (!(tot[1] == tot[1]) || !(tot[0] == tot[0])) { st->status = MK_ERR_NAN; st->done = 1; }
-        else if (tot[1] <= st->tol2 * st->bb) st->done = 1;
-    }
-};
-struct FinCgRr {  // rr after the x / r update -> convergence
-    static constexpr bool guard = true;
-    __device__ static void apply(CgState* st, const double* tot, double*) {
-        st->rr = tot[0];
-        st->it += 1;
-        if (!(tot[0] == tot[0])) { st->status = MK_ERR_NAN; st->done = 1; }
-        else if (tot[0] <= st->tol2 * st->bb) st->done = 1;
-    }
-};
-struct FinCgBeta {  // rz of the preconditioned residual -> beta
-    static constexpr bool guard = true;
-    __device__ static void apply(CgState* st, const double* tot, double*) {
-        if (!(tot[0] > 0.0)) { st->status = (tot[0] == tot[0]) ? MK_ERR_NOT_SPD : MK_ERR_NAN; st->done = 1; }
-        else { st->beta = tot[0] / st->rz; st->rz = tot[0]; }
-    }
-};
-template <int K, typename F>
-static inline void finish(mk_ctx* c, unsigned nparts, double* out = nullptr, const int* skip = nullptr) {
-    hipLaunchKernelGGL((k_finish<K, F>), dim3(1), dim3(1024), 0, c->stream, c->state.p, (const double*)c->partials.p,
+static inline void finish(mk_ctx* c, unsigned nparts, double* out, const int* skip = nullptr,
+                          const double* partials = nullptr) {
+    hipLaunchKernelGGL(k_finish, dim3(1), dim3(1024), 0, c->stream, partials ? partials : (const double*)c->partials.p,
                        int(nparts), out, skip);
 }
 
@@ -138,15 +91,14 @@ __global__ void __launch_bounds__(256) sell_spmv(SellDev<T> A, const T* __restri
         if constexpr (CPLX) {
             if constexpr (MODE == 2 || MODE == 3) { ar = re.v[0] - ar; ai = re.v[1] - ai; }
             if constexpr (MODE == 4) { ar += re.v[0]; ai += re.v[1]; }
-            y[2 * row] = ar;
-            y[2 * row + 1] = ai;
+            if (MODE != 2 || y) { y[2 * row] = ar; y[2 * row + 1] = ai; }  // residual norm alone: no y
             if constexpr (MODE == 1) contrib += double(re.v[0]) * double(ar) + double(re.v[1]) * double(ai);
             if constexpr (MODE == 2) contrib += double(ar) * double(ar) + double(ai) * double(ai);
         } else {
             T a = ar;
             if constexpr (MODE == 2 || MODE == 3) a = re.v[0] - a;
             if constexpr (MODE == 4) a += re.v[0];
-            y[row] = a;
+            if (MODE != 2 || y) y[row] = a;
             if constexpr (MODE == 1) contrib += double(re.v[0]) * double(a);
             if constexpr (MODE == 2) contrib += double(a) * double(a);
         }
@@ -187,66 +139,194 @@ __global__ void __launch_bounds__(256) cg_init(int n, const T* __restrict__ r, c
     partials_write<3>(v, partials);
 }
 
-// q = A p ; pq = p^H q ; alpha = rz / pq
+// One iteration is cg_step1 (p = z + beta p ; q = A p ; p^H q) and cg_step2 (x += alpha p ;
+// r -= alpha q ; with Jacobi z = dinv r and rz), plus, with an external preconditioner, its
+// application and cg_beta (rz).  The scalars between them: rz in row 0 of the partials, rr in row 1,
+// p^H q in row 2.  Up to kFoldParts blocks every block of the kernel that needs a scalar adds the
+// previous kernel's partials itself, in the same order (the same value in every block, one block
+// stores what the host reads); above that, one-block kernels add them in between.  A one-block
+// kernel costs 2.3 to 3 us, a fold of 200 partials 0.6: with folds and the update of p inside the
+// product (from the old p of the gathered rows; p alternates between two buffers) a Jacobi
+// iteration on 50,953 rows went from five launches of 18.4 us to two of 9.
+static constexpr unsigned kFoldParts = 2048;
+static constexpr int kRowRz = 0, kRowRr = 1, kRowPq = 2;
+
+// The gathered p = z + beta p_old, never stored before it is used
 template <typename T, bool CPLX>
-__global__ void __launch_bounds__(256) cg_spmv(SellDev<T> A, const T* __restrict__ p, T* __restrict__ q,
-                                             const CgState* st, double* partials) {
+struct DirectionGather {
+    const T* __restrict__ z;
+    const T* __restrict__ p;
+    T beta;
+    __device__ __forceinline__ void operator()(int c, T& xr, T& xi) const {
+        if constexpr (CPLX) { xr = z[2 * c] + beta * p[2 * c]; xi = z[2 * c + 1] + beta * p[2 * c + 1]; }
+        else { xr = z[c] + beta * p[c]; xi = T(0); }
+    }
+};
+template <typename T, bool CPLX>
+struct DirectionOperands {
+    static constexpr int W = CPLX ? 2 : 1;
+    const T* __restrict__ z;
+    const T* __restrict__ p;
+    T zv[W], pv[W];
+    __device__ __forceinline__ void operator()(int row) {
+#pragma unroll
+        for (int q = 0; q < W; q++) { zv[q] = z[W * row + q]; pv[q] = p[W * row + q]; }
+    }
+};
+
+// nin: partials of rz (Jacobi: and rr) to fold (0: the state holds beta).  The iteration's rz goes to
+// st->rz_new, which no block of this launch reads; cg_step2 moves it to st->rz, which none of its
+// blocks reads.
+template <typename T, bool CPLX, bool JAC>
+__global__ void __launch_bounds__(256) cg_step1(SellDev<T> A, const T* __restrict__ z, const T* __restrict__ p,
+                                              T* __restrict__ pn, T* __restrict__ q, CgState* st, double* partials, int nin) {
     if (st->done) return;
+    constexpr int W = CPLX ? 2 : 1;
+    const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+    T beta;
+    if (nin) {
+        double tot[JAC ? 2 : 1];
+        partials_sum<JAC ? 2 : 1>(partials, nin, tot);
+        const double rz = tot[0];
+        bool stop = false;
+        if constexpr (JAC) {
+            const double rr = tot[1];
+            const bool nan = !(rr == rr) || !(rz == rz);
+            stop = nan || rr <= st->tol2 * st->bb;
+            if (writer) {
+                st->rr = rr;
+                st->it += 1;
+                if (nan) st->status = MK_ERR_NAN;
+                if (stop) st->done = 1;
+            }
+        } else {
+            stop = !(rz > 0.0);
+            if (writer && stop) { st->status = (rz == rz) ? MK_ERR_NOT_SPD : MK_ERR_NAN; st->done = 1; }
+        }
+        if (stop) return;
+        beta = T(rz / st->rz);
+        if (writer) st->rz_new = rz;
+    } else {
+        beta = T(st->beta);
+        if (writer) st->rz_new = st->rz;
+    }
     double contrib = 0.0;
     for (int vb = blockIdx.x; vb < A.nvb; vb += gridDim.x) {
         int row = 0;
-        T ar, ai;
-        if (!spmv_row<T, CPLX>(A, p, vb, row, ar, ai)) continue;
-        if constexpr (CPLX) {
-            q[2 * row] = ar;
-            q[2 * row + 1] = ai;
-            contrib += double(p[2 * row]) * double(ar) + double(p[2 * row + 1]) * double(ai);
-        } else {
-            q[row] = ar;
-            contrib += double(p[row]) * double(ar);
+        T a[2];
+        DirectionOperands<T, CPLX> o{z, p};
+        if (!spmv_row_gp<T, CPLX>(A, DirectionGather<T, CPLX>{z, p, beta}, vb, row, a[0], a[1], o)) continue;
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            const T pk = o.zv[w] + beta * o.pv[w];
+            pn[W * row + w] = pk;
+            q[W * row + w] = a[w];
+            contrib += double(pk) * double(a[w]);
         }
     }
     double v[1] = {contrib};
-    partials_write<1>(v, partials);
+    partials_write<1>(v, partials + kRowPq * kMaxParts);
 }
 
-// x += alpha p ; r -= alpha q ; z = dinv r ; rz, rr ; beta
-template <typename T, bool CPLX>
-__global__ void __launch_bounds__(256) cg_update(int n, T* __restrict__ x, T* __restrict__ r, T* __restrict__ z,
-                                               const T* __restrict__ p, const T* __restrict__ q,
-                                               const T* __restrict__ dinv, const CgState* st, double* partials) {
+// npq: partials of p^H q to fold (0: the state holds alpha)
+template <typename T, bool CPLX, bool JAC>
+__global__ void __launch_bounds__(256) cg_step2(int n, T* __restrict__ x, T* __restrict__ r, T* __restrict__ z,
+                                              const T* __restrict__ p, const T* __restrict__ q,
+                                              const T* __restrict__ dinv, CgState* st, double* partials, int npq) {
     if (st->done) return;
-    const T alpha = T(st->alpha);
+    constexpr int W = CPLX ? 2 : 1;
+    const double rz_new = st->rz_new;
+    T alpha;
+    if (npq) {
+        double tot[1];
+        partials_sum<1>(partials + kRowPq * kMaxParts, npq, tot);
+        const double pq = tot[0];
+        if (!(pq > 0.0)) {
+            if (blockIdx.x == 0 && threadIdx.x == 0) {
+                st->status = (pq == pq) ? MK_ERR_NOT_SPD : MK_ERR_NAN;
+                st->done = 1;
+            }
+            return;
+        }
+        alpha = T(rz_new / pq);
+    } else {
+        alpha = T(st->alpha);
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->rz = rz_new;
     double rz = 0.0, rr = 0.0;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const T d = dinv ? dinv[i] : T(1);
-        if constexpr (CPLX) {
+        const T d = JAC && dinv ? dinv[i] : T(1);
 #pragma unroll
-            for (int c = 0; c < 2; c++) {
-                const int k = 2 * i + c;
-                x[k] += alpha * p[k];
-                const T rk = r[k] - alpha * q[k];
-                r[k] = rk;
-                const T zk = d * rk;
-                z[k] = zk;
-                rz += double(rk) * zk;
-                rr += double(rk) * rk;
-            }
-        } else {
-            x[i] += alpha * p[i];
-            const T rk = r[i] - alpha * q[i];
-            r[i] = rk;
-            const T zk = d * rk;
-            z[i] = zk;
-            rz += double(rk) * zk;
+        for (int w = 0; w < W; w++) {
+            const int e = W * i + w;
+            x[e] += alpha * p[e];
+            const T rk = r[e] - alpha * q[e];
+            r[e] = rk;
             rr += double(rk) * rk;
+            if constexpr (JAC) {
+                const T zk = d * rk;
+                z[e] = zk;
+                rz += double(rk) * zk;
+            }
         }
     }
-    double v[2] = {rz, rr};
-    partials_write<2>(v, partials);
+    if constexpr (JAC) {
+        double v[2] = {rz, rr};
+        partials_write<2>(v, partials);
+    } else {
+        double v[1] = {rr};
+        partials_write<1>(v, partials + kRowRr * kMaxParts);
+    }
 }
 
-// preconditioned variant (z from an external preconditioner): init, update, beta
+// p^H q -> alpha (launches of more than kFoldParts blocks)
+__global__ void __launch_bounds__(1024) cg_alpha_fin(CgState* st, const double* __restrict__ partials, int nparts) {
+    if (st->done) return;
+    double tot[1];
+    partials_sum<1>(partials + kRowPq * kMaxParts, nparts, tot);
+    if (threadIdx.x == 0) {
+        if (!(tot[0] > 0.0)) { st->status = (tot[0] == tot[0]) ? MK_ERR_NOT_SPD : MK_ERR_NAN; st->done = 1; }
+        else st->alpha = st->rz_new / tot[0];
+    }
+}
+// rr of the external preconditioner's iteration -> convergence, before the preconditioner runs
+__global__ void __launch_bounds__(1024) cg_rr_fin(CgState* st, const double* __restrict__ partials, int nparts) {
+    if (st->done) return;
+    double tot[1];
+    partials_sum<1>(partials + kRowRr * kMaxParts, nparts, tot);
+    if (threadIdx.x == 0) {
+        st->rr = tot[0];
+        st->it += 1;
+        if (!(tot[0] == tot[0])) { st->status = MK_ERR_NAN; st->done = 1; }
+        else if (tot[0] <= st->tol2 * st->bb) st->done = 1;
+    }
+}
+// the last iteration's rz (Jacobi: and rr) -> rz, beta (and convergence) in the state, for the host
+// and for the next batch's first iteration
+template <bool JAC>
+__global__ void __launch_bounds__(1024) cg_beta_fin(CgState* st, const double* __restrict__ partials, int nparts) {
+    if (st->done) return;
+    double tot[JAC ? 2 : 1];
+    partials_sum<JAC ? 2 : 1>(partials, nparts, tot);
+    if (threadIdx.x == 0) {
+        const double rz = tot[0];
+        if constexpr (JAC) {
+            const double rr = tot[1];
+            st->rr = rr;
+            st->it += 1;
+            if (!(rr == rr) || !(rz == rz)) { st->status = MK_ERR_NAN; st->done = 1; }
+            else if (rr <= st->tol2 * st->bb) st->done = 1;
+        } else if (!(rz > 0.0)) {
+            st->status = (rz == rz) ? MK_ERR_NOT_SPD : MK_ERR_NAN;
+            st->done = 1;
+            return;
+        }
+        st->beta = rz / st->rz;
+        st->rz = rz;
+    }
+}
+
+// z from an external preconditioner: init, rz
 template <typename T, bool CPLX>
 __global__ void __launch_bounds__(256) cg_init_z(int n, const T* __restrict__ r, const T* __restrict__ b,
                                                const T* __restrict__ z, T* __restrict__ p, double* partials) {
@@ -281,34 +361,13 @@ __global__ void __launch_bounds__(1024) cg_init_fin(CgState* st, const double* _
         st->rr = st->rr0 = tot[1];
         st->bb = tot[2];
         st->tol2 = tol2;
+        st->beta = 0.0;
         st->it = 0;
         st->status = MK_OK;
         st->done = (tot[1] <= tol2 * tot[2]) ? 1 : 0;
         if (!(tot[0] == tot[0]) || !(tot[1] == tot[1])) { st->status = MK_ERR_NAN; st->done = 1; }
         if (check_z && !st->done && !(tot[0] > 0.0)) { st->status = MK_ERR_NOT_SPD; st->done = 1; }
     }
-}
-
-template <typename T, bool CPLX>
-__global__ void __launch_bounds__(256) cg_update_noz(int n, T* __restrict__ x, T* __restrict__ r,
-                                                   const T* __restrict__ p, const T* __restrict__ q,
-                                                   const CgState* st, double* partials) {
-    if (st->done) return;
-    const T alpha = T(st->alpha);
-    double rr = 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const int w = CPLX ? 2 : 1;
-#pragma unroll
-        for (int c = 0; c < w; c++) {
-            const int k = w * i + c;
-            x[k] += alpha * p[k];
-            const T rk = r[k] - alpha * q[k];
-            r[k] = rk;
-            rr += double(rk) * rk;
-        }
-    }
-    double v[1] = {rr};
-    partials_write<1>(v, partials);
 }
 
 template <typename T, bool CPLX>
@@ -324,42 +383,59 @@ __global__ void __launch_bounds__(256) cg_beta(int n, const T* __restrict__ r, c
     partials_write<1>(v, partials);
 }
 
-template <typename T>
-__global__ void __launch_bounds__(256) cg_pupdate(size_t len, T* __restrict__ p, const T* __restrict__ z,
-                                                const CgState* st) {
-    if (st->done) return;
-    const T beta = T(st->beta);
-    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < len) p[i] = z[i] + beta * p[i];
-}
-
 // ---------------------------------------------------------------------------------------
 // FP64 PCG with an FP32 multigrid preconditioner (vectors as real arrays of len entries;
 // complex interleaved gives Re(r^H z) as the plain sum).  The preconditioner runs in FP32,
 // so it is not exactly symmetric: beta is the flexible (Polak-Ribiere) form
 // beta = r_{k+1}.(z_{k+1} - z_k) / r_k.z_k, with z_k kept in FP64 (zold).
 
-// x += alpha p ; r -= alpha q ; r32 = float(r) ; rr
+// The scalars go through the partials as in cg_step1 / cg_step2 (a = r.z and m = r.zold in rows 0 and
+// 1, p^H q in row 2, rr in row 3): folded by the kernel that needs them up to kFoldParts blocks.
+static constexpr int kRowUpd = 3;
+
+// x += alpha p ; r -= alpha q ; r32 = float(r) ; rr.  npq: partials of p^H q to fold (0: the state
+// holds alpha).
 __global__ void __launch_bounds__(256) cgm_update(size_t len, double* __restrict__ x, double* __restrict__ r,
                                                 float* __restrict__ r32, const double* __restrict__ p,
-                                                const double* __restrict__ q, CgState* st, double* partials) {
+                                                const double* __restrict__ q, CgState* st, double* partials, int npq) {
     if (st->done) return;
-    const double alpha = st->alpha;
+    const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+    // the first element's loads are in flight while alpha is folded
+    size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    const size_t stride = size_t(gridDim.x) * blockDim.x;
+    double xi = 0.0, ri = 0.0, pi = 0.0, qi = 0.0;
+    if (i < len) { xi = x[i]; ri = r[i]; pi = p[i]; qi = q[i]; }
+    double alpha;
+    if (npq) {
+        const double rz_new = st->rz_new;
+        double tot[1];
+        partials_sum<1>(partials + kRowPq * kMaxParts, npq, tot);
+        if (!(tot[0] > 0.0)) {
+            if (writer) { st->status = (tot[0] == tot[0]) ? MK_ERR_NOT_SPD : MK_ERR_NAN; st->done = 1; }
+            return;
+        }
+        alpha = rz_new / tot[0];
+        if (writer) { st->rz = rz_new; st->first = 0; }
+    } else {
+        alpha = st->alpha;
+    }
     double rr = 0.0;
-    for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < len; i += size_t(gridDim.x) * blockDim.x) {
-        x[i] += alpha * p[i];
-        const double rk = r[i] - alpha * q[i];
+    while (i < len) {
+        x[i] = xi + alpha * pi;
+        const double rk = ri - alpha * qi;
         r[i] = rk;
         r32[i] = float(rk);
         rr += rk * rk;
+        i += stride;
+        if (i < len) { xi = x[i]; ri = r[i]; pi = p[i]; qi = q[i]; }
     }
     double v[1] = {rr};
-    partials_write<1>(v, partials);
+    partials_write<1>(v, partials + kRowUpd * kMaxParts);
 }
 __global__ void __launch_bounds__(1024) cgm_update_fin(CgState* st, const double* __restrict__ partials, int nparts) {
     if (st->done) return;
     double tot[1];
-    partials_sum<1>(partials, nparts, tot);
+    partials_sum<1>(partials + kRowUpd * kMaxParts, nparts, tot);
     if (threadIdx.x == 0) {
         st->rr = tot[0];
         st->it += 1;
@@ -372,7 +448,7 @@ __global__ void __launch_bounds__(1024) cgm_update_fin(CgState* st, const double
 // iteration); rz = a
 __global__ void __launch_bounds__(256) cgm_beta2(size_t len, const double* __restrict__ r,
                                                const float* __restrict__ z32, const double* __restrict__ zold,
-                                               CgState* st, double* partials) {
+                                               const CgState* st, double* partials) {
     if (st->done) return;
     double a = 0.0, m = 0.0;
     for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < len; i += size_t(gridDim.x) * blockDim.x) {
@@ -425,16 +501,32 @@ struct CgmOperands {
 };
 template <bool CPLX>
 __global__ void __launch_bounds__(256) cgm_spmv(SellDev<double> A, const float* __restrict__ z32, double* p, double* q,
-                                              double* __restrict__ zold, CgState* st, double* partials) {
+                                              double* __restrict__ zold, CgState* st, double* partials, int nin) {
     if (st->done) return;
     constexpr int W = CPLX ? 2 : 1;
-    const double beta = st->beta;
+    double beta = st->beta;
+    bool folded = nin == 0;
     double contrib = 0.0;
     for (int vb = blockIdx.x; vb < A.nvb; vb += gridDim.x) {
         int row = 0;
         double a[2];
         CgmOperands<CPLX> o{z32, p, q};
-        if (!spmv_row_gp<double, CPLX>(A, Fp32Gather<CPLX>{z32}, vb, row, a[0], a[1], o)) continue;
+        const bool own = spmv_row_gp<double, CPLX>(A, Fp32Gather<CPLX>{z32}, vb, row, a[0], a[1], o);
+        if (!folded) {  // a and m, while the first row's gathers are in flight; rz_new is cgm_update's
+            const double rz = st->rz;
+            const int first = st->first;
+            double tot[2];
+            partials_sum<2>(partials, nin, tot);
+            const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+            if (!(tot[0] > 0.0)) {
+                if (writer) { st->status = (tot[0] == tot[0]) ? MK_ERR_NOT_SPD : MK_ERR_NAN; st->done = 1; }
+                return;
+            }
+            beta = first ? 0.0 : (tot[0] - tot[1]) / rz;
+            if (writer) st->rz_new = tot[0];
+            folded = true;
+        }
+        if (!own) continue;
 #pragma unroll
         for (int k = 0; k < W; k++) {
             const double pk = o.zv[k] + beta * o.pv[k], qk = a[k] + beta * o.qv[k];
@@ -445,12 +537,12 @@ __global__ void __launch_bounds__(256) cgm_spmv(SellDev<double> A, const float* 
         }
     }
     double v[1] = {contrib};
-    partials_write<1>(v, partials);
+    partials_write<1>(v, partials + kRowPq * kMaxParts);
 }
 __global__ void __launch_bounds__(1024) cgm_spmv_fin(CgState* st, const double* __restrict__ partials, int nparts) {
     if (st->done) return;
     double tot[1];
-    partials_sum<1>(partials, nparts, tot);
+    partials_sum<1>(partials + kRowPq * kMaxParts, nparts, tot);
     if (threadIdx.x == 0) {
         st->pq = tot[0];
         if (!(tot[0] > 0.0)) {
@@ -834,9 +926,12 @@ void spmv_launch(mk_ctx* c, const mk_op* A, const T* val, const T* x, T* y, cons
     static const char* kname[] = {"spmv", "spmv_dot", "spmv_resid", "spmv_resid_nored", "spmv_accum"};
     SpmvTimer tm(c, bytes, A, kname[int(mode)], sizeof(T) == 4);
     const unsigned gr = std::max(1u, std::min(g, fin_grid()));  // reducing modes: capped grid
+    // the norm alone of a residual is taken between two batches of iterations, whose preconditioned
+    // residual's dots wait in rows 0 and 1
+    double* part = c->partials.p + (mode == SPMV_RESID && !y ? kRowPq * kMaxParts : 0);
 #define MK_SPMV(CPLX, MODE)                                                                                \
     MK_TLAUNCH(tm, 0, (sell_spmv<T, CPLX, MODE>), dim3((MODE == 1 || MODE == 2) ? gr : g), dim3(A->block), 0, \
-               c->stream, D, x, y, b, c->partials.p, skip)
+               c->stream, D, x, y, b, part, skip)
 #define MK_SPMV_ALL(CPLX)                            \
     switch (mode) {                                  \
         case SPMV_PLAIN: MK_SPMV(CPLX, 0); break;    \
@@ -848,7 +943,7 @@ void spmv_launch(mk_ctx* c, const mk_op* A, const T* val, const T* x, T* y, cons
     if (A->cplx) { MK_SPMV_ALL(true) } else { MK_SPMV_ALL(false) }
 #undef MK_SPMV_ALL
 #undef MK_SPMV
-    if (mode == SPMV_DOT || mode == SPMV_RESID) finish<1, FinOut>(c, gr, out, skip);
+    if (mode == SPMV_DOT || mode == SPMV_RESID) finish(c, gr, out, skip, part);
     MK_HIP(hipGetLastError());
 }
 // One Chebyshev step fused with the residual it needs, row-local:
@@ -1002,35 +1097,68 @@ struct TwoSourceGather {
         else { xr = s[k]; xi = T(0); }
     }
 };
+// DOTS: also a = r.y and m = r.yold of FP64 vectors r, yold, the dots a flexible PCG needs of its
+// preconditioned residual y: partials per block in rows 0 and 1.
 template <typename T, bool CPLX>
+struct DotOperands {
+    static constexpr int W = CPLX ? 2 : 1;
+    const double* __restrict__ r;
+    const double* __restrict__ yold;
+    double rv[W], ov[W];
+    __device__ __forceinline__ void operator()(int row) {
+#pragma unroll
+        for (int q = 0; q < W; q++) { rv[q] = r[W * row + q]; ov[q] = yold[W * row + q]; }
+    }
+};
+template <typename T, bool CPLX, bool DOTS>
 __global__ void __launch_bounds__(256) sell_spmv2(SellDev<T> A, int m1, const T* __restrict__ u, const T* __restrict__ v,
-                                                T* __restrict__ y, const int* skip) {
+                                                T* __restrict__ y, const int* skip, const double* __restrict__ r,
+                                                const double* __restrict__ yold, double* __restrict__ partials) {
     if (skip && *skip) return;
     int row = 0;
-    T ar, ai;
-    if (!spmv_row_g<T, CPLX>(A, TwoSourceGather<T, CPLX>{u, v, m1}, blockIdx.x, row, ar, ai)) return;
-    if constexpr (CPLX) { y[2 * row] = ar; y[2 * row + 1] = ai; }
-    else y[row] = ar;
+    T a[2];
+    if constexpr (!DOTS) {
+        if (!spmv_row_g<T, CPLX>(A, TwoSourceGather<T, CPLX>{u, v, m1}, blockIdx.x, row, a[0], a[1])) return;
+        if constexpr (CPLX) { y[2 * row] = a[0]; y[2 * row + 1] = a[1]; }
+        else y[row] = a[0];
+    } else {
+        constexpr int W = CPLX ? 2 : 1;
+        DotOperands<T, CPLX> o{r, yold};
+        double d[2] = {0.0, 0.0};
+        if (spmv_row_gp<T, CPLX>(A, TwoSourceGather<T, CPLX>{u, v, m1}, blockIdx.x, row, a[0], a[1], o)) {
+#pragma unroll
+            for (int q = 0; q < W; q++) {
+                y[W * row + q] = a[q];
+                d[0] += o.rv[q] * double(a[q]);
+                d[1] += o.rv[q] * o.ov[q];
+            }
+        }
+        partials_write<2>(d, partials);
+    }
 }
 
+// r (with yold and partials): the dots too; returns the number of partials
 template <typename T>
-void spmv2_launch(mk_ctx* c, const mk_op* A, int m1, const T* u, const T* v, T* y, const int* skip, const char* name) {
+unsigned spmv2_launch(mk_ctx* c, const mk_op* A, int m1, const T* u, const T* v, T* y, const int* skip, const char* name,
+                      const double* r, const double* yold, double* partials) {
     unsigned g = 0;
     const T* val;
     if constexpr (std::is_same<T, double>::value) val = A->val64.p;
     else val = A->val32.p;
     const SellDev<T> D = sell_dev<T>(A, val, A->block, &g);
+    MK_CHECK(!r || g <= kMaxParts, MK_ERR_ARG, "operator too large for the reduction buffer");
     SpmvTimer tm(c, sizeof(T) == 8 ? A->bytes64 : A->bytes32, A, name, sizeof(T) == 4);
-    if (A->cplx)
-        MK_TLAUNCH(tm, 0, (sell_spmv2<T, true>), dim3(g), dim3(A->block), 0, c->stream, D, m1, u, v, y, skip);
-    else
-        MK_TLAUNCH(tm, 0, (sell_spmv2<T, false>), dim3(g), dim3(A->block), 0, c->stream, D, m1, u, v, y, skip);
+#define MK_SPMV2(CP, DOTS)                                                                                                 MK_TLAUNCH(tm, 0, (sell_spmv2<T, CP, DOTS>), dim3(g), dim3(A->block), 0, c->stream, D, m1, u, v, y, skip, r, yold, partials)
+    if (A->cplx) { if (r) MK_SPMV2(true, true); else MK_SPMV2(true, false); }
+    else { if (r) MK_SPMV2(false, true); else MK_SPMV2(false, false); }
+#undef MK_SPMV2
     MK_HIP(hipGetLastError());
+    return g;
 }
-template void spmv2_launch<double>(mk_ctx*, const mk_op*, int, const double*, const double*, double*, const int*,
-                                   const char*);
-template void spmv2_launch<float>(mk_ctx*, const mk_op*, int, const float*, const float*, float*, const int*,
-                                  const char*);
+template unsigned spmv2_launch<double>(mk_ctx*, const mk_op*, int, const double*, const double*, double*, const int*,
+                                       const char*, const double*, const double*, double*);
+template unsigned spmv2_launch<float>(mk_ctx*, const mk_op*, int, const float*, const float*, float*, const int*,
+                                      const char*, const double*, const double*, double*);
 
 template <typename T>
 __global__ void k_copy(size_t len, const T* __restrict__ x, T* __restrict__ y, const int* skip) {
@@ -1067,7 +1195,7 @@ void axpby64(mk_ctx* c, size_t len, double a, const double* x, double b, double*
 void dot64(mk_ctx* c, size_t len, const double* x, const double* y, double* out_dev) {
     const unsigned g = fgrid(len);
     hipLaunchKernelGGL(k_dot, dim3(g), dim3(256), 0, c->stream, len, x, y, c->partials.p);
-    finish<1, FinOut>(c, g, out_dev);
+    finish(c, g, out_dev);
     MK_HIP(hipGetLastError());
 }
 void mass_mul(mk_ctx* c, int n, const double* mass, const double* u, double* b) {
@@ -1077,7 +1205,7 @@ void mass_mul(mk_ctx* c, int n, const double* mass, const double* u, double* b) 
 void mass_dot(mk_ctx* c, int n, const double* mass, const double* x, double* out_dev) {
     const unsigned g = fgrid(size_t(n));
     hipLaunchKernelGGL(k_mass_dot, dim3(g), dim3(256), 0, c->stream, n, mass, x, c->partials.p);
-    finish<1, FinOut>(c, g, out_dev);
+    finish(c, g, out_dev);
     MK_HIP(hipGetLastError());
 }
 void cvt64to32_scaled(mk_ctx* c, size_t len, const double* x, const double* s_dev, float* y) {
@@ -1093,38 +1221,18 @@ void add32to64_scaled(mk_ctx* c, size_t len, const float* d, const double* s_dev
 static inline void mg_apply(mk_ctx* c, Mg* g, const double* b, double* x, const int* skip) { mg_apply64(c, g, b, x, skip); }
 static inline void mg_apply(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip) { mg_apply32(c, g, b, x, skip); }
 
-// q = A p fused with p^H q and alpha (CG state on the device)
-template <typename T>
-static void launch_cg_spmv(mk_ctx* c, const mk_op* A, const T* val, const T* p, T* q, double bytes) {
-    unsigned g = 0;
-    const SellDev<T> D = sell_dev<T>(A, val, A->block, &g);
-    const unsigned gr = std::max(1u, std::min(g, fin_grid()));
-    {
-        SpmvTimer tm(c, bytes, A, "cg_spmv", sizeof(T) == 4);
-        if (A->cplx)
-            MK_TLAUNCH(tm, 0, (cg_spmv<T, true>), dim3(gr), dim3(A->block), 0, c->stream, D, p, q,
-                       (const CgState*)c->state.p, c->partials.p);
-        else
-            MK_TLAUNCH(tm, 0, (cg_spmv<T, false>), dim3(gr), dim3(A->block), 0, c->stream, D, p, q,
-                       (const CgState*)c->state.p, c->partials.p);
-    }
-    finish<1, FinCgAlpha>(c, gr);
-}
-
-// Runs `batch` calls of body() on the context stream: eagerly, or -- when graphs are on, timing
-// is off and batch is the operator's usual check interval -- by replaying a hipGraph captured
-// from the same calls the first time this key is seen.  body() must only launch kernels on
+// Runs body(batch) on the context stream: eagerly, or -- when graphs are on and timing is off -- by
+// replaying a hipGraph captured from the same call the first time this key is seen.  It must only launch kernels on
 // c->stream whose arguments are fixed by the key: the context (its id and its partials, state
 // and scalar buffers), the hierarchy (its id: its level buffers live as long as it does) and
 // the solve's vectors and value arrays (`buffers`).  The graphs are cached on the operator, so
 // an operator is only ever run on the context it was created on.
 template <typename F>
-static void run_batch(mk_ctx* c, const mk_op* A_, const Mg* mg, std::vector<uintptr_t> buffers, int batch,
-                      bool graphable, F&& body) {
+static void run_batch(mk_ctx* c, const mk_op* A_, const Mg* mg, std::vector<uintptr_t> buffers, int batch, F&& body) {
     mk_op* A = const_cast<mk_op*>(A_);
     MK_CHECK(A->ctx == c, MK_ERR_ARG, "operator used with a context other than the one it was created on");
-    if (!c->use_graphs || c->time_spmv || !graphable) {
-        for (int b = 0; b < batch; b++) body();
+    if (!c->use_graphs || c->time_spmv) {
+        body(batch);
         c->eager_batches++;
         return;
     }
@@ -1140,7 +1248,7 @@ static void run_batch(mk_ctx* c, const mk_op* A_, const Mg* mg, std::vector<uint
     mk_op::Graph* G = nullptr;
     for (auto& g : A->graphs) if (g.key == key) { G = &g; break; }
     if (!G) {
-        if (A->graphs.size() >= 8) {  // bounded cache: drop the oldest
+        if (A->graphs.size() >= 16) {  // bounded cache: drop the oldest
             if (A->graphs.front().exec) MK_HIP(hipGraphExecDestroy(A->graphs.front().exec));
             A->graphs.erase(A->graphs.begin());
         }
@@ -1150,7 +1258,7 @@ static void run_batch(mk_ctx* c, const mk_op* A_, const Mg* mg, std::vector<uint
         MK_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeRelaxed));
         hipGraph_t graph = nullptr;
         try {
-            for (int b = 0; b < batch; b++) body();
+            body(batch);
         } catch (...) {
             (void)hipStreamEndCapture(c->stream, &graph);
             if (graph) (void)hipGraphDestroy(graph);
@@ -1187,33 +1295,6 @@ static void run_batches(int m, int interval, F&& batch) {
         if (p <= m) { batch(p); m -= p; }
 }
 
-// one PCG iteration with an external (multigrid) preconditioner
-template <typename T>
-static void cg_iter_mg(mk_ctx* c, const mk_op* A, const T* val, Mg* mg, T* x, T* r, T* z, T* p, T* q, double bytes) {
-    const int n = A->n;
-    const size_t len = size_t(n) * (A->cplx ? 2 : 1);
-    const unsigned g = blocks_for(n);
-    CgState* st = c->state.p;
-    const unsigned gn = fgrid(size_t(n));
-    launch_cg_spmv<T>(c, A, val, p, q, bytes);
-    if (A->cplx)
-        hipLaunchKernelGGL((cg_update_noz<T, true>), dim3(gn), dim3(256), 0, c->stream, n, x, r, p, q,
-                           (const CgState*)st, c->partials.p);
-    else
-        hipLaunchKernelGGL((cg_update_noz<T, false>), dim3(gn), dim3(256), 0, c->stream, n, x, r, p, q,
-                           (const CgState*)st, c->partials.p);
-    finish<1, FinCgRr>(c, gn);
-    mg_apply(c, mg, r, z, &st->done);
-    if (A->cplx)
-        hipLaunchKernelGGL((cg_beta<T, true>), dim3(gn), dim3(256), 0, c->stream, n, r, z, (const CgState*)st,
-                           c->partials.p);
-    else
-        hipLaunchKernelGGL((cg_beta<T, false>), dim3(gn), dim3(256), 0, c->stream, n, r, z, (const CgState*)st,
-                           c->partials.p);
-    finish<1, FinCgBeta>(c, gn);
-    hipLaunchKernelGGL(cg_pupdate<T>, dim3(blocks_for(len)), dim3(256), 0, c->stream, len, p, z, (const CgState*)st);
-}
-
 // Runs a started solve (its state on the device): launch(m) queues m iterations; resid() queues
 // the true residual of x into the state behind a batch that is expected to be the last, so that a
 // solve that ends where its operator's last one did costs one round trip to the host.
@@ -1242,8 +1323,8 @@ static CgResult drive(mk_ctx* c, int hint, int maxiter, int check_every, L&& lau
 
 // PCG on r (the initial residual); b for its norm.  resid as in drive().
 template <typename T, typename R>
-static CgResult cg_run(mk_ctx* c, const mk_op* A, const T* val, const T* dinv, const T* b, T* x, T* r, T* z, T* p, T* q,
-                       double rel_tol, int hint, int maxiter, int check_every, double bytes, Mg* mg, R&& resid) {
+static CgResult cg_run(mk_ctx* c, const mk_op* A, const T* val, const T* dinv, const T* b, T* x, T* r, T* z, T* p, T* p2,
+                       T* q, double rel_tol, int hint, int maxiter, int check_every, double bytes, Mg* mg, R&& resid) {
     const int n = A->n;
     const size_t len = size_t(n) * (A->cplx ? 2 : 1);
     const unsigned g = blocks_for(n);
@@ -1267,35 +1348,64 @@ static CgResult cg_run(mk_ctx* c, const mk_op* A, const T* val, const T* dinv, c
     hipLaunchKernelGGL(cg_init_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)c->partials.p, int(gn),
                        rel_tol * rel_tol, mg ? 1 : 0);
     MK_HIP(hipGetLastError());
-    if (mg)
-        return drive(c, hint, maxiter, check_every, [&](int batch) {
-            run_batches(batch, check_every, [&](int m) {
-                run_batch(c, A, mg, {uintptr_t(sizeof(T)), uintptr_t(val), uintptr_t(x), uintptr_t(r),
-                                     uintptr_t(z), uintptr_t(p), uintptr_t(q)},
-                          m, true, [&] { cg_iter_mg<T>(c, A, val, mg, x, r, z, p, q, bytes); });
-            });
-        }, resid);
-    return drive(c, hint, maxiter, check_every, [&](int batch) {
-        for (int k = 0; k < batch; k++) {
-            launch_cg_spmv<T>(c, A, val, p, q, bytes);
-            if (A->cplx)
-                hipLaunchKernelGGL((cg_update<T, true>), dim3(gn), dim3(256), 0, c->stream, n, x, r, z, p, q, dinv,
-                                   (const CgState*)st, c->partials.p);
+    unsigned gs = 0;
+    const SellDev<T> D = sell_dev<T>(A, val, A->block, &gs);
+    const unsigned gr = std::max(1u, std::min(gs, fin_grid()));
+    const bool fold = std::max(gr, gn) <= kFoldParts;
+    double* part = c->partials.p;
+    // `batch` iterations from direction buffer pa (the other one: pb), which alternate
+    auto iterations = [&](int batch, T* pa, T* pb) {
+        for (int k = 0; k < batch; k++, std::swap(pa, pb)) {
+            const int nin = fold && k ? int(gn) : 0;
+            {
+                SpmvTimer tm(c, bytes, A, "cg_spmv", sizeof(T) == 4);
+#define MK_STEP1(CP, JAC)                                                                                                    MK_TLAUNCH(tm, 0, (cg_step1<T, CP, JAC>), dim3(gr), dim3(A->block), 0, c->stream, D, (const T*)z, (const T*)pa, pb, q, st,                part, nin)
+                if (A->cplx) { if (mg) MK_STEP1(true, false); else MK_STEP1(true, true); }
+                else { if (mg) MK_STEP1(false, false); else MK_STEP1(false, true); }
+#undef MK_STEP1
+            }
+            if (!fold) hipLaunchKernelGGL(cg_alpha_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gr));
+            const int npq = fold ? int(gr) : 0;
+#define MK_STEP2(CP, JAC)                                                                                                hipLaunchKernelGGL((cg_step2<T, CP, JAC>), dim3(gn), dim3(256), 0, c->stream, n, x, r, z, (const T*)pb, (const T*)q,                        dinv, st, part, npq)
+            if (A->cplx) { if (mg) MK_STEP2(true, false); else MK_STEP2(true, true); }
+            else { if (mg) MK_STEP2(false, false); else MK_STEP2(false, true); }
+#undef MK_STEP2
+            if (mg) {
+                hipLaunchKernelGGL(cg_rr_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gn));
+                mg_apply(c, mg, r, z, &st->done);
+                if (A->cplx)
+                    hipLaunchKernelGGL((cg_beta<T, true>), dim3(gn), dim3(256), 0, c->stream, n, r, z, (const CgState*)st,
+                                       part);
+                else
+                    hipLaunchKernelGGL((cg_beta<T, false>), dim3(gn), dim3(256), 0, c->stream, n, r, z,
+                                       (const CgState*)st, part);
+            }
+            if (fold && k + 1 < batch) continue;
+            if (mg)
+                hipLaunchKernelGGL((cg_beta_fin<false>), dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gn));
             else
-                hipLaunchKernelGGL((cg_update<T, false>), dim3(gn), dim3(256), 0, c->stream, n, x, r, z, p, q, dinv,
-                                   (const CgState*)st, c->partials.p);
-            finish<2, FinCgUpdate>(c, gn);
-            hipLaunchKernelGGL(cg_pupdate<T>, dim3(blocks_for(len)), dim3(256), 0, c->stream, len, p, z,
-                               (const CgState*)st);
+                hipLaunchKernelGGL((cg_beta_fin<true>), dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gn));
         }
+    };
+    return drive(c, hint, maxiter, check_every, [&](int batch) {
+        if (!mg) {
+            iterations(batch, p, p2);
+            if (batch & 1) std::swap(p, p2);
+            return;
+        }
+        run_batches(batch, check_every, [&](int m) {
+            run_batch(c, A, mg, {uintptr_t(sizeof(T)), uintptr_t(val), uintptr_t(x), uintptr_t(r), uintptr_t(z), uintptr_t(p),
+                                 uintptr_t(p2), uintptr_t(q)},
+                      m, [&](int k) { iterations(k, p, p2); });
+            if (m & 1) std::swap(p, p2);
+        });
     }, resid);
 }
 
 // ||b - A x||^2 into the CG state, for drive()
 static auto true_residual(mk_ctx* c, const mk_op* A, const double* b, const double* x) {
     return [=] {
-        work(c).t.ensure(size_t(A->n) * (A->cplx ? 2 : 1));
-        spmv64(c, A, x, work(c).t.p, b, SPMV_RESID, &c->state.p->true_rr, nullptr);
+        spmv64(c, A, x, nullptr, b, SPMV_RESID, &c->state.p->true_rr, nullptr);
         return true;
     };
 }
@@ -1304,9 +1414,9 @@ CgResult cg64(mk_ctx* c, const mk_op* A, const double* b, double* x, double rel_
               int check_every, Mg* mg) {
     Work& w = work(c);
     const size_t len = size_t(A->n) * (A->cplx ? 2 : 1);
-    w.r.ensure(len); w.z.ensure(len); w.p.ensure(len); w.q.ensure(len);
+    w.r.ensure(len); w.z.ensure(len); w.p.ensure(len); w.p2.ensure(len); w.q.ensure(len);
     spmv64(c, A, x, w.r.p, b, SPMV_RESID_NORED, nullptr, nullptr);
-    return cg_run<double>(c, A, A->val64.p, jacobi ? A->dinv64.p : nullptr, b, x, w.r.p, w.z.p, w.p.p, w.q.p, rel_tol,
+    return cg_run<double>(c, A, A->val64.p, jacobi ? A->dinv64.p : nullptr, b, x, w.r.p, w.z.p, w.p.p, w.p2.p, w.q.p, rel_tol,
                           hint, maxiter, check_every, A->bytes64, mg, true_residual(c, A, b, x));
 }
 
@@ -1315,10 +1425,10 @@ CgResult cg32(mk_ctx* c, const mk_op* A, const float* b, float* x, double rel_to
               int check_every, Mg* mg) {
     Work& w = work(c);
     const size_t len = size_t(A->n) * (A->cplx ? 2 : 1);
-    w.r32.ensure(len); w.z32.ensure(len); w.p32.ensure(len); w.q32.ensure(len);
+    w.r32.ensure(len); w.z32.ensure(len); w.p32.ensure(len); w.p2_32.ensure(len); w.q32.ensure(len);
     MK_HIP(hipMemsetAsync(x, 0, len * sizeof(float), c->stream));
     MK_HIP(hipMemcpyAsync(w.r32.p, b, len * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
-    return cg_run<float>(c, A, A->val32.p, jacobi ? A->dinv32.p : nullptr, b, x, w.r32.p, w.z32.p, w.p32.p, w.q32.p,
+    return cg_run<float>(c, A, A->val32.p, jacobi ? A->dinv32.p : nullptr, b, x, w.r32.p, w.z32.p, w.p32.p, w.p2_32.p, w.q32.p,
                          rel_tol, 0, maxiter, check_every, A->bytes32, mg, [] { return false; });
 }
 
@@ -1337,37 +1447,49 @@ CgResult cg64_mg32(mk_ctx* c, const mk_op* A, const double* b, double* x, double
                        w.z.p, c->partials.p);
     hipLaunchKernelGGL(cgm_init_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)c->partials.p, int(gl),
                        rel_tol * rel_tol);
-    mg_apply32(c, mg, w.r32.p, w.z32.p, &st->done);
+    double* part = c->partials.p;
+    // the V-cycle on r32 and the two dots beta needs, in its last kernel where that can; returns
+    // their partials
+    auto precondition = [&] {
+        const unsigned np = mg_apply32_dots(c, mg, w.r32.p, w.z32.p, &st->done, w.r.p, w.z.p, part);
+        if (np) return np;
+        hipLaunchKernelGGL(cgm_beta2, dim3(gl), dim3(256), 0, c->stream, len, (const double*)w.r.p,
+                           (const float*)w.z32.p, (const double*)w.z.p, (const CgState*)st, part);
+        return gl;
+    };
+    const unsigned gb = precondition();
     MK_HIP(hipGetLastError());
     unsigned gs = 0;
     const SellDev<double> D = sell_dev<double>(A, A->val64.p, A->block, &gs);
     const unsigned gsr = std::max(1u, std::min(gs, fin_grid()));
+    const bool fold_b = gb <= kFoldParts && gsr <= kFoldParts;
     // one iteration: beta, p/q update with A z (fused), x/r update, V-cycle on the new residual
     auto iteration = [&] {
-        hipLaunchKernelGGL(cgm_beta2, dim3(gl), dim3(256), 0, c->stream, len, (const double*)w.r.p,
-                           (const float*)w.z32.p, (const double*)w.z.p, st, c->partials.p);
-        hipLaunchKernelGGL(cgm_beta2_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)c->partials.p, int(gl));
+        if (!fold_b)
+            hipLaunchKernelGGL(cgm_beta2_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gb));
+        const int nin = fold_b ? int(gb) : 0;
         {
             SpmvTimer tm(c, A->bytes64 + double(len) * (4.0 + 8.0 * 5.0), A, "cg_spmv", false);
             if (A->cplx)
                 MK_TLAUNCH(tm, 0, (cgm_spmv<true>), dim3(gsr), dim3(A->block), 0, c->stream, D,
-                           (const float*)w.z32.p, w.p.p, w.q.p, w.z.p, st, c->partials.p);
+                           (const float*)w.z32.p, w.p.p, w.q.p, w.z.p, st, part, nin);
             else
                 MK_TLAUNCH(tm, 0, (cgm_spmv<false>), dim3(gsr), dim3(A->block), 0, c->stream, D,
-                           (const float*)w.z32.p, w.p.p, w.q.p, w.z.p, st, c->partials.p);
+                           (const float*)w.z32.p, w.p.p, w.q.p, w.z.p, st, part, nin);
         }
-        hipLaunchKernelGGL(cgm_spmv_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)c->partials.p, int(gsr));
+        if (!fold_b)
+            hipLaunchKernelGGL(cgm_spmv_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gsr));
         hipLaunchKernelGGL(cgm_update, dim3(gl), dim3(256), 0, c->stream, len, x, w.r.p, w.r32.p,
-                           (const double*)w.p.p, (const double*)w.q.p, st, c->partials.p);
-        hipLaunchKernelGGL(cgm_update_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)c->partials.p, int(gl));
-        mg_apply32(c, mg, w.r32.p, w.z32.p, &st->done);
+                           (const double*)w.p.p, (const double*)w.q.p, st, part, fold_b ? int(gsr) : 0);
+        hipLaunchKernelGGL(cgm_update_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gl));
+        precondition();
     };
     return drive(c, hint, maxiter, check_every, [&](int batch) {
         run_batches(batch, check_every, [&](int m) {
             run_batch(c, A, mg, {uintptr_t(4), uintptr_t(A->val64.p), uintptr_t(x), uintptr_t(w.r.p),
                                  uintptr_t(w.r32.p), uintptr_t(w.z32.p), uintptr_t(w.z.p), uintptr_t(w.p.p),
                                  uintptr_t(w.q.p)},
-                      m, true, iteration);
+                      m, [&](int k) { for (; k > 0; k--) iteration(); });
         });
     }, true_residual(c, A, b, x));
 }

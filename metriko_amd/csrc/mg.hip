@@ -1057,19 +1057,22 @@ void chebyshev(mk_ctx* c, const Mg* g, MgLevel& L, const T* b, T* x, bool zero_s
     if (cur != x) copy_launch<T>(c, size_t(n) * (g->cplx ? 2 : 1), cur, x, skip);
 }
 
+// r, xold, partials (the finest level only): the dots of mg_apply32_dots, formed by the last kernel of
+// a level that is one product or the dense inverse; returns their partials (0: not formed)
 template <typename T>
-void vcycle(mk_ctx* c, Mg* g, int l, const T* b, T* x, const int* skip) {
+unsigned vcycle(mk_ctx* c, Mg* g, int l, const T* b, T* x, const int* skip, const double* r_ = nullptr,
+                const double* xold = nullptr, double* partials = nullptr) {
     MgLevel& L = g->lv[size_t(l)];
     if (l + 1 == int(g->lv.size())) {
-        g->coarse.apply<T>(c, b, x, skip);
-        return;
+        const unsigned np = g->coarse.apply<T>(c, b, x, skip, r_, xold, partials);
+        return r_ ? np : 0;
     }
     MgLevel& Cn = g->lv[size_t(l) + 1];
     if (L.M) {
         spmv_launch<T>(c, L.W, Sel<T>::val(L.W), b, Sel<T>::b(Cn), nullptr, SPMV_PLAIN, nullptr, Sel<T>::bytes(L.W), skip);
         vcycle<T>(c, g, l + 1, Sel<T>::b(Cn), Sel<T>::x(Cn), skip);
-        spmv2_launch<T>(c, L.M, L.n, b, Sel<T>::x(Cn), x, skip, "cheb_level");
-        return;
+        const unsigned np = spmv2_launch<T>(c, L.M, L.n, b, Sel<T>::x(Cn), x, skip, "cheb_level", r_, xold, partials);
+        return r_ ? np : 0;
     }
     chebyshev<T>(c, g, L, b, x, true, skip);
     if (L.RR) {  // b_c = [R | -R A] [b; x] = R (b - A x) in one launch
@@ -1083,6 +1086,7 @@ void vcycle(mk_ctx* c, Mg* g, int l, const T* b, T* x, const int* skip) {
     vcycle<T>(c, g, l + 1, Sel<T>::b(Cn), Sel<T>::x(Cn), skip);
     spmv_launch<T>(c, L.P, Sel<T>::val(L.P), Sel<T>::x(Cn), x, nullptr, SPMV_ACCUM, nullptr, Sel<T>::bytes(L.P), skip);
     chebyshev<T>(c, g, L, b, x, false, skip);
+    return 0;
 }
 
 // ---- batched V-cycle (n x mw row-major blocks, FP32 or FP64) --------------------------------------
@@ -1336,6 +1340,10 @@ Mg* mg_build_complex(mk_ctx* c, int n, const int64_t* ptr, const int* col, const
 }
 void mg_apply64(mk_ctx* c, Mg* g, const double* b, double* x, const int* skip) { vcycle<double>(c, g, 0, b, x, skip); }
 void mg_apply32(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip) { vcycle<float>(c, g, 0, b, x, skip); }
+unsigned mg_apply32_dots(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip, const double* r, const double* xold,
+                         double* partials) {
+    return vcycle<float>(c, g, 0, b, x, skip, r, xold, partials);
+}
 template <typename T>
 void mg_apply_block(mk_ctx* c, Mg* g, int mw, const T* b, T* x, const int* skip) {
     MK_CHECK(!g->cplx, MK_ERR_UNSUPPORTED, "batched V-cycle: real hierarchies only");

@@ -89,6 +89,7 @@ struct CgState {
     int status;     // MK_OK / MK_ERR_NOT_SPD / MK_ERR_NAN
     int it;         // iterations taken
     int first;      // 1 until the first beta of the fused FP32-multigrid iteration
+    double rz_new;  // rz of the running iteration, moved to rz by its second kernel
     double rr0;     // ||r||^2 at the start
     double true_rr; // ||b - A x||^2 recomputed behind a batch that is expected to converge
 };
@@ -141,8 +142,8 @@ struct BatchPlanner {
 
 // per-context scratch vectors
 struct Work {
-    DevBuf<double> r, z, p, q, t;
-    DevBuf<float> r32, z32, p32, q32, x32, d32;
+    DevBuf<double> r, z, p, p2, q, t;
+    DevBuf<float> r32, z32, p32, p2_32, q32, x32, d32;
 };
 
 // batched (multi-right-hand-side) solves (block.hip): up to 64 columns, row-major blocks
@@ -166,8 +167,11 @@ struct DenseInverse {
     DenseInverse() = default;
     // from CSR arrays on the host (complex: values interleaved)
     DenseInverse(mk_ctx* c, bool cplx, int n, const int64_t* ptr, const int* col, const double* val);
+    // x = A^-1 b; with r, also per-block partials of r.x and r.xold (rows 0 and 1, kMaxParts apart).
+    // Returns the number of blocks.
     template <typename T>
-    void apply(mk_ctx* c, const T* b, T* x, const int* skip) const;  // x = A^-1 b
+    unsigned apply(mk_ctx* c, const T* b, T* x, const int* skip, const double* r = nullptr, const double* xold = nullptr,
+                   double* partials = nullptr) const;
     template <typename T>
     void apply_block(mk_ctx* c, int mw, const T* B, T* X, const int* skip) const;  // n x mw row-major
 };
@@ -187,6 +191,10 @@ Mg* mg_build_real(mk_ctx* c, int n, const int64_t* ptr, const int* col, const do
 Mg* mg_build_complex(mk_ctx* c, int n, const int64_t* ptr, const int* col, const double* val, const mk_solve_opts& o);
 void mg_apply64(mk_ctx* c, Mg* g, const double* b, double* x, const int* skip);
 void mg_apply32(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip);
+// mg_apply32 whose last kernel also leaves the per-block partials of r.x and r.xold (FP64 vectors, rows 0
+// and 1 of partials) where that kernel can: returns their number, 0 when the caller has to form them
+unsigned mg_apply32_dots(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip, const double* r, const double* xold,
+                         double* partials);
 // V-cycle on an n x mw row-major block (T = float: FP32 values and vectors; double: FP64)
 template <typename T>
 void mg_apply_block(mk_ctx* c, Mg* g, int mw, const T* b, T* x, const int* skip);
@@ -340,9 +348,11 @@ void cheb_launch(mk_ctx* c, const mk_op* A, const T* x_in, T* x_out, const T* b,
 // zero-start Chebyshev steps 1+2 fused: x_out = x1 + d, x1 = c0 D^-1 b, d = a x1 + s D^-1 (b - A x1)
 template <typename T>
 void cheb0_launch(mk_ctx* c, const mk_op* A, const T* b, T* x_out, T* d, T c0, T a, T s, const int* skip);
-// y = M [u; v], columns [0, m1) of M act on u, the rest on v (name: the timing key)
+// y = M [u; v], columns [0, m1) of M act on u, the rest on v (name: the timing key); with r, also the
+// per-block partials of r.y and r.yold in rows 0 and 1 of partials.  Returns the number of blocks.
 template <typename T>
-void spmv2_launch(mk_ctx* c, const mk_op* A, int m1, const T* u, const T* v, T* y, const int* skip, const char* name);
+unsigned spmv2_launch(mk_ctx* c, const mk_op* A, int m1, const T* u, const T* v, T* y, const int* skip, const char* name,
+                      const double* r = nullptr, const double* yold = nullptr, double* partials = nullptr);
 template <typename T>
 void copy_launch(mk_ctx* c, size_t len, const T* x, T* y, const int* skip);
 template <typename T>

@@ -3,7 +3,7 @@
 // Some callers cannot allocate device memory during a solve: code under HIP graph capture,
 // tight serving loops, harnesses that forbid it.  This entry point runs mk_spd_solve's FP64
 // PCG (Jacobi or no preconditioner) on caller-owned device vectors with every piece of
-// scratch -- the Krylov vectors r, z, p, q, the residual check's t, the per-block partial sums
+// scratch -- the Krylov vectors r, z, p, q and p's second buffer, the per-block partial sums
 // of the two-launch reductions, the CG state and the device scalars -- taken from one static
 // per-device array, `scratch`, instead of the context's buffers (which grow by hipMalloc).
 //
@@ -24,7 +24,7 @@ constexpr size_t kNoAllocLen = size_t(1) << 19;           // scalars per work ve
 constexpr size_t kPartials = kMaxParts * size_t(kMaxK);   // two-launch reduction partials
 constexpr size_t kStateDoubles = 32;                      // CgState (<= 256 bytes)
 constexpr size_t kScalDoubles = 64;                       // device scalars (as mk_ctx::scal)
-constexpr size_t kVectors = 5;                            // r, z, p, q, t
+constexpr size_t kVectors = 5;                            // r, z, p, q, p2
 constexpr size_t kVecOffset = kPartials + kStateDoubles + kScalDoubles;
 constexpr size_t kScratchDoubles = kVecOffset + kVectors * kNoAllocLen;
 static_assert(sizeof(CgState) <= kStateDoubles * sizeof(double), "CgState does not fit its scratch slot");
@@ -123,7 +123,7 @@ extern "C" mk_status mk_spd_solve_noalloc(mk_ctx* c, const mk_op* A, const doubl
             Rebind<double> r2(w.z, vec + 1 * kNoAllocLen, kNoAllocLen);
             Rebind<double> r3(w.p, vec + 2 * kNoAllocLen, kNoAllocLen);
             Rebind<double> r4(w.q, vec + 3 * kNoAllocLen, kNoAllocLen);
-            Rebind<double> r5(w.t, vec + 4 * kNoAllocLen, kNoAllocLen);
+            Rebind<double> r5(w.p2, vec + 4 * kNoAllocLen, kNoAllocLen);
             const bool timing = c->time_spmv;
             c->time_spmv = false;  // event timing creates events on first use
             struct RestoreTiming { mk_ctx* c; bool on; ~RestoreTiming() { c->time_spmv = on; } } rt{c, timing};

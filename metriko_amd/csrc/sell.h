@@ -18,32 +18,52 @@ static constexpr int kSellMaxLen = 12;
 // wavefronts instead of one serial chain)
 static constexpr int kLongSeg = 128;
 
+// Sum over the wavefront, the same in every lane, by DPP row shifts and broadcasts: no LDS round
+// trips (the xor-butterfly's twelve ds_bpermute per double made a reduction of 16 quantities take
+// 4 us).  Fixed order.
+template <int CTRL>
+__device__ __forceinline__ double dpp_shift(double v) {  // lanes without a source get 0
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+// row_bcast: the last lane of a row of 16 to the next row (CTRL 0x142, rows 1 and 3) or of the lower
+// half to the upper (0x143, rows 2 and 3); other rows get 0
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_bcast(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+    v += dpp_shift<0x111>(v);  // row_shr:1, 2, 4, 8
+    v += dpp_shift<0x112>(v);
+    v += dpp_shift<0x114>(v);
+    v += dpp_shift<0x118>(v);
+    v += dpp_bcast<0x142, 0xa>(v);
+    v += dpp_bcast<0x143, 0xc>(v);
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                            __builtin_amdgcn_readlane(__double2loint(v), 63));
 }
 
-// Block-reduce K values; thread 0 gets the block totals.
-template <int K>
+// Block-reduce K values; every thread gets the block totals.  One barrier: a kernel that reduces more
+// than once gives each reduction its own TAG (its own LDS).
+template <int K, int TAG = 0>
 __device__ __forceinline__ void block_sum(double (&v)[K]) {
     __shared__ double sh[K][kMaxWaves];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
 #pragma unroll
     for (int k = 0; k < K; k++) {
-        double s = wave_sum(v[k]);
+        const double s = wave_sum(v[k]);
         if (lane == 0) sh[k][wid] = s;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
 #pragma unroll
-        for (int k = 0; k < K; k++) {
-            double s = 0.0;
-            for (int w = 0; w < nw; w++) s += sh[k][w];
-            v[k] = s;
-        }
+    for (int k = 0; k < K; k++) {
+        double s = 0.0;
+        for (int w = 0; w < nw; w++) s += sh[k][w];
+        v[k] = s;
     }
-    __syncthreads();
 }
 
 // Fence-free grid reduction in two launches: the working kernel leaves one partial sum per
@@ -59,24 +79,17 @@ __device__ __forceinline__ void partials_write(double (&v)[K], double* partials)
         for (int k = 0; k < K; k++) partials[k * kMaxParts + blockIdx.x] = v[k];
     }
 }
-// Sum of nparts partials per value, fixed order; every thread of the (single) block gets tot.
+// Sum of nparts partials per value, fixed order; every thread of the block gets tot.
 template <int K>
 __device__ __forceinline__ void partials_sum(const double* __restrict__ partials, int nparts, double (&tot)[K]) {
-    __shared__ double shtot[K];
-    double acc[K];
 #pragma unroll
-    for (int k = 0; k < K; k++) {
-        acc[k] = 0.0;
-        for (int i = threadIdx.x; i < nparts; i += blockDim.x) acc[k] += partials[k * kMaxParts + i];
+    for (int k = 0; k < K; k++) tot[k] = 0.0;
+#pragma unroll 4
+    for (int i = threadIdx.x; i < nparts; i += blockDim.x) {
+#pragma unroll
+        for (int k = 0; k < K; k++) tot[k] += partials[k * kMaxParts + i];
     }
-    block_sum<K>(acc);
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int k = 0; k < K; k++) shtot[k] = acc[k];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < K; k++) tot[k] = shtot[k];
+    block_sum<K, 1>(tot);
 }
 
 // The blocks of a launch go round-robin over the 8 XCDs, each with its own L2.  xcd_block maps
@@ -302,12 +315,6 @@ __device__ __forceinline__ bool spmv_row_g(const SellDev<T>& A, const G& g, int 
     return spmv_row_gp<T, CPLX>(A, g, vb, row, ar, ai, none);
 }
 
-
-template <typename T, bool CPLX>
-__device__ __forceinline__ bool spmv_row(const SellDev<T>& A, const T* __restrict__ x, int vb, int& row, T& ar,
-                                         T& ai) {
-    return spmv_row_g<T, CPLX>(A, PlainGather<T, CPLX>{x}, vb, row, ar, ai);
-}
 
 static inline unsigned blocks_for(size_t len, int bs = 256) { return unsigned((len + bs - 1) / bs); }
 // grid of the grid-stride reduction kernels: few enough blocks that the per-block arrival
