@@ -6,9 +6,9 @@
 // length inside windows of sigma rows (perm maps a stored row to the original row).
 //
 // Reductions are deterministic: each block reduces with xor-butterfly shuffles
-// (DPP / ds_swizzle on CDNA) and LDS, writes one partial per block, and the last
-// block to arrive (atomic ticket) sums the partials in a fixed order.  Reruns are
-// therefore bit-identical.
+// (DPP on CDNA) and LDS and writes one partial per block; the kernel that needs the total, or a
+// one-block kernel in between, sums the partials in a fixed order.  Reruns are therefore
+// bit-identical.
 #include <algorithm>
 #include <chrono>
 #include <memory>
@@ -147,7 +147,10 @@ __global__ void __launch_bounds__(256) cg_init(int n, const T* __restrict__ r, c
 // stores what the host reads); above that, one-block kernels add them in between.  A one-block
 // kernel costs 2.3 to 3 us, a fold of 200 partials 0.6: with folds and the update of p inside the
 // product (from the old p of the gathered rows; p alternates between two buffers) a Jacobi
-// iteration on 50,953 rows went from five launches of 18.4 us to two of 9.
+// iteration on 50,953 rows went from five launches to two (703 iterations 14 to 8.4 ms, 20 to 12 us
+// each).  The line: every block reads all partials, so the fold grows with the square of the grid;
+// with it at 4096 a field on 655,362 vertices took 501 ms (455 at 2048) and 655,743 unknowns 5.15 ms
+// (4.8); at 1024 no size measured was faster than at 2048.
 static constexpr unsigned kFoldParts = 2048;
 static constexpr int kRowRz = 0, kRowRr = 1, kRowPq = 2;
 
@@ -398,13 +401,14 @@ static constexpr int kRowUpd = 3;
 __global__ void __launch_bounds__(256) cgm_update(size_t len, double* __restrict__ x, double* __restrict__ r,
                                                 float* __restrict__ r32, const double* __restrict__ p,
                                                 const double* __restrict__ q, CgState* st, double* partials, int npq) {
-    if (st->done) return;
+    const int done = st->done;
     const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
     // the first element's loads are in flight while alpha is folded
     size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     const size_t stride = size_t(gridDim.x) * blockDim.x;
     double xi = 0.0, ri = 0.0, pi = 0.0, qi = 0.0;
     if (i < len) { xi = x[i]; ri = r[i]; pi = p[i]; qi = q[i]; }
+    if (done) return;
     double alpha;
     if (npq) {
         const double rz_new = st->rz_new;
@@ -502,29 +506,44 @@ struct CgmOperands {
 template <bool CPLX>
 __global__ void __launch_bounds__(256) cgm_spmv(SellDev<double> A, const float* __restrict__ z32, double* p, double* q,
                                               double* __restrict__ zold, CgState* st, double* partials, int nin) {
-    if (st->done) return;
+    // the state and the first partials are loaded ahead of the row, used behind it
+    const int done = st->done;
     constexpr int W = CPLX ? 2 : 1;
     double beta = st->beta;
-    bool folded = nin == 0;
+    const double rz = st->rz;
+    const int first = st->first;
+    double pre[2][2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int i = threadIdx.x + u * blockDim.x;
+#pragma unroll
+        for (int k = 0; k < 2; k++) pre[u][k] = i < nin ? partials[k * kMaxParts + i] : 0.0;
+    }
+    bool folded = false;
     double contrib = 0.0;
     for (int vb = blockIdx.x; vb < A.nvb; vb += gridDim.x) {
         int row = 0;
         double a[2];
         CgmOperands<CPLX> o{z32, p, q};
         const bool own = spmv_row_gp<double, CPLX>(A, Fp32Gather<CPLX>{z32}, vb, row, a[0], a[1], o);
-        if (!folded) {  // a and m, while the first row's gathers are in flight; rz_new is cgm_update's
-            const double rz = st->rz;
-            const int first = st->first;
-            double tot[2];
-            partials_sum<2>(partials, nin, tot);
-            const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
-            if (!(tot[0] > 0.0)) {
-                if (writer) { st->status = (tot[0] == tot[0]) ? MK_ERR_NOT_SPD : MK_ERR_NAN; st->done = 1; }
-                return;
-            }
-            beta = first ? 0.0 : (tot[0] - tot[1]) / rz;
-            if (writer) st->rz_new = tot[0];
+        if (!folded) {
+            if (done) return;
             folded = true;
+            if (nin) {  // a and m; rz_new is cgm_update's
+                double tot[2] = {pre[0][0] + pre[1][0], pre[0][1] + pre[1][1]};
+                for (int i = threadIdx.x + 2 * blockDim.x; i < nin; i += blockDim.x) {
+                    tot[0] += partials[i];
+                    tot[1] += partials[kMaxParts + i];
+                }
+                block_sum<2, 1>(tot);
+                const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+                if (!(tot[0] > 0.0)) {
+                    if (writer) { st->status = (tot[0] == tot[0]) ? MK_ERR_NOT_SPD : MK_ERR_NAN; st->done = 1; }
+                    return;
+                }
+                beta = first ? 0.0 : (tot[0] - tot[1]) / rz;
+                if (writer) st->rz_new = tot[0];
+            }
         }
         if (!own) continue;
 #pragma unroll
@@ -1381,10 +1400,11 @@ static CgResult cg_run(mk_ctx* c, const mk_op* A, const T* val, const T* dinv, c
                                        (const CgState*)st, part);
             }
             if (fold && k + 1 < batch) continue;
-            if (mg)
-                hipLaunchKernelGGL((cg_beta_fin<false>), dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gn));
-            else
-                hipLaunchKernelGGL((cg_beta_fin<true>), dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gn));
+            // as many threads as the fold has, so the order of the sum, and with it every bit of the
+            // solution, does not depend on where a batch ends
+            const dim3 nt(fold ? A->block : 1024);
+            if (mg) hipLaunchKernelGGL((cg_beta_fin<false>), dim3(1), nt, 0, c->stream, st, (const double*)part, int(gn));
+            else hipLaunchKernelGGL((cg_beta_fin<true>), dim3(1), nt, 0, c->stream, st, (const double*)part, int(gn));
         }
     };
     return drive(c, hint, maxiter, check_every, [&](int batch) {
