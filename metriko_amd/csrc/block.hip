@@ -16,7 +16,8 @@
 
 namespace mk {
 
-static constexpr int kBlkParts = 2048;  // grid of the column-reduction kernels
+static constexpr int kBlkParts = 2048;   // grid of the column-reduction kernels
+static constexpr int kBlkStride = 4096;  // partials kept per column: bk_step's three launches fill up to all of them
 
 // 16-byte vectors of T (4 floats or 2 doubles) carried by one lane
 template <typename T>
@@ -67,6 +68,11 @@ __device__ __forceinline__ float4 vscale(float a, const float4& x) {
 }
 __device__ __forceinline__ double2 vscale(double a, const double2& x) { return make_double2(a * x.x, a * x.y); }
 
+// what a lane gathers, in the type it sums in (an FP64 product gathers FP32 vectors in bk_step)
+__device__ __forceinline__ const float4& wide(const float4& v) { return v; }
+__device__ __forceinline__ const double2& wide(const double2& v) { return v; }
+__device__ __forceinline__ double2 wide(const float2& v) { return make_double2(double(v.x), double(v.y)); }
+
 // Y = A X (MODE 0), Y = B - A X (3), Y += A X (4) for MW right-hand sides.  MODES 5-7: one
 // Chebyshev smoothing step fused with the residual it needs, in the three-term form (the
 // step d_{k-1} of the two-term form is x_k - x_{k-1}), row-local, X = x_k (gathered) and
@@ -108,18 +114,19 @@ __device__ __forceinline__ void spmm_store(const V& acc, int row, int j, const V
 // Gathered row c of the iterate: X's (lane vector j), or in mode 8 x_1 = c0 D^-1 B formed on
 // the fly (the same product the separate first step would have stored).
 template <typename T, int MODE, int LPR, typename V>
-__device__ __forceinline__ V gather_row(const V* __restrict__ Gv, const T* __restrict__ dinv, T c0, int c, int j) {
-    const V g = Gv[size_t(c) * LPR + j];
+__device__ __forceinline__ auto gather_row(const V* __restrict__ Gv, const T* __restrict__ dinv, T c0, int c, int j) {
+    const auto g = wide(Gv[size_t(c) * LPR + j]);
     if constexpr (MODE == 8) return vscale(c0 * dinv[c], g);
     else return g;
 }
 
 // Sum over entries [k0, k1) of a CSR row (stride R between a lane group's entries, starting
 // at k0 + sub): eight independent gathers in flight per lane.
-template <typename T, int R, int LPR, int MODE, typename V>
-__device__ __forceinline__ V chain_sum(int64_t k0, int64_t k1, int sub, int j, const int* __restrict__ cols,
-                                       const T* __restrict__ vals, const V* __restrict__ Xv,
-                                       const T* __restrict__ dinv, T s0) {
+template <typename T, int R, int LPR, int MODE, typename G>
+__device__ __forceinline__ auto chain_sum(int64_t k0, int64_t k1, int sub, int j, const int* __restrict__ cols,
+                                          const T* __restrict__ vals, const G* __restrict__ Xv,
+                                          const T* __restrict__ dinv, T s0) {
+    using V = typename Vec16<T>::type;
     V acc, a1, a2, a3, a4, a5, a6, a7;
     vzero(acc); vzero(a1); vzero(a2); vzero(a3); vzero(a4); vzero(a5); vzero(a6); vzero(a7);
     int64_t k = k0 + sub;
@@ -371,7 +378,7 @@ template void spmm_launch<float>(mk_ctx*, const mk_op*, int, const float*, float
 
 // Per-column partial sums of K quantities of this block (the thread's column is
 // threadIdx.x % MW, blockDim 256, grid <= kBlkParts), stored at
-// partials[(k * 64 + j) * kBlkParts + block].  No fence or ticket: a finishing kernel with one
+// partials[(k * 64 + j) * kBlkStride + block].  No fence or ticket: a finishing kernel with one
 // block per column adds them (colsum_total) after the kernel boundary, in a fixed order.
 template <int K, int MW>
 __device__ __forceinline__ void colsum_write(double (&v)[K], double* partials) {
@@ -389,7 +396,7 @@ __device__ __forceinline__ void colsum_write(double (&v)[K], double* partials) {
         const int t = threadIdx.x;
 #pragma unroll
         for (int k = 0; k < K; k++)
-            partials[(size_t(k) * 64 + t) * kBlkParts + blockIdx.x] = sh[k][0][t] + sh[k][1][t] + sh[k][2][t] + sh[k][3][t];
+            partials[(size_t(k) * 64 + t) * kBlkStride + blockIdx.x] = sh[k][0][t] + sh[k][1][t] + sh[k][2][t] + sh[k][3][t];
     }
 }
 // Totals of column j over nparts blocks (one block of 256 threads per column, reading the
@@ -401,7 +408,7 @@ template <int K>
 __device__ __forceinline__ void colsum_total(const double* __restrict__ partials, int nparts, int j, double (&tot)[K]) {
 #pragma unroll
     for (int k = 0; k < K; k++) {
-        const double* pk = partials + (size_t(k) * 64 + j) * kBlkParts;
+        const double* pk = partials + (size_t(k) * 64 + j) * kBlkStride;
         double a = 0.0;
 #pragma unroll 8
         for (int b = threadIdx.x; b < nparts; b += 256) a += pk[b];
@@ -444,14 +451,15 @@ __global__ void __launch_bounds__(256) bk_init0_fin(BState* st, const double* __
     }
 }
 
-// P = Z ; rz_j = R.Z ; rr_j = R.R ; done flags
+// P = Q = 0 (bk_step starts from beta = 0) ; rz_j = R.Z ; rr_j = R.R ; done flags
 template <int MW, typename ZT>
 __global__ void __launch_bounds__(256) bk_init1(size_t len, const double* __restrict__ R, const ZT* __restrict__ Z,
-                                              double* __restrict__ P, double* partials) {
+                                              double* __restrict__ P, double* __restrict__ Q, double* partials) {
     double v[2] = {0.0, 0.0};
     for (size_t e = size_t(blockIdx.x) * 256 + threadIdx.x; e < len; e += size_t(gridDim.x) * 256) {
         const double z = double(Z[e]), r = R[e];
-        P[e] = z;
+        P[e] = 0.0;
+        Q[e] = 0.0;
         v[0] += r * z;
         v[1] += r * r;
     }
@@ -473,17 +481,133 @@ __global__ void __launch_bounds__(256) bk_init1_fin(BState* st, const double* __
     }
 }
 
-// pq_j = P.Q ; alpha_j = rz_j / pq_j (0 for finished columns)
-template <int MW>
-__global__ void __launch_bounds__(256) bk_alpha(size_t len, const double* __restrict__ P, const double* __restrict__ Q,
-                                              const BState* st, double* partials) {
+// X += alpha P (the previous iteration's step) ; P = Z + beta P ; Q = A Z + beta Q (Q follows A P
+// without a product with P) ; pq_j = P.Q.  A block of 64 FP64 vectors is 512 bytes a row: this is
+// bound by the passes over them and by the L2's gathers, so the product gathers the V-cycle's FP32
+// output (half the bytes of P) and the row's own P, Q and X pass once, loaded with its columns.  At
+// 302,102 rows x 64 the product with P, P.Q, the update of P and that of X in bk_update took 340 us
+// an iteration, this 227 (4.4 TB/s; a large copy reaches 5.1).  Finished columns keep P and Q; their last step still reaches X (their alpha
+// is 0 from the next bk_alpha_fin on).
+// PART 1: the SELL rows, a wavefront's R at a time; 2: medium rows, a wavefront each, and the
+// segments' partial sums of the long rows; 3: the long rows.  Grid-stride over nw wavefronts' worth of
+// work; the launches leave their partials behind one another (block + pbase).
+template <int MW, typename ZT, int PART>
+__global__ void __launch_bounds__(256) bk_step(SellDev<double> A, int nw, const ZT* __restrict__ Z, double* __restrict__ P,
+                                             double* __restrict__ Q, double* __restrict__ X, BState* st,
+                                             double* partials, int pbase) {
     if (st->all_done) return;
-    double v[1] = {0.0};
-    for (size_t e = size_t(blockIdx.x) * 256 + threadIdx.x; e < len; e += size_t(gridDim.x) * 256) v[0] += P[e] * Q[e];
-    colsum_write<1, MW>(v, partials);
+    if (PART == 1 && blockIdx.x == 0 && threadIdx.x == 0) st->stepped = 1;
+    constexpr int LPR = MW / 2, R = 64 / LPR;
+    using G = typename std::conditional<std::is_same<ZT, float>::value, float2, double2>::type;
+    const G* __restrict__ Zv = reinterpret_cast<const G*>(Z);
+    double2* __restrict__ Pv = reinterpret_cast<double2*>(P);
+    double2* __restrict__ Qv = reinterpret_cast<double2*>(Q);
+    double2* __restrict__ Xv = reinterpret_cast<double2*>(X);
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int sub = lane / LPR, j = lane - sub * LPR;
+    const double a0 = st->alpha[2 * j], a1 = st->alpha[2 * j + 1], b0 = st->beta[2 * j], b1 = st->beta[2 * j + 1];
+    const bool d0 = st->done[2 * j], d1 = st->done[2 * j + 1];
+    double2 pq = make_double2(0.0, 0.0);
+    auto finish_row = [&](const double2& acc, const double2& z, const double2& p, const double2& q, const double2& x, size_t o) {
+        const double2 pn = make_double2(d0 ? p.x : z.x + b0 * p.x, d1 ? p.y : z.y + b1 * p.y);
+        const double2 qn = make_double2(d0 ? q.x : acc.x + b0 * q.x, d1 ? q.y : acc.y + b1 * q.y);
+        Xv[o] = make_double2(a0 != 0.0 ? x.x + a0 * p.x : x.x, a1 != 0.0 ? x.y + a1 * p.y : x.y);
+        Pv[o] = pn;
+        Qv[o] = qn;
+        pq.x += pn.x * qn.x;
+        pq.y += pn.y * qn.y;
+    };
+    const int nvb = (nw + 3) >> 2;
+    for (int vb = blockIdx.x; vb < nvb; vb += gridDim.x) {
+        const int gw = __builtin_amdgcn_readfirstlane(xcd_block(vb, nvb) * 4 + wid);
+        if (gw >= nw) continue;
+        if constexpr (PART == 1) {
+            const int r = gw * R + sub, r0 = gw * R;
+            if (r >= A.n_short) continue;
+            const int s = A.C == 64 ? r0 >> 6 : r0 / A.C;  // R divides 64 and 64 divides C: one slice
+            const int64_t base = A.slice_ptr[s];
+            const int w = A.slice_w[s];
+            const int row = A.perm ? A.perm[r] : r;
+            const size_t o = size_t(row) * LPR + j;
+            const int* __restrict__ col = A.col + base + (r - s * A.C);
+            const double* __restrict__ val = A.val + base + (r - s * A.C);
+            int ci[kSellMaxLen];
+            double cv[kSellMaxLen];
+#pragma unroll
+            for (int k = 0; k < kSellMaxLen; k++)
+                if (k < w) {
+                    ci[k] = col[k * A.C];
+                    cv[k] = val[k * A.C];
+                }
+            const double2 p = Pv[o], q = Qv[o], x = Xv[o];
+            const double2 z = wide(Zv[o]);
+            double2 acc = make_double2(0.0, 0.0);
+            constexpr int kG = 8;
+#pragma unroll
+            for (int k0 = 0; k0 < kSellMaxLen; k0 += kG) {
+                if (k0 >= w) break;
+                G xg[kG];
+#pragma unroll
+                for (int u = 0; u < kG; u++)
+                    if (k0 + u < kSellMaxLen && k0 + u < w) xg[u] = Zv[size_t(ci[k0 + u]) * LPR + j];
+#pragma unroll
+                for (int u = 0; u < kG; u++)
+                    if (k0 + u < kSellMaxLen && k0 + u < w) vfma(acc, cv[k0 + u], wide(xg[u]));
+            }
+            finish_row(acc, z, p, q, x, o);
+        } else if constexpr (PART == 2) {
+            const bool mid = gw < A.nmid;
+            const int e = mid ? gw : gw - A.nmid;
+            double2 acc = mid ? chain_sum<double, R, LPR, 0>(A.mid_ptr[e], A.mid_ptr[e + 1], sub, j, A.mid_col, A.mid_val, Zv,
+                                                             (const double*)nullptr, 0.0)
+                              : chain_sum<double, R, LPR, 0>(A.seg_beg[e], A.seg_end[e], sub, j, A.long_col, A.long_val, Zv,
+                                                             (const double*)nullptr, 0.0);
+#pragma unroll
+            for (int off = LPR; off < 64; off <<= 1) vshfl_add(acc, off);
+            if (sub != 0) continue;
+            if (mid) {
+                const size_t o = size_t(A.mid_rows[e]) * LPR + j;
+                finish_row(acc, wide(Zv[o]), Pv[o], Qv[o], Xv[o], o);
+            } else {
+                reinterpret_cast<double2*>(A.seg_part)[size_t(e) * LPR + j] = acc;
+            }
+        } else {
+            if (sub != 0) continue;
+            const double2* __restrict__ S = reinterpret_cast<const double2*>(A.seg_part);
+            double2 acc = make_double2(0.0, 0.0);
+            for (int q = A.lseg_ptr[gw]; q < A.lseg_ptr[gw + 1]; q++) acc = vadd(acc, S[size_t(q) * LPR + j]);
+            const size_t o = size_t(A.long_rows[gw]) * LPR + j;
+            finish_row(acc, wide(Zv[o]), Pv[o], Qv[o], Xv[o], o);
+        }
+    }
+    // the block's sums per column: its wavefronts' lane groups, then the wavefronts
+    __shared__ double sh[4][MW];
+#pragma unroll
+    for (int off = LPR; off < 64; off <<= 1) vshfl_add(pq, off);
+    if (sub == 0) {
+        sh[wid][2 * j] = pq.x;
+        sh[wid][2 * j + 1] = pq.y;
+    }
+    __syncthreads();
+    if (threadIdx.x < MW) {
+        const int t = threadIdx.x;
+        partials[size_t(t) * kBlkStride + pbase + blockIdx.x] = sh[0][t] + sh[1][t] + sh[2][t] + sh[3][t];
+    }
 }
+// The step of the last iteration, which no bk_step follows: X += alpha P.
+template <int MW>
+__global__ void __launch_bounds__(256) bk_last_step(size_t len, double* __restrict__ X, const double* __restrict__ P,
+                                                  const BState* st) {
+    const double alpha = st->alpha[threadIdx.x % MW];
+    if (alpha == 0.0) return;
+    for (size_t e = size_t(blockIdx.x) * 256 + threadIdx.x; e < len; e += size_t(gridDim.x) * 256) X[e] += alpha * P[e];
+}
+
+// alpha_j = rz_j / pq_j (0 for finished columns).  Nothing where bk_step was skipped: the alpha of the
+// iteration that finished the last column is then still to be applied.
 template <int MW>
 __global__ void __launch_bounds__(256) bk_alpha_fin(BState* st, const double* __restrict__ partials, int nparts) {
+    if (!st->stepped) return;
     const int j = blockIdx.x;
     if (st->done[j]) {  // only this block writes done[j]: uniform
         if (threadIdx.x == 0) st->alpha[j] = 0.0;
@@ -503,10 +627,9 @@ __global__ void __launch_bounds__(256) bk_alpha_fin(BState* st, const double* __
     }
 }
 
-// X += alpha P ; R -= alpha Q ; Rz = ZT(R) (none for an FP64 V-cycle) ; rr_j ; convergence
+// R -= alpha Q ; Rz = ZT(R) (none for an FP64 V-cycle) ; rr_j ; convergence
 template <int MW, typename ZT>
-__global__ void __launch_bounds__(256) bk_update(size_t len, double* __restrict__ X, double* __restrict__ R,
-                                               ZT* __restrict__ Rz, const double* __restrict__ P,
+__global__ void __launch_bounds__(256) bk_update(size_t len, double* __restrict__ R, ZT* __restrict__ Rz,
                                                const double* __restrict__ Q, const BState* st, double* partials) {
     if (st->all_done) return;
     const double alpha = st->alpha[threadIdx.x % MW];
@@ -514,7 +637,6 @@ __global__ void __launch_bounds__(256) bk_update(size_t len, double* __restrict_
     for (size_t e = size_t(blockIdx.x) * 256 + threadIdx.x; e < len; e += size_t(gridDim.x) * 256) {
         double r = R[e];
         if (alpha != 0.0) {
-            X[e] += alpha * P[e];
             r -= alpha * Q[e];
             R[e] = r;
             if (Rz) Rz[e] = ZT(r);
@@ -526,6 +648,7 @@ __global__ void __launch_bounds__(256) bk_update(size_t len, double* __restrict_
 template <int MW>
 __global__ void __launch_bounds__(256) bk_update_fin(BState* st, const double* __restrict__ partials, int nparts) {
     const int j = blockIdx.x;
+    if (j == 0 && threadIdx.x == 0) st->stepped = 0;
     if (st->done[j]) return;
     double tot[1];
     colsum_total<1>(partials, nparts, j, tot);
@@ -569,22 +692,30 @@ __global__ void __launch_bounds__(256) bk_beta_fin(BState* st, const double* __r
     }
 }
 
-// P = Z + beta P (running columns only)
-template <int MW, typename ZT>
-__global__ void __launch_bounds__(256) bk_pupdate(size_t len, double* __restrict__ P, const ZT* __restrict__ Z,
-                                                const BState* st) {
-    if (st->all_done) return;
-    const int j = threadIdx.x % MW;
-    if (st->done[j]) return;
-    const double beta = st->beta[j];
-    for (size_t e = size_t(blockIdx.x) * 256 + threadIdx.x; e < len; e += size_t(gridDim.x) * 256)
-        P[e] = double(Z[e]) + beta * P[e];
-}
-
 __global__ void k_set_bstate(BState* st, double tol2) {
     st->tol2 = tol2;
     st->all_done = 0;
     st->ndone = 0;
+    st->stepped = 0;
+}
+
+// Launches bk_step; returns the number of partials it leaves per column.
+template <int MW, typename ZT>
+static int block_step(mk_ctx* c, const mk_op* A, const ZT* Z, double* P, double* Q, double* X, BState* st, double* part) {
+    unsigned gs = 0;
+    const SellDev<double> D = sell_dev<double>(A, A->val64.p, 256, &gs);
+    constexpr int R = 64 / (MW / 2);
+    const int nw1 = int((int64_t(A->n_short) + R - 1) / R), nw2 = int(int64_t(A->nmid) + A->nseg), nw3 = A->nlong;
+    auto blocks = [](int nw, int cap) { return std::min((nw + 3) / 4, cap); };
+    const int g1 = std::max(1, blocks(nw1, 2048)), g2 = blocks(nw2, 1536), g3 = blocks(nw3, 512);
+    static_assert(2048 + 1536 + 512 <= kBlkStride, "the three launches' partials fit a column's row");
+    const double vb = double(A->n) * MW;
+    SpmvTimer tm(c, A->bytes64 - double(A->n) * 16.0 + vb * (sizeof(ZT) + 6.0 * 8.0), A,
+                 MW == 64 ? "spmm64" : MW == 32 ? "spmm32" : MW == 16 ? "spmm16" : "spmm8", false, 3);
+    MK_TLAUNCH(tm, 0, (bk_step<MW, ZT, 1>), dim3(g1), dim3(256), 0, c->stream, D, nw1, Z, P, Q, X, st, part, 0);
+    if (g2) MK_TLAUNCH(tm, 1, (bk_step<MW, ZT, 2>), dim3(g2), dim3(256), 0, c->stream, D, nw2, Z, P, Q, X, st, part, g1);
+    if (g3) MK_TLAUNCH(tm, 2, (bk_step<MW, ZT, 3>), dim3(g3), dim3(256), 0, c->stream, D, nw3, Z, P, Q, X, st, part, g1 + g2);
+    return g1 + g2 + g3;
 }
 
 // ZT: the V-cycle's precision (float: FP32 multigrid inside the FP64 recurrences; double: an
@@ -594,7 +725,7 @@ static BlockResult block_pcg_mw(mk_ctx* c, const mk_op* A, Mg* mg, const double*
                                 int maxiter, int check_every) {
     constexpr bool fp64 = std::is_same<ZT, double>::value;
     const size_t len = size_t(A->n) * MW;
-    DevBuf<double> R(len), P(len), Q(len), part(size_t(2) * 64 * kBlkParts);
+    DevBuf<double> R(len), P(len), Q(len), part(size_t(2) * 64 * kBlkStride);
     // two preconditioned residual blocks, swapped every iteration: the flexible beta needs the
     // previous one (kept in the V-cycle's own precision, so no copy is made)
     DevBuf<ZT> Rz(fp64 ? 0 : len), Za(len), Zb(len);
@@ -613,8 +744,7 @@ static BlockResult block_pcg_mw(mk_ctx* c, const mk_op* A, Mg* mg, const double*
     hipLaunchKernelGGL((bk_init0_fin<MW>), dim3(MW), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
     mg_apply_block<ZT>(c, mg, MW, vin, zc, nullptr);
     hipLaunchKernelGGL((bk_init1<MW, ZT>), dim3(g), dim3(256), 0, c->stream, len, (const double*)R.p,
-                       (const ZT*)zc, P.p, part.p);
-    std::swap(zc, zo);
+                       (const ZT*)zc, P.p, Q.p, part.p);
     hipLaunchKernelGGL((bk_init1_fin<MW>), dim3(MW), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
     MK_HIP(hipGetLastError());
     static_assert(sizeof(BState) <= mk_ctx::kPinBytes, "BState does not fit the readback memory");
@@ -628,20 +758,16 @@ static BlockResult block_pcg_mw(mk_ctx* c, const mk_op* A, Mg* mg, const double*
     for (;;) {
         const int batch = std::max(0, std::min(plan, maxiter - iters));
         for (int k = 0; k < batch; k++) {
-            spmm_launch<double>(c, A, MW, P.p, Q.p, nullptr, SPMV_PLAIN, &st.p->all_done);
-            hipLaunchKernelGGL((bk_alpha<MW>), dim3(g), dim3(256), 0, c->stream, len, (const double*)P.p,
+            const int np = block_step<MW, ZT>(c, A, zc, P.p, Q.p, X, st.p, part.p);
+            std::swap(zc, zo);
+            hipLaunchKernelGGL((bk_alpha_fin<MW>), dim3(MW), dim3(256), 0, c->stream, st.p, (const double*)part.p, np);
+            hipLaunchKernelGGL((bk_update<MW, ZT>), dim3(g), dim3(256), 0, c->stream, len, R.p, rz,
                                (const double*)Q.p, (const BState*)st.p, part.p);
-            hipLaunchKernelGGL((bk_alpha_fin<MW>), dim3(MW), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
-            hipLaunchKernelGGL((bk_update<MW, ZT>), dim3(g), dim3(256), 0, c->stream, len, X, R.p, rz,
-                               (const double*)P.p, (const double*)Q.p, (const BState*)st.p, part.p);
             hipLaunchKernelGGL((bk_update_fin<MW>), dim3(MW), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
             mg_apply_block<ZT>(c, mg, MW, vin, zc, &st.p->all_done);
             hipLaunchKernelGGL((bk_beta<MW, ZT>), dim3(g), dim3(256), 0, c->stream, len, (const double*)R.p,
                                (const ZT*)zc, (const ZT*)zo, (const BState*)st.p, part.p);
             hipLaunchKernelGGL((bk_beta_fin<MW>), dim3(MW), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
-            hipLaunchKernelGGL((bk_pupdate<MW, ZT>), dim3(g), dim3(256), 0, c->stream, len, P.p, (const ZT*)zc,
-                               (const BState*)st.p);
-            std::swap(zc, zo);
         }
         iters += batch;
         MK_HIP(hipGetLastError());
@@ -662,6 +788,8 @@ static BlockResult block_pcg_mw(mk_ctx* c, const mk_op* A, Mg* mg, const double*
         for (int j = 0; j < MW; j++) prev_rr[j] = h.rr[j];
         prev_iters = iters;
     }
+    hipLaunchKernelGGL((bk_last_step<MW>), dim3(g), dim3(256), 0, c->stream, len, X, (const double*)P.p, (const BState*)st.p);
+    MK_HIP(hipGetLastError());
     BlockResult res;
     res.status = MK_OK;
     res.iters = 0;

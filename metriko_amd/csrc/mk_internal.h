@@ -151,6 +151,7 @@ struct BState {
     double rz[64], rr[64], rr0[64], bb[64], alpha[64], beta[64];
     int done[64], status[64], it[64];
     int all_done, ndone;  // every column finished; columns finished so far
+    int stepped;          // bk_step ran in this iteration
     double tol2;
 };
 struct BlockResult {

@@ -43,3 +43,31 @@ def test_a_column_with_nan_is_reported(gpu_ctx):
     B[5, 7] = 0.0
     X, _ = op.solve_many(B)  # the operator is still usable
     assert np.linalg.norm(A @ X - B) <= 1e-10 * np.linalg.norm(B)
+
+
+@pytest.mark.parametrize("precision", [mk.PREC_MIXED_MG, mk.PREC_FP64])
+@pytest.mark.parametrize("nx,ny", [(1, 1), (3, 1), (9, 7), (83, 61)])
+@pytest.mark.parametrize("m", [3, 16, 31, 64])
+def test_short_medium_and_long_rows(gpu_ctx, m, nx, ny, precision):
+    """Rows of every kind of the layout (5 entries; 24 to 60; hundreds to all of them), at counts below
+    and beside a wavefront's share; a right-hand side that is solved at once among the others, whose
+    last step is applied while they go on."""
+    A = _grid(nx, ny, 1e-2) if nx * ny > 1 else sp.csr_matrix([[3.0]])
+    n = A.shape[0]
+    rng = np.random.default_rng(n + m)
+    for _ in range(5):
+        k = rng.choice(n, min(30, n), replace=False)
+        v = sp.csr_matrix((np.full(k.size, 0.3 / np.sqrt(k.size)), (k, np.zeros(k.size, int))), shape=(n, 1))
+        A = A + v @ v.T
+    for row, size in ((0, n), (n // 2, (n + 1) // 2), (n - 1, min(n, 300))):  # couplings below the shift
+        k = rng.choice(n, size, replace=False)
+        v = sp.csr_matrix((np.full(size, 1e-3 / np.sqrt(size)), (np.full(size, row), k)), shape=(n, n))
+        A = A + v + v.T
+    B = rng.standard_normal((n, m))
+    B[:, 1] = A @ np.ones(n)
+    op = gpu_ctx.op_real(A)
+    X, st = op.solve_many(B, o=mk.opts(precision=precision))
+    res = np.linalg.norm(A @ X - B, axis=0) / np.linalg.norm(B, axis=0)
+    assert res.max() <= 1e-10
+    again, _ = op.solve_many(B, o=mk.opts(precision=precision))
+    assert np.array_equal(X, again)
