@@ -86,30 +86,45 @@ __device__ __forceinline__ double2 wide(const float2& v) { return make_double2(d
 // wavefront whose row groups split the entries.  PART 1 / 2: only the SELL rows / only the
 // medium and long rows (launched with nw_sell = 0), so the SELL launch does not carry the
 // registers of the eight-gather chains and runs at full occupancy.
-// Stores row `row` of the result (lane j of its LPR lanes): Y = acc (MODE 0), B - acc (3),
-// Y + acc (4), the Chebyshev updates (5-7, x_k = xd when the row's own entry was gathered).
-template <typename T, int MW, int MODE, typename V>
-__device__ __forceinline__ void spmm_store(const V& acc, int row, int j, const V* __restrict__ Xv, T* __restrict__ Y,
-                                           const T* __restrict__ B, const T* __restrict__ dinv, T ca, T cs, T c0,
-                                           bool have_xd, const V& xd) {
-    constexpr int LPR = MW / Vec16<T>::N;
-    V* Yv = reinterpret_cast<V*>(Y);
-    const size_t o = size_t(row) * LPR + j;
-    if constexpr (MODE == 0) Yv[o] = acc;
-    if constexpr (MODE == 3) Yv[o] = vsub(reinterpret_cast<const V*>(B)[o], acc);
-    if constexpr (MODE == 4) Yv[o] = vadd(Yv[o], acc);
-    if constexpr (MODE >= 5) {
-        const V bo = reinterpret_cast<const V*>(B)[o];
-        const V xo = have_xd ? xd : MODE == 8 ? vscale(c0 * dinv[row], bo) : Xv[o];
-        const V r = vsub(bo, acc);
-        const T sd = cs * dinv[row];
-        if constexpr (MODE == 5) Yv[o] = vaxpy(T(1), xo, sd, r);
-        if constexpr (MODE == 7 || MODE == 8) Yv[o] = vaxpy(T(1) + ca, xo, sd, r);
-        if constexpr (MODE == 6) Yv[o] = vaxpy(T(1), vaxpy(T(1) + ca, xo, -ca, Yv[o]), sd, r);
-        if constexpr (MODE == 9)
-            Yv[o] = vaxpy(T(1), vaxpy(T(1) + ca, xo, -ca, vscale(c0 * dinv[row], bo)), sd, r);
+// Bound by the L2's gathers and the chain slice -> columns -> gathers -> the row's own operands -> store
+// (a wavefront has few rows, so the chain repeats some ten times per compute unit slot): the slice's
+// position is a scalar load and the row's own operands (SpmmRow) are loaded ahead of the gathers.  FP32,
+// 302,102 rows x 64: mode 8 89 -> 80 us, 5 74 -> 65, 6 73 -> 69, 4 45 -> 42, 3 55 (unchanged).
+//
+// Row `row` of the result (lane j of its LPR lanes): Y = acc (MODE 0), B - acc (3), Y + acc (4),
+// the Chebyshev updates (5-9, x_k = xd when the row's own entry was gathered).
+template <typename T, int MW, int MODE>
+struct SpmmRow {
+    using V = typename Vec16<T>::type;
+    static constexpr int LPR = MW / Vec16<T>::N;
+    V b, y;
+    T d;
+    // the row's own operands
+    __device__ __forceinline__ void load(int row, int j, const T* __restrict__ Y, const T* __restrict__ B,
+                                         const T* __restrict__ dinv) {
+        const size_t o = size_t(row) * LPR + j;
+        if constexpr (MODE == 3 || MODE >= 5) b = reinterpret_cast<const V*>(B)[o];
+        if constexpr (MODE == 4 || MODE == 6) y = reinterpret_cast<const V*>(Y)[o];
+        if constexpr (MODE >= 5) d = dinv[row];
     }
-}
+    __device__ __forceinline__ void store(const V& acc, int row, int j, const V* __restrict__ Xv, T* __restrict__ Y, T ca,
+                                          T cs, T c0, bool have_xd, const V& xd) const {
+        const size_t o = size_t(row) * LPR + j;
+        V* Yv = reinterpret_cast<V*>(Y);
+        if constexpr (MODE == 0) Yv[o] = acc;
+        if constexpr (MODE == 3) Yv[o] = vsub(b, acc);
+        if constexpr (MODE == 4) Yv[o] = vadd(y, acc);
+        if constexpr (MODE >= 5) {
+            const V xo = have_xd ? xd : MODE == 8 ? vscale(c0 * d, b) : Xv[o];
+            const V r = vsub(b, acc);
+            const T sd = cs * d;
+            if constexpr (MODE == 5) Yv[o] = vaxpy(T(1), xo, sd, r);
+            if constexpr (MODE == 7 || MODE == 8) Yv[o] = vaxpy(T(1) + ca, xo, sd, r);
+            if constexpr (MODE == 6) Yv[o] = vaxpy(T(1), vaxpy(T(1) + ca, xo, -ca, y), sd, r);
+            if constexpr (MODE == 9) Yv[o] = vaxpy(T(1), vaxpy(T(1) + ca, xo, -ca, vscale(c0 * d, b)), sd, r);
+        }
+    }
+};
 
 // Gathered row c of the iterate: X's (lane vector j), or in mode 8 x_1 = c0 D^-1 B formed on
 // the fly (the same product the separate first step would have stored).
@@ -164,7 +179,8 @@ __global__ void __launch_bounds__(256) sell_spmm(SellDev<T> A, int nw_sell, cons
     const V* __restrict__ Xv = reinterpret_cast<const V*>(MODE == 8 ? B : X);
     const int lane = threadIdx.x & 63;
     const int sub = lane / LPR, j = lane - sub * LPR;
-    const int gw = xcd_block(int(blockIdx.x), int(gridDim.x)) * int(blockDim.x >> 6) + int(threadIdx.x >> 6);
+    const int gw = __builtin_amdgcn_readfirstlane(xcd_block(int(blockIdx.x), int(gridDim.x)) * int(blockDim.x >> 6) +
+                                                  int(threadIdx.x >> 6));
     V acc;
     vzero(acc);
     // modes 5-7 need the row's own x_k: taken from the gather of the diagonal entry, so the
@@ -173,13 +189,17 @@ __global__ void __launch_bounds__(256) sell_spmm(SellDev<T> A, int nw_sell, cons
     vzero(xd);
     bool have_xd = false;
     int row = -1;
+    SpmmRow<T, MW, MODE> own;
     if (PART != 2 && gw < nw_sell) {
         const int r = gw * R + sub;
         if (r >= A.n_short) return;
-        const int s = r / A.C, lr = r - s * A.C;
-        const int64_t base = A.slice_ptr[s] + lr;
+        // R divides 64 and 64 divides C: the wavefront's rows are in one slice, a scalar load
+        const int s = A.C == 64 ? (gw * R) >> 6 : (gw * R) / A.C, lr = r - s * A.C;
+        const int64_t base = A.slice_ptr[s];
         const int w = A.slice_w[s];
         row = A.perm ? A.perm[r] : r;
+        const int* __restrict__ col = A.col + base + lr;
+        const T* __restrict__ val = A.val + base + lr;
         // the row's column indices and values first (w <= kSellMaxLen, uniform in the
         // wavefront), then its gathers kG at a time in flight, summed in entry order
         int ci[kSellMaxLen];
@@ -187,9 +207,10 @@ __global__ void __launch_bounds__(256) sell_spmm(SellDev<T> A, int nw_sell, cons
 #pragma unroll
         for (int k = 0; k < kSellMaxLen; k++)
             if (k < w) {
-                ci[k] = A.col[base + int64_t(k) * A.C];
-                cv[k] = A.val[base + int64_t(k) * A.C];
+                ci[k] = col[k * A.C];
+                cv[k] = val[k * A.C];
             }
+        own.load(row, j, Y, B, dinv);
         constexpr int kG = 8;
 #pragma unroll
         for (int k0 = 0; k0 < kSellMaxLen; k0 += kG) {
@@ -217,6 +238,7 @@ __global__ void __launch_bounds__(256) sell_spmm(SellDev<T> A, int nw_sell, cons
             for (int off = LPR; off < 64; off <<= 1) vshfl_add(acc, off);
             if (sub != 0) return;
             row = A.mid_rows[lw];
+            own.load(row, j, Y, B, dinv);
         } else {  // a segment of a long row: its partial sum, combined by sell_spmm_long
             lw -= A.nmid;
             if (lw >= A.nseg) return;  // uniform inside the wavefront
@@ -228,7 +250,7 @@ __global__ void __launch_bounds__(256) sell_spmm(SellDev<T> A, int nw_sell, cons
             return;
         }
     }
-    spmm_store<T, MW, MODE>(acc, row, j, Xv, Y, B, dinv, ca, cs, c0, have_xd, xd);
+    own.store(acc, row, j, Xv, Y, ca, cs, c0, have_xd, xd);
 }
 
 // Long rows of the multi-column kernels: one wavefront per row adds its segments' partial
@@ -249,7 +271,9 @@ __global__ void __launch_bounds__(256) sell_spmm_long(SellDev<T> A, const T* __r
     for (int q = A.lseg_ptr[w]; q < A.lseg_ptr[w + 1]; q++) acc = vadd(acc, P[size_t(q) * LPR + j]);
     V xd;
     vzero(xd);
-    spmm_store<T, MW, MODE>(acc, A.long_rows[w], j, reinterpret_cast<const V*>(X), Y, B, dinv, ca, cs, c0, false, xd);
+    SpmmRow<T, MW, MODE> own;
+    own.load(A.long_rows[w], j, Y, B, dinv);
+    own.store(acc, A.long_rows[w], j, reinterpret_cast<const V*>(X), Y, ca, cs, c0, false, xd);
 }
 
 template <typename T, int MW>
@@ -486,7 +510,7 @@ __global__ void __launch_bounds__(256) bk_init1_fin(BState* st, const double* __
 // bound by the passes over them and by the L2's gathers, so the product gathers the V-cycle's FP32
 // output (half the bytes of P) and the row's own P, Q and X pass once, loaded with its columns.  At
 // 302,102 rows x 64 the product with P, P.Q, the update of P and that of X in bk_update took 340 us
-// an iteration, this 227 (4.4 TB/s; a large copy reaches 5.1).  Finished columns keep P and Q; their last step still reaches X (their alpha
+// an iteration, this 227 to 250 (4.0 to 4.4 TB/s; a large copy reaches 5.1).  Finished columns keep P and Q; their last step still reaches X (their alpha
 // is 0 from the next bk_alpha_fin on).
 // PART 1: the SELL rows, a wavefront's R at a time; 2: medium rows, a wavefront each, and the
 // segments' partial sums of the long rows; 3: the long rows.  Grid-stride over nw wavefronts' worth of

@@ -71,3 +71,12 @@ def test_short_medium_and_long_rows(gpu_ctx, m, nx, ny, precision):
     assert res.max() <= 1e-10
     again, _ = op.solve_many(B, o=mk.opts(precision=precision))
     assert np.array_equal(X, again)
+
+
+@pytest.mark.parametrize("height", [64, 128, 192, 256])
+@pytest.mark.parametrize("m", [8, 13, 64])
+def test_slice_heights(gpu_ctx, m, height):
+    A = _grid(37, 29, 1e-2)
+    B = np.random.default_rng(height).standard_normal((A.shape[0], m))
+    X, _ = gpu_ctx.op_real(A, o=mk.opts(slice_height=height)).solve_many(B)
+    assert (np.linalg.norm(A @ X - B, axis=0) / np.linalg.norm(B, axis=0)).max() <= 1e-10
