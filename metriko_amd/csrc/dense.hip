@@ -217,7 +217,7 @@ __global__ void __launch_bounds__(256) k_gj_update(int ld, int k0, double* __res
 template <typename T, bool CPLX, bool DOTS>
 __global__ void __launch_bounds__(256) k_dense_gemv(int n, int ld, const double* __restrict__ inv,
                                                     const T* __restrict__ b, T* __restrict__ x, const int* skip,
-                                                    const double* __restrict__ r, const double* __restrict__ xold,
+                                                    const double* __restrict__ r, const float* __restrict__ xold,
                                                     double* __restrict__ partials) {
     if (skip && *skip) return;
     const int row_ = blockIdx.x * 4 + int(threadIdx.x >> 6);
@@ -228,7 +228,7 @@ __global__ void __launch_bounds__(256) k_dense_gemv(int n, int ld, const double*
     // the row's entries of r and xold, in flight with the row
     double rv[2] = {0.0, 0.0}, ov[2] = {0.0, 0.0};
     if (DOTS && in && lane == 0)
-        for (int q = 0; q < (CPLX ? 2 : 1); q++) { rv[q] = r[(CPLX ? 2 : 1) * i + q]; ov[q] = xold[(CPLX ? 2 : 1) * i + q]; }
+        for (int q = 0; q < (CPLX ? 2 : 1); q++) { rv[q] = r[(CPLX ? 2 : 1) * i + q]; ov[q] = double(xold[(CPLX ? 2 : 1) * i + q]); }
     constexpr int kU = 4;
     const double2* __restrict__ row = reinterpret_cast<const double2*>(inv + size_t(i) * ld * (CPLX ? 2 : 1));
     const int nv = CPLX ? n : (n + 1) / 2;  // 16-byte pieces; an odd n's last one ends in the padding
@@ -357,7 +357,7 @@ DenseInverse::DenseInverse(mk_ctx* c, bool cplx_, int n_, const int64_t* ptr, co
 }
 
 template <typename T>
-unsigned DenseInverse::apply(mk_ctx* c, const T* b, T* x, const int* skip, const double* r, const double* xold,
+unsigned DenseInverse::apply(mk_ctx* c, const T* b, T* x, const int* skip, const double* r, const float* xold,
                              double* partials) const {
     const unsigned g = unsigned((n + 3) / 4);
 #define MK_GEMV(CP, DOTS)                                                                                               \
@@ -368,9 +368,9 @@ unsigned DenseInverse::apply(mk_ctx* c, const T* b, T* x, const int* skip, const
 #undef MK_GEMV
     return g;
 }
-template unsigned DenseInverse::apply<float>(mk_ctx*, const float*, float*, const int*, const double*, const double*,
+template unsigned DenseInverse::apply<float>(mk_ctx*, const float*, float*, const int*, const double*, const float*,
                                              double*) const;
-template unsigned DenseInverse::apply<double>(mk_ctx*, const double*, double*, const int*, const double*, const double*,
+template unsigned DenseInverse::apply<double>(mk_ctx*, const double*, double*, const int*, const double*, const float*,
                                               double*) const;
 
 template <typename T>

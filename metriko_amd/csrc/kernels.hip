@@ -390,7 +390,9 @@ __global__ void __launch_bounds__(256) cg_beta(int n, const T* __restrict__ r, c
 // FP64 PCG with an FP32 multigrid preconditioner (vectors as real arrays of len entries;
 // complex interleaved gives Re(r^H z) as the plain sum).  The preconditioner runs in FP32,
 // so it is not exactly symmetric: beta is the flexible (Polak-Ribiere) form
-// beta = r_{k+1}.(z_{k+1} - z_k) / r_k.z_k, with z_k kept in FP64 (zold).
+// beta = r_{k+1}.(z_{k+1} - z_k) / r_k.z_k, with z_k in the other of two FP32 buffers (zold).
+// (An FP64 copy of it, written by cgm_spmv and read for m, was 31 MB of an iteration's 1.1 GB on
+// 1,310,720 complex rows: 350 us an iteration with it, 342 without.)
 
 // The scalars go through the partials as in cg_step1 / cg_step2 (a = r.z and m = r.zold in rows 0 and
 // 1, p^H q in row 2, rr in row 3): folded by the kernel that needs them up to kFoldParts blocks.
@@ -451,13 +453,13 @@ __global__ void __launch_bounds__(1024) cgm_update_fin(CgState* st, const double
 // beta of the flexible recurrence: a = r.z32, m = r.zold; beta = (a - m) / rz (0 on the first
 // iteration); rz = a
 __global__ void __launch_bounds__(256) cgm_beta2(size_t len, const double* __restrict__ r,
-                                               const float* __restrict__ z32, const double* __restrict__ zold,
+                                               const float* __restrict__ z32, const float* __restrict__ zold,
                                                const CgState* st, double* partials) {
     if (st->done) return;
     double a = 0.0, m = 0.0;
     for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < len; i += size_t(gridDim.x) * blockDim.x) {
         a += r[i] * double(z32[i]);
-        m += r[i] * zold[i];
+        m += r[i] * double(zold[i]);
     }
     double v[2] = {a, m};
     partials_write<2>(v, partials);
@@ -476,7 +478,7 @@ __global__ void __launch_bounds__(1024) cgm_beta2_fin(CgState* st, const double*
     }
 }
 
-// p = z + beta p ; q = A z + beta q (q tracks A p without a second product) ; zold = z ;
+// p = z + beta p ; q = A z + beta q (q tracks A p without a second product) ;
 // pq = p^H q ; alpha = rz / pq.  z is the FP32 preconditioned residual, A and p, q FP64.
 template <bool CPLX>
 struct Fp32Gather {
@@ -505,7 +507,7 @@ struct CgmOperands {
 };
 template <bool CPLX>
 __global__ void __launch_bounds__(256) cgm_spmv(SellDev<double> A, const float* __restrict__ z32, double* p, double* q,
-                                              double* __restrict__ zold, CgState* st, double* partials, int nin) {
+                                              CgState* st, double* partials, int nin) {
     // the state and the first partials are loaded ahead of the row, used behind it
     const int done = st->done;
     constexpr int W = CPLX ? 2 : 1;
@@ -551,7 +553,6 @@ __global__ void __launch_bounds__(256) cgm_spmv(SellDev<double> A, const float* 
             const double pk = o.zv[k] + beta * o.pv[k], qk = a[k] + beta * o.qv[k];
             p[W * row + k] = pk;
             q[W * row + k] = qk;
-            zold[W * row + k] = o.zv[k];
             contrib += pk * qk;
         }
     }
@@ -576,13 +577,13 @@ __global__ void __launch_bounds__(1024) cgm_spmv_fin(CgState* st, const double* 
 // p = q = zold = 0 ; r32 = float(r) ; rr, bb ; state for the first iteration
 __global__ void __launch_bounds__(256) cgm_init(size_t len, const double* __restrict__ r, const double* __restrict__ b,
                                               float* __restrict__ r32, double* __restrict__ p, double* __restrict__ q,
-                                              double* __restrict__ zold, double* partials) {
+                                              float* __restrict__ zold, double* partials) {
     double rr = 0.0, bb = 0.0;
     for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < len; i += size_t(gridDim.x) * blockDim.x) {
         const double ri = r[i], bi = b[i];
         p[i] = 0.0;
         q[i] = 0.0;
-        zold[i] = 0.0;
+        zold[i] = 0.f;
         r32[i] = float(ri);
         rr += ri * ri;
         bb += bi * bi;
@@ -1122,17 +1123,17 @@ template <typename T, bool CPLX>
 struct DotOperands {
     static constexpr int W = CPLX ? 2 : 1;
     const double* __restrict__ r;
-    const double* __restrict__ yold;
+    const float* __restrict__ yold;
     double rv[W], ov[W];
     __device__ __forceinline__ void operator()(int row) {
 #pragma unroll
-        for (int q = 0; q < W; q++) { rv[q] = r[W * row + q]; ov[q] = yold[W * row + q]; }
+        for (int q = 0; q < W; q++) { rv[q] = r[W * row + q]; ov[q] = double(yold[W * row + q]); }
     }
 };
 template <typename T, bool CPLX, bool DOTS>
 __global__ void __launch_bounds__(256) sell_spmv2(SellDev<T> A, int m1, const T* __restrict__ u, const T* __restrict__ v,
                                                 T* __restrict__ y, const int* skip, const double* __restrict__ r,
-                                                const double* __restrict__ yold, double* __restrict__ partials) {
+                                                const float* __restrict__ yold, double* __restrict__ partials) {
     if (skip && *skip) return;
     int row = 0;
     T a[2];
@@ -1159,7 +1160,7 @@ __global__ void __launch_bounds__(256) sell_spmv2(SellDev<T> A, int m1, const T*
 // r (with yold and partials): the dots too; returns the number of partials
 template <typename T>
 unsigned spmv2_launch(mk_ctx* c, const mk_op* A, int m1, const T* u, const T* v, T* y, const int* skip, const char* name,
-                      const double* r, const double* yold, double* partials) {
+                      const double* r, const float* yold, double* partials) {
     unsigned g = 0;
     const T* val;
     if constexpr (std::is_same<T, double>::value) val = A->val64.p;
@@ -1175,9 +1176,9 @@ unsigned spmv2_launch(mk_ctx* c, const mk_op* A, int m1, const T* u, const T* v,
     return g;
 }
 template unsigned spmv2_launch<double>(mk_ctx*, const mk_op*, int, const double*, const double*, double*, const int*,
-                                       const char*, const double*, const double*, double*);
+                                       const char*, const double*, const float*, double*);
 template unsigned spmv2_launch<float>(mk_ctx*, const mk_op*, int, const float*, const float*, float*, const int*,
-                                      const char*, const double*, const double*, double*);
+                                      const char*, const double*, const float*, double*);
 
 template <typename T>
 __global__ void k_copy(size_t len, const T* __restrict__ x, T* __restrict__ y, const int* skip) {
@@ -1457,34 +1458,35 @@ CgResult cg64_mg32(mk_ctx* c, const mk_op* A, const double* b, double* x, double
                    int check_every, Mg* mg) {
     Work& w = work(c);
     const size_t len = size_t(A->n) * (A->cplx ? 2 : 1);
-    w.r.ensure(len); w.z.ensure(len); w.p.ensure(len); w.q.ensure(len);
-    w.r32.ensure(len); w.z32.ensure(len);
+    w.r.ensure(len); w.p.ensure(len); w.q.ensure(len);
+    w.r32.ensure(len); w.z32.ensure(len); w.z2_32.ensure(len);
+    float *zc = w.z32.p, *zo = w.z2_32.p;  // the V-cycle's current output and the previous one
     MK_CHECK(blocks_for(len) <= kMaxParts, MK_ERR_ARG, "operator too large for the reduction buffer");
     spmv64(c, A, x, w.r.p, b, SPMV_RESID_NORED, nullptr, nullptr);
     CgState* st = c->state.p;
     const unsigned gl = fgrid(len);
     hipLaunchKernelGGL(cgm_init, dim3(gl), dim3(256), 0, c->stream, len, (const double*)w.r.p, b, w.r32.p, w.p.p, w.q.p,
-                       w.z.p, c->partials.p);
+                       zo, c->partials.p);
     hipLaunchKernelGGL(cgm_init_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)c->partials.p, int(gl),
                        rel_tol * rel_tol);
     double* part = c->partials.p;
     // the V-cycle on r32 and the two dots beta needs, in its last kernel where that can; returns
     // their partials
-    auto precondition = [&] {
-        const unsigned np = mg_apply32_dots(c, mg, w.r32.p, w.z32.p, &st->done, w.r.p, w.z.p, part);
+    auto precondition = [&](float* z, const float* zold) {
+        const unsigned np = mg_apply32_dots(c, mg, w.r32.p, z, &st->done, w.r.p, zold, part);
         if (np) return np;
         hipLaunchKernelGGL(cgm_beta2, dim3(gl), dim3(256), 0, c->stream, len, (const double*)w.r.p,
-                           (const float*)w.z32.p, (const double*)w.z.p, (const CgState*)st, part);
+                           (const float*)z, zold, (const CgState*)st, part);
         return gl;
     };
-    const unsigned gb = precondition();
+    const unsigned gb = precondition(zc, zo);
     MK_HIP(hipGetLastError());
     unsigned gs = 0;
     const SellDev<double> D = sell_dev<double>(A, A->val64.p, A->block, &gs);
     const unsigned gsr = std::max(1u, std::min(gs, fin_grid()));
     const bool fold_b = gb <= kFoldParts && gsr <= kFoldParts;
     // one iteration: beta, p/q update with A z (fused), x/r update, V-cycle on the new residual
-    auto iteration = [&] {
+    auto iteration = [&](const float* z, float* zn) {
         if (!fold_b)
             hipLaunchKernelGGL(cgm_beta2_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gb));
         const int nin = fold_b ? int(gb) : 0;
@@ -1492,24 +1494,28 @@ CgResult cg64_mg32(mk_ctx* c, const mk_op* A, const double* b, double* x, double
             SpmvTimer tm(c, A->bytes64 + double(len) * (4.0 + 8.0 * 5.0), A, "cg_spmv", false);
             if (A->cplx)
                 MK_TLAUNCH(tm, 0, (cgm_spmv<true>), dim3(gsr), dim3(A->block), 0, c->stream, D,
-                           (const float*)w.z32.p, w.p.p, w.q.p, w.z.p, st, part, nin);
+                           z, w.p.p, w.q.p, st, part, nin);
             else
                 MK_TLAUNCH(tm, 0, (cgm_spmv<false>), dim3(gsr), dim3(A->block), 0, c->stream, D,
-                           (const float*)w.z32.p, w.p.p, w.q.p, w.z.p, st, part, nin);
+                           z, w.p.p, w.q.p, st, part, nin);
         }
         if (!fold_b)
             hipLaunchKernelGGL(cgm_spmv_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gsr));
         hipLaunchKernelGGL(cgm_update, dim3(gl), dim3(256), 0, c->stream, len, x, w.r.p, w.r32.p,
                            (const double*)w.p.p, (const double*)w.q.p, st, part, fold_b ? int(gsr) : 0);
         hipLaunchKernelGGL(cgm_update_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gl));
-        precondition();
+        precondition(zn, z);
     };
     return drive(c, hint, maxiter, check_every, [&](int batch) {
         run_batches(batch, check_every, [&](int m) {
             run_batch(c, A, mg, {uintptr_t(4), uintptr_t(A->val64.p), uintptr_t(x), uintptr_t(w.r.p),
-                                 uintptr_t(w.r32.p), uintptr_t(w.z32.p), uintptr_t(w.z.p), uintptr_t(w.p.p),
+                                 uintptr_t(w.r32.p), uintptr_t(zc), uintptr_t(zo), uintptr_t(w.p.p),
                                  uintptr_t(w.q.p)},
-                      m, [&](int k) { for (; k > 0; k--) iteration(); });
+                      m, [&](int k) {
+                          float *a = zc, *b2 = zo;
+                          for (; k > 0; k--, std::swap(a, b2)) iteration(a, b2);
+                      });
+            if (m & 1) std::swap(zc, zo);
         });
     }, true_residual(c, A, b, x));
 }

@@ -1061,7 +1061,7 @@ void chebyshev(mk_ctx* c, const Mg* g, MgLevel& L, const T* b, T* x, bool zero_s
 // a level that is one product or the dense inverse; returns their partials (0: not formed)
 template <typename T>
 unsigned vcycle(mk_ctx* c, Mg* g, int l, const T* b, T* x, const int* skip, const double* r_ = nullptr,
-                const double* xold = nullptr, double* partials = nullptr) {
+                const float* xold = nullptr, double* partials = nullptr) {
     MgLevel& L = g->lv[size_t(l)];
     if (l + 1 == int(g->lv.size())) {
         const unsigned np = g->coarse.apply<T>(c, b, x, skip, r_, xold, partials);
@@ -1340,7 +1340,7 @@ Mg* mg_build_complex(mk_ctx* c, int n, const int64_t* ptr, const int* col, const
 }
 void mg_apply64(mk_ctx* c, Mg* g, const double* b, double* x, const int* skip) { vcycle<double>(c, g, 0, b, x, skip); }
 void mg_apply32(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip) { vcycle<float>(c, g, 0, b, x, skip); }
-unsigned mg_apply32_dots(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip, const double* r, const double* xold,
+unsigned mg_apply32_dots(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip, const double* r, const float* xold,
                          double* partials) {
     return vcycle<float>(c, g, 0, b, x, skip, r, xold, partials);
 }

@@ -143,7 +143,7 @@ struct BatchPlanner {
 // per-context scratch vectors
 struct Work {
     DevBuf<double> r, z, p, p2, q, t;
-    DevBuf<float> r32, z32, p32, p2_32, q32, x32, d32;
+    DevBuf<float> r32, z32, z2_32, p32, p2_32, q32, x32, d32;
 };
 
 // batched (multi-right-hand-side) solves (block.hip): up to 64 columns, row-major blocks
@@ -171,7 +171,7 @@ struct DenseInverse {
     // x = A^-1 b; with r, also per-block partials of r.x and r.xold (rows 0 and 1, kMaxParts apart).
     // Returns the number of blocks.
     template <typename T>
-    unsigned apply(mk_ctx* c, const T* b, T* x, const int* skip, const double* r = nullptr, const double* xold = nullptr,
+    unsigned apply(mk_ctx* c, const T* b, T* x, const int* skip, const double* r = nullptr, const float* xold = nullptr,
                    double* partials = nullptr) const;
     template <typename T>
     void apply_block(mk_ctx* c, int mw, const T* B, T* X, const int* skip) const;  // n x mw row-major
@@ -194,7 +194,7 @@ void mg_apply64(mk_ctx* c, Mg* g, const double* b, double* x, const int* skip);
 void mg_apply32(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip);
 // mg_apply32 whose last kernel also leaves the per-block partials of r.x and r.xold (FP64 vectors, rows 0
 // and 1 of partials) where that kernel can: returns their number, 0 when the caller has to form them
-unsigned mg_apply32_dots(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip, const double* r, const double* xold,
+unsigned mg_apply32_dots(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip, const double* r, const float* xold,
                          double* partials);
 // V-cycle on an n x mw row-major block (T = float: FP32 values and vectors; double: FP64)
 template <typename T>
@@ -353,7 +353,7 @@ void cheb0_launch(mk_ctx* c, const mk_op* A, const T* b, T* x_out, T* d, T c0, T
 // per-block partials of r.y and r.yold in rows 0 and 1 of partials.  Returns the number of blocks.
 template <typename T>
 unsigned spmv2_launch(mk_ctx* c, const mk_op* A, int m1, const T* u, const T* v, T* y, const int* skip, const char* name,
-                      const double* r = nullptr, const double* yold = nullptr, double* partials = nullptr);
+                      const double* r = nullptr, const float* yold = nullptr, double* partials = nullptr);
 template <typename T>
 void copy_launch(mk_ctx* c, size_t len, const T* x, T* y, const int* skip);
 template <typename T>
