@@ -1491,7 +1491,7 @@ CgResult cg64_mg32(mk_ctx* c, const mk_op* A, const double* b, double* x, double
             hipLaunchKernelGGL(cgm_beta2_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gb));
         const int nin = fold_b ? int(gb) : 0;
         {
-            SpmvTimer tm(c, A->bytes64 + double(len) * (4.0 + 8.0 * 5.0), A, "cg_spmv", false);
+            SpmvTimer tm(c, A->bytes64 + double(len) * (4.0 + 8.0 * 4.0), A, "cg_spmv", false);
             if (A->cplx)
                 MK_TLAUNCH(tm, 0, (cgm_spmv<true>), dim3(gsr), dim3(A->block), 0, c->stream, D,
                            z, w.p.p, w.q.p, st, part, nin);
