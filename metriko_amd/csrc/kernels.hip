@@ -177,15 +177,21 @@ struct DirectionOperands {
     }
 };
 
-// nin: partials of rz (Jacobi: and rr) to fold (0: the state holds beta).  The iteration's rz goes to
-// st->rz_new, which no block of this launch reads; cg_step2 moves it to st->rz, which none of its
-// blocks reads.
+// nin: partials of rz (Jacobi: and rr) to fold (0: the state holds beta).
+//
+// No block of a launch reads a word that another block of it writes (a block that starts late would
+// see either value, each of its wavefronts for itself).  The iteration's rz goes to st->rz_new, and
+// cg_step2 moves it to st->rz; the end of the solve, found by a fold, is in the same way handed on
+// in st->stop, which cg_step2 tests and moves to st->done, the word all other kernels test.
 template <typename T, bool CPLX, bool JAC>
 __global__ void __launch_bounds__(256) cg_step1(SellDev<T> A, const T* __restrict__ z, const T* __restrict__ p,
                                               T* __restrict__ pn, T* __restrict__ q, CgState* st, double* partials, int nin) {
-    if (st->done) return;
     constexpr int W = CPLX ? 2 : 1;
     const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+    if (st->done) {
+        if (writer) st->stop = 1;
+        return;
+    }
     T beta;
     if (nin) {
         double tot[JAC ? 2 : 1];
@@ -200,11 +206,11 @@ __global__ void __launch_bounds__(256) cg_step1(SellDev<T> A, const T* __restric
                 st->rr = rr;
                 st->it += 1;
                 if (nan) st->status = MK_ERR_NAN;
-                if (stop) st->done = 1;
+                if (stop) st->stop = 1;
             }
         } else {
             stop = !(rz > 0.0);
-            if (writer && stop) { st->status = (rz == rz) ? MK_ERR_NOT_SPD : MK_ERR_NAN; st->done = 1; }
+            if (writer && stop) { st->status = (rz == rz) ? MK_ERR_NOT_SPD : MK_ERR_NAN; st->stop = 1; }
         }
         if (stop) return;
         beta = T(rz / st->rz);
@@ -236,8 +242,12 @@ template <typename T, bool CPLX, bool JAC>
 __global__ void __launch_bounds__(256) cg_step2(int n, T* __restrict__ x, T* __restrict__ r, T* __restrict__ z,
                                               const T* __restrict__ p, const T* __restrict__ q,
                                               const T* __restrict__ dinv, CgState* st, double* partials, int npq) {
-    if (st->done) return;
     constexpr int W = CPLX ? 2 : 1;
+    const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+    if (st->stop) {
+        if (writer) st->done = 1;
+        return;
+    }
     const double rz_new = st->rz_new;
     T alpha;
     if (npq) {
@@ -245,7 +255,7 @@ __global__ void __launch_bounds__(256) cg_step2(int n, T* __restrict__ x, T* __r
         partials_sum<1>(partials + kRowPq * kMaxParts, npq, tot);
         const double pq = tot[0];
         if (!(pq > 0.0)) {
-            if (blockIdx.x == 0 && threadIdx.x == 0) {
+            if (writer) {
                 st->status = (pq == pq) ? MK_ERR_NOT_SPD : MK_ERR_NAN;
                 st->done = 1;
             }
@@ -255,7 +265,7 @@ __global__ void __launch_bounds__(256) cg_step2(int n, T* __restrict__ x, T* __r
     } else {
         alpha = T(st->alpha);
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) st->rz = rz_new;
+    if (writer) st->rz = rz_new;
     double rz = 0.0, rr = 0.0;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const T d = JAC && dinv ? dinv[i] : T(1);
@@ -288,7 +298,7 @@ __global__ void __launch_bounds__(1024) cg_alpha_fin(CgState* st, const double* 
     double tot[1];
     partials_sum<1>(partials + kRowPq * kMaxParts, nparts, tot);
     if (threadIdx.x == 0) {
-        if (!(tot[0] > 0.0)) { st->status = (tot[0] == tot[0]) ? MK_ERR_NOT_SPD : MK_ERR_NAN; st->done = 1; }
+        if (!(tot[0] > 0.0)) { st->status = (tot[0] == tot[0]) ? MK_ERR_NOT_SPD : MK_ERR_NAN; st->done = st->stop = 1; }
         else st->alpha = st->rz_new / tot[0];
     }
 }
@@ -366,6 +376,7 @@ __global__ void __launch_bounds__(1024) cg_init_fin(CgState* st, const double* _
         st->tol2 = tol2;
         st->beta = 0.0;
         st->it = 0;
+        st->stop = 0;
         st->status = MK_OK;
         st->done = (tot[1] <= tol2 * tot[2]) ? 1 : 0;
         if (!(tot[0] == tot[0]) || !(tot[1] == tot[1])) { st->status = MK_ERR_NAN; st->done = 1; }
@@ -403,14 +414,17 @@ static constexpr int kRowUpd = 3;
 __global__ void __launch_bounds__(256) cgm_update(size_t len, double* __restrict__ x, double* __restrict__ r,
                                                 float* __restrict__ r32, const double* __restrict__ p,
                                                 const double* __restrict__ q, CgState* st, double* partials, int npq) {
-    const int done = st->done;
+    const int stop = st->stop;
     const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
     // the first element's loads are in flight while alpha is folded
     size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     const size_t stride = size_t(gridDim.x) * blockDim.x;
     double xi = 0.0, ri = 0.0, pi = 0.0, qi = 0.0;
     if (i < len) { xi = x[i]; ri = r[i]; pi = p[i]; qi = q[i]; }
-    if (done) return;
+    if (stop) {
+        if (writer) st->done = 1;
+        return;
+    }
     double alpha;
     if (npq) {
         const double rz_new = st->rz_new;
@@ -529,7 +543,11 @@ __global__ void __launch_bounds__(256) cgm_spmv(SellDev<double> A, const float* 
         CgmOperands<CPLX> o{z32, p, q};
         const bool own = spmv_row_gp<double, CPLX>(A, Fp32Gather<CPLX>{z32}, vb, row, a[0], a[1], o);
         if (!folded) {
-            if (done) return;
+            const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+            if (done) {
+                if (writer) st->stop = 1;
+                return;
+            }
             folded = true;
             if (nin) {  // a and m; rz_new is cgm_update's
                 double tot[2] = {pre[0][0] + pre[1][0], pre[0][1] + pre[1][1]};
@@ -538,9 +556,8 @@ __global__ void __launch_bounds__(256) cgm_spmv(SellDev<double> A, const float* 
                     tot[1] += partials[kMaxParts + i];
                 }
                 block_sum<2, 1>(tot);
-                const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
                 if (!(tot[0] > 0.0)) {
-                    if (writer) { st->status = (tot[0] == tot[0]) ? MK_ERR_NOT_SPD : MK_ERR_NAN; st->done = 1; }
+                    if (writer) { st->status = (tot[0] == tot[0]) ? MK_ERR_NOT_SPD : MK_ERR_NAN; st->stop = 1; }
                     return;
                 }
                 beta = first ? 0.0 : (tot[0] - tot[1]) / rz;
@@ -567,7 +584,7 @@ __global__ void __launch_bounds__(1024) cgm_spmv_fin(CgState* st, const double* 
         st->pq = tot[0];
         if (!(tot[0] > 0.0)) {
             st->status = (tot[0] == tot[0]) ? MK_ERR_NOT_SPD : MK_ERR_NAN;
-            st->done = 1;
+            st->done = st->stop = 1;
         } else {
             st->alpha = st->rz / tot[0];
         }
@@ -601,6 +618,7 @@ __global__ void __launch_bounds__(1024) cgm_init_fin(CgState* st, const double* 
         st->tol2 = tol2;
         st->rz = 1.0;
         st->it = 0;
+        st->stop = 0;
         st->first = 1;
         st->status = MK_OK;
         st->done = (tot[0] <= tol2 * tot[1]) ? 1 : 0;

@@ -86,6 +86,7 @@ struct CgState {
     double bb;      // ||b||^2 (reference norm)
     double tol2;    // convergence threshold on rr/bb
     int done;       // 1 = converged or failed
+    int stop;       // as done, from the iteration's first kernel to its second (see cg_step1)
     int status;     // MK_OK / MK_ERR_NOT_SPD / MK_ERR_NAN
     int it;         // iterations taken
     int first;      // 1 until the first beta of the fused FP32-multigrid iteration
