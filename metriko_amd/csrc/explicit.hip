@@ -334,14 +334,8 @@ bool explicit_level(mk_ctx* c, bool cplx, const HostCsr& hA, const HostCsr& hP, 
     b.fill(V, Mc.ptr.p, cT.p, n, Mc.col.p, Mc.val.p);
     const int64_t wz = int64_t(Wc.col.n);
     *W = b.op(nc, n, wz, std::move(Wc.ptr), std::move(Wc.col), std::move(Wc.val), block);
-    try {
-        *M = b.op(n, n + nc, nz, std::move(Mc.ptr), std::move(Mc.col), std::move(Mc.val), block);
-        MK_HIP(hipStreamSynchronize(c->stream));  // the temporaries are freed on return
-    } catch (...) {
-        delete *W;
-        *W = nullptr;
-        throw;
-    }
+    *M = b.op(n, n + nc, nz, std::move(Mc.ptr), std::move(Mc.col), std::move(Mc.val), block);
+    MK_HIP(hipStreamSynchronize(c->stream));  // the temporaries are freed on return
     return true;
 }
 

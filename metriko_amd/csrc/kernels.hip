@@ -702,6 +702,13 @@ __global__ void __launch_bounds__(256) k_sell_fill(int ns, int C, int n_rows, in
     }
 }
 
+void check_layout(int block, int C, int sigma) {
+    MK_CHECK(C > 0 && C % 64 == 0, MK_ERR_ARG, "slice height must be a positive multiple of 64");
+    // every SpMV kernel is compiled with __launch_bounds__(256)
+    MK_CHECK(block % 64 == 0 && block >= 64 && block <= 256, MK_ERR_ARG, "block_size must be 64, 128 or 256");
+    MK_CHECK(sigma >= 1, MK_ERR_ARG, "sigma must be >= 1");
+}
+
 void build_sell(mk_op* op, const int64_t* rowptr, const int32_t* col, const double* val, int C, int sigma, double scale,
                 const int* rsrc, const int* cmap) {
     const int n = op->n;
@@ -709,11 +716,7 @@ void build_sell(mk_op* op, const int64_t* rowptr, const int32_t* col, const doub
     auto src = [rsrc](int i) { return rsrc ? rsrc[i] : i; };
     auto cm = [cmap](int c) { return cmap ? cmap[c] : c; };
     const int vw = op->cplx ? 2 : 1;
-    MK_CHECK(C > 0 && C % 64 == 0, MK_ERR_ARG, "slice height must be a positive multiple of 64");
-    // every SpMV kernel is compiled with __launch_bounds__(256)
-    MK_CHECK(op->block % 64 == 0 && op->block >= 64 && op->block <= 256, MK_ERR_ARG,
-             "block_size must be 64, 128 or 256");
-    MK_CHECK(sigma >= 1, MK_ERR_ARG, "sigma must be >= 1");
+    check_layout(op->block, C, sigma);
     const auto t_start = std::chrono::steady_clock::now();
     auto lap_ms = [&] {
         return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_start).count();

@@ -859,6 +859,8 @@ HostHier<T> build_host(Csr<T> A, double theta, int finest_max, int coarse_max, b
 template <typename T>
 Mg* build_impl(mk_ctx* c, Csr<T>&& A0, const mk_solve_opts& o, double theta, int coarse_max, int finest_ordered,
                const std::vector<T>* nullvec = nullptr, int nnull = 0, std::vector<int>* order_out = nullptr) {
+    // the dense inverse and the explicit levels do not pass build_sell, which checks these too
+    check_layout(o.block_size, o.slice_height, o.format == MK_FMT_CSR ? 1 : o.sigma);
     HostHier<T> H = build_host<T>(std::move(A0), theta, order_out ? finest_ordered : coarse_max, coarse_max, false, nullvec,
                                   nnull);
     const auto t_up = std::chrono::steady_clock::now();
@@ -884,7 +886,7 @@ Mg* build_impl(mk_ctx* c, Csr<T>&& A0, const mk_solve_opts& o, double theta, int
         g->cplx = !std::is_same<T, double>::value;
         g->deg = tune().deg;
         for (size_t l = 0; l < H.A.size(); l++) {
-            MgLevel L;
+            MgLevel& L = g->lv.emplace_back();  // in the hierarchy before it is filled: freed with it on a throw
             L.n = H.A[l].nr;
             L.lmax = H.lmax[l];
             // the coarsest operator is only needed as its inverse
@@ -929,7 +931,6 @@ Mg* build_impl(mk_ctx* c, Csr<T>&& A0, const mk_solve_opts& o, double theta, int
                     L.RR = upload(c, H.RR[l], o, I_(l + 1), pos2.empty() ? nullptr : pos2.data());
                 }
             }
-            g->lv.push_back(std::move(L));
             if (verbose) std::fprintf(stderr, "[mg]   level %zu uploaded %.0f ms\n", l, since_up());
         }
         const Csr<T>& Ac = H.A.back();

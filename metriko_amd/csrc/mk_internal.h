@@ -181,7 +181,8 @@ struct DenseInverse {
 struct HostCsr { int rows; const int64_t* ptr; const int* col; const double* val; };
 // One multigrid level as two products, b_c = W b and x = M [b; x_c] (explicit.hip), for the smoother
 // q = alpha D^-1 - beta D^-1 A D^-1; dinv: the smoother's inverse diagonal.  false (nothing built): a
-// row of the products is too long, or M in FP32 takes more than max_bytes
+// row of the products is too long, or M in FP32 takes more than max_bytes.  What a throw leaves in W and M
+// is the caller's to delete.
 bool explicit_level(mk_ctx* c, bool cplx, const HostCsr& A, const HostCsr& P, const HostCsr& R, const double* dinv,
                     double alpha, double beta, double max_bytes, int block, mk_op** W, mk_op** M);
 // multigrid (mg.hip)
@@ -375,6 +376,8 @@ BlockResult block_pcg(mk_ctx* c, const mk_op* A, Mg* mg, int mw, const double* B
 // values are multiplied by scale on upload.  Renumbered operator (host arrays, either may be
 // null): stored row i is CSR row rsrc[i] and CSR column c is stored as cmap[c]; each row keeps
 // its entries in CSR order, so products sum in the same order as the unrenumbered operator.
+// Throws MK_ERR_ARG unless build_sell takes this block size, slice height and sorting window.
+void check_layout(int block, int C, int sigma);
 void build_sell(mk_op* op, const int64_t* rowptr, const int32_t* col, const double* val, int C, int sigma,
                 double scale = 1.0, const int* rsrc = nullptr, const int* cmap = nullptr);
 // y = A x (mode PLAIN); y = A x and partial x^H y (DOT); y = b - A x and partial |y|^2 (RESID)
