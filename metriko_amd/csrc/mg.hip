@@ -131,6 +131,40 @@ Csr<T> conj_transpose(const Csr<T>& A) {
     return t;
 }
 
+// Entries of a row that name the same column are summed into the first of them (a caller's operator may
+// hold such rows; the dense inverse stores and the explicit products add one entry per column at a time).
+// Rows in ascending order, the usual case, cost one pass over the columns.
+template <typename T>
+void sum_duplicates(Csr<T>& A) {
+    std::atomic<int> unsorted{0};
+#pragma omp parallel for schedule(static, 4096) if (A.nr > 100000)
+    for (int i = 0; i < A.nr; i++) {
+        bool ascending = true;
+        for (int64_t k = A.ptr[i] + 1; k < A.ptr[i + 1]; k++) ascending = ascending && A.col[k - 1] < A.col[k];
+        if (!ascending) unsorted.store(1, std::memory_order_relaxed);
+    }
+    if (!unsorted.load()) return;
+    std::vector<int64_t> at(size_t(A.nc), -1);  // the column's entry in the row being built
+    int64_t w = 0, b = 0;
+    for (int i = 0; i < A.nr; i++) {
+        const int64_t e = A.ptr[size_t(i) + 1], row = w;
+        for (int64_t k = b; k < e; k++) {
+            const int c = A.col[size_t(k)];
+            if (at[size_t(c)] >= row) {
+                A.val[size_t(at[size_t(c)])] += A.val[size_t(k)];
+            } else {
+                at[size_t(c)] = w;
+                A.col[size_t(w)] = c;
+                A.val[size_t(w++)] = A.val[size_t(k)];
+            }
+        }
+        b = e;
+        A.ptr[size_t(i) + 1] = w;
+    }
+    A.col.resize(size_t(w));
+    A.val.resize(size_t(w));
+}
+
 template <typename T>
 std::vector<double> diag_of(const Csr<T>& A) {
     std::vector<double> d(size_t(A.nr), 0.0);
@@ -645,6 +679,7 @@ HostHier<T> build_host(Csr<T> A, double theta, int finest_max, int coarse_max, b
                        const std::vector<T>* B0 = nullptr, int nb = 0) {
     HostHier<T> H;
     const bool cplx = !std::is_same<T, double>::value;
+    sum_duplicates(A);
     std::vector<T> B;
     if (B0 && nb > 0) {
         if (B0->size() != size_t(A.nr) * size_t(nb)) throw Error(MK_ERR_ARG, "multigrid: near-null block size mismatch");
