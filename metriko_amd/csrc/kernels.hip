@@ -519,50 +519,58 @@ struct CgmOperands {
         }
     }
 };
-template <bool CPLX>
+// FOLD: nin partials of a and m to fold, under the first row's loads; otherwise the state holds beta, a
+// launch past the end returns before it loads a row, and nothing of the fold is in the row loop: 78
+// VGPRs and 6 wavefronts per SIMD (complex; 68 and 7 real) against 87 and 5 (75 and 6), 39.2 us on
+// 1,310,720 complex rows of 4 against 45.8 with one kernel for both.
+template <bool CPLX, bool FOLD>
 __global__ void __launch_bounds__(256) cgm_spmv(SellDev<double> A, const float* __restrict__ z32, double* p, double* q,
                                               CgState* st, double* partials, int nin) {
-    // the state and the first partials are loaded ahead of the row, used behind it
     const int done = st->done;
-    constexpr int W = CPLX ? 2 : 1;
-    double beta = st->beta;
-    const double rz = st->rz;
-    const int first = st->first;
-    double pre[2][2];
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-        const int i = threadIdx.x + u * blockDim.x;
-#pragma unroll
-        for (int k = 0; k < 2; k++) pre[u][k] = i < nin ? partials[k * kMaxParts + i] : 0.0;
+    const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+    if (!FOLD && done) {
+        if (writer) st->stop = 1;
+        return;
     }
-    bool folded = false;
+    constexpr int W = CPLX ? 2 : 1;
+    double beta = FOLD ? 0.0 : st->beta;
+    // the state and the first partials are loaded ahead of the row, used behind it
+    const double rz = FOLD ? st->rz : 0.0;
+    const int first = FOLD ? st->first : 0;
+    double pre[2][2];
+    if constexpr (FOLD) {
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int i = threadIdx.x + u * blockDim.x;
+#pragma unroll
+            for (int k = 0; k < 2; k++) pre[u][k] = i < nin ? partials[k * kMaxParts + i] : 0.0;
+        }
+    }
+    bool folded = !FOLD;
     double contrib = 0.0;
     for (int vb = blockIdx.x; vb < A.nvb; vb += gridDim.x) {
         int row = 0;
         double a[2];
         CgmOperands<CPLX> o{z32, p, q};
         const bool own = spmv_row_gp<double, CPLX>(A, Fp32Gather<CPLX>{z32}, vb, row, a[0], a[1], o);
-        if (!folded) {
-            const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+        if (FOLD && !folded) {
             if (done) {
                 if (writer) st->stop = 1;
                 return;
             }
             folded = true;
-            if (nin) {  // a and m; rz_new is cgm_update's
-                double tot[2] = {pre[0][0] + pre[1][0], pre[0][1] + pre[1][1]};
-                for (int i = threadIdx.x + 2 * blockDim.x; i < nin; i += blockDim.x) {
-                    tot[0] += partials[i];
-                    tot[1] += partials[kMaxParts + i];
-                }
-                block_sum<2, 1>(tot);
-                if (!(tot[0] > 0.0)) {
-                    if (writer) { st->status = (tot[0] == tot[0]) ? MK_ERR_NOT_SPD : MK_ERR_NAN; st->stop = 1; }
-                    return;
-                }
-                beta = first ? 0.0 : (tot[0] - tot[1]) / rz;
-                if (writer) st->rz_new = tot[0];
+            double tot[2] = {pre[0][0] + pre[1][0], pre[0][1] + pre[1][1]};
+            for (int i = threadIdx.x + 2 * blockDim.x; i < nin; i += blockDim.x) {
+                tot[0] += partials[i];
+                tot[1] += partials[kMaxParts + i];
             }
+            block_sum<2, 1>(tot);
+            if (!(tot[0] > 0.0)) {
+                if (writer) { st->status = (tot[0] == tot[0]) ? MK_ERR_NOT_SPD : MK_ERR_NAN; st->stop = 1; }
+                return;
+            }
+            beta = first ? 0.0 : (tot[0] - tot[1]) / rz;
+            if (writer) st->rz_new = tot[0];  // moved to rz by cgm_update
         }
         if (!own) continue;
 #pragma unroll
@@ -1513,12 +1521,11 @@ CgResult cg64_mg32(mk_ctx* c, const mk_op* A, const double* b, double* x, double
         const int nin = fold_b ? int(gb) : 0;
         {
             SpmvTimer tm(c, A->bytes64 + double(len) * (4.0 + 8.0 * 4.0), A, "cg_spmv", false);
-            if (A->cplx)
-                MK_TLAUNCH(tm, 0, (cgm_spmv<true>), dim3(gsr), dim3(A->block), 0, c->stream, D,
-                           z, w.p.p, w.q.p, st, part, nin);
-            else
-                MK_TLAUNCH(tm, 0, (cgm_spmv<false>), dim3(gsr), dim3(A->block), 0, c->stream, D,
-                           z, w.p.p, w.q.p, st, part, nin);
+#define MK_CGM(CP, FOLD) \
+    MK_TLAUNCH(tm, 0, (cgm_spmv<CP, FOLD>), dim3(gsr), dim3(A->block), 0, c->stream, D, z, w.p.p, w.q.p, st, part, nin)
+            if (A->cplx) { if (fold_b) MK_CGM(true, true); else MK_CGM(true, false); }
+            else { if (fold_b) MK_CGM(false, true); else MK_CGM(false, false); }
+#undef MK_CGM
         }
         if (!fold_b)
             hipLaunchKernelGGL(cgm_spmv_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gsr));

@@ -96,8 +96,9 @@ struct CgState {
 };
 
 // Iterations to launch before the next host convergence check.  Iterations launched past
-// convergence return at once, but each still costs its launches (about a third of a multigrid
-// PCG iteration on a large system, more than half on a small one), and every check costs a
+// convergence return at once (a product that folds scalars only after its first row's loads), but
+// each still costs its launches (about a third of a multigrid PCG iteration on a large system, more
+// than half on a small one), and every check costs a
 // round trip to the host of about 20 us.  The first batch takes as many iterations as the
 // operator's last solve needed (kFirst without one), at most the interval; after that the count is
 // predicted: the residual's geometric decrease per iteration since the previous check,
