@@ -80,3 +80,19 @@ def test_slice_heights(gpu_ctx, m, height):
     B = np.random.default_rng(height).standard_normal((A.shape[0], m))
     X, _ = gpu_ctx.op_real(A, o=mk.opts(slice_height=height)).solve_many(B)
     assert (np.linalg.norm(A @ X - B, axis=0) / np.linalg.norm(B, axis=0)).max() <= 1e-10
+
+
+@pytest.mark.parametrize("m", [3, 40])
+@pytest.mark.parametrize("precision", [mk.PREC_FP64, mk.PREC_MIXED_MG])
+def test_true_residual_of_a_strongly_scaled_operator(gpu_ctx, m, precision):
+    """The block recurrence carries A P along (q = A z + beta q) and reports its own residual, driven to half
+    the target.  Rows and columns scaled by 10^-2 to 10^2: the true residual, whose drift is of the order
+    of eps |A| |x| / |b| per iteration, still meets the target."""
+    nx = 90
+    T = sp.diags([-np.ones(nx - 1), 2.0 * np.ones(nx), -np.ones(nx - 1)], [-1, 0, 1])
+    rng = np.random.default_rng(m)
+    S = sp.diags(10.0 ** rng.uniform(-2.0, 2.0, nx * nx))
+    A = (S @ (sp.kron(T, sp.identity(nx)) + sp.kron(sp.identity(nx), T) + 1e-2 * sp.identity(nx * nx)) @ S).tocsr()
+    B = rng.standard_normal((A.shape[0], m))
+    X, st = gpu_ctx.op_real(A).solve_many(B, o=mk.opts(precision=precision))
+    assert (np.linalg.norm(A @ X - B, axis=0) <= 1e-10 * np.linalg.norm(B, axis=0)).all(), st

@@ -90,3 +90,49 @@ def test_long_rows_are_smoothed(gpu_ctx):
     b = rng.standard_normal(n)
     x, st = gpu_ctx.op_real(A).solve(b)
     assert st["mg_levels"] >= 2 and np.linalg.norm(A @ x - b) <= 1e-10 * np.linalg.norm(b)
+
+
+def _random_couplings(n, row):
+    S = sp.random(n, n, density=row / (2.0 * n), random_state=3, format="csr")
+    S = -(S + S.T)
+    S.setdiag(0)
+    return (S + sp.diags(-1.02 * np.asarray(S.sum(axis=1)).ravel() + 1e-2)).tocsr()
+
+
+def _hub(nx, ny):
+    A = _operator("five", nx, ny, np.random.default_rng(5)).tolil()
+    for j in np.random.default_rng(5).choice(np.arange(1, nx * ny), 900, replace=False):
+        A[0, j] = A[j, 0] = A[0, j] - 0.05
+        A[j, j] += 0.05
+    A[0, 0] += 0.05 * 900
+    return A.tocsr()
+
+
+def _thirteen(nx, ny):
+    K = sp.kron(_T(ny), sp.identity(nx)) + sp.kron(sp.identity(ny), _T(nx))
+    return (K @ K + 1e-2 * sp.identity(nx * ny)).tocsr()
+
+
+# M of the thirteen-point operator has 85 + 10 to 15 entries a row, 8 bytes each: 64 MiB are about 86,000 rows
+@pytest.mark.parametrize("what,explicit", [(("five", 49, 50), True), (("nine", 61, 43), True), (("hpd", 46, 47), True),
+                                           (("rows", 362, 362), True), (("rows", 363, 362), False),
+                                           (("bytes", 270, 270), True), (("bytes", 310, 310), False),
+                                           (("random", 3000, 40), False), (("random", 5000, 12), False),
+                                           (("hub", 60, 61), False)])
+def test_which_finest_levels_are_explicit(gpu_ctx, what, explicit):
+    """On both sides of every limit (131,072 rows, 64 MiB, 896 entries a row, long rows), by the kernels
+    that a first PCG step runs on the finest level."""
+    kind, p, q = what
+    A = (_random_couplings(p, q) if kind == "random" else _hub(p, q) if kind == "hub" else
+         _thirteen(p, q) if kind == "bytes" else _operator("five" if kind == "rows" else kind, p, q, np.random.default_rng(p)))
+    op = gpu_ctx.op_complex(A) if kind == "hpd" else gpu_ctx.op_real(A)
+    for precision, tag in ((mk.PREC_FP64, "fp64"), (mk.PREC_MIXED_MG, "fp32")):
+        try:
+            gpu_ctx.set_timing(True)
+            gpu_ctx.timing_report(reset=True)
+            _first_step(gpu_ctx, op, np.ones(A.shape[0]), mk.opts(precision=precision, maxiter=1))
+            keys = {k["key"] for k in gpu_ctx.timing_report(reset=True)}
+        finally:
+            gpu_ctx.set_timing(False)
+        assert (f"op_mg0_M:cheb_level:{tag}" in keys) == explicit, keys
+        assert any(k.startswith("op_mg0:cheb") and k.endswith(tag) for k in keys) != explicit, keys
