@@ -510,8 +510,8 @@ __global__ void __launch_bounds__(256) bk_init1_fin(BState* st, const double* __
 // bound by the passes over them and by the L2's gathers, so the product gathers the V-cycle's FP32
 // output (half the bytes of P) and the row's own P, Q and X pass once, loaded with its columns.  At
 // 302,102 rows x 64 the product with P, P.Q, the update of P and that of X in bk_update took 340 us
-// an iteration, this 227 to 250 (4.0 to 4.4 TB/s; a large copy reaches 5.1).  Finished columns keep P and Q; their last step still reaches X (their alpha
-// is 0 from the next bk_alpha_fin on).
+// an iteration, this 227 to 250 (4.0 to 4.4 TB/s; a large copy reaches 5.1).  Finished columns keep P
+// and Q; their last step still reaches X (their alpha is 0 from the next bk_alpha_fin on).
 // PART 1: the SELL rows, a wavefront's R at a time; 2: medium rows, a wavefront each, and the
 // segments' partial sums of the long rows; 3: the long rows.  Grid-stride over nw wavefronts' worth of
 // work; the launches leave their partials behind one another (block + pbase).
@@ -762,7 +762,9 @@ static BlockResult block_pcg_mw(mk_ctx* c, const mk_op* A, Mg* mg, const double*
     const unsigned g = unsigned(std::min<size_t>(std::min<size_t>(size_t(fin_grid()), size_t(kBlkParts)),
                                                  std::max<size_t>(1, (len + 255) / 256)));
     const int ng = int(g);
-    // the recurrence residual is driven to half the target so the true residual meets it
+    // The recurrence residual is driven to half the target and not compared with B - A X: forming Q by its
+    // recurrence leaves the same true residual as a product with P would, 5e-11 for a target of 1e-10 on
+    // operators scaled by 10^-2 to 10^2; scaled by 10^-4 to 10^4 (condition 1e16) both end at 1e-8.
     hipLaunchKernelGGL(k_set_bstate, dim3(1), dim3(1), 0, c->stream, st.p, 0.25 * rel_tol * rel_tol);
     hipLaunchKernelGGL((bk_init0<MW, ZT>), dim3(g), dim3(256), 0, c->stream, len, B, X, R.p, rz, part.p);
     hipLaunchKernelGGL((bk_init0_fin<MW>), dim3(MW), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);

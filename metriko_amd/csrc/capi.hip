@@ -146,7 +146,7 @@ __global__ void k_window_dots(int n, int nw, const double* __restrict__ W, const
         for (int k = 0; k < kWinDots; k++) part[size_t(blockIdx.x) * kWinDots + k] = acc[k];
 }
 // Fixed-order sum of the per-block partials: one wavefront per value, lane l adds the
-// partials l, l + 64, ... and the wavefront's fixed shuffle tree combines the lanes.
+// partials l, l + 64, ... and the wavefront's fixed DPP tree combines the lanes.
 __global__ void __launch_bounds__(64 * kWinDots) k_window_sum(int nparts, const double* __restrict__ part,
                                                                double* __restrict__ out) {
     const int k = threadIdx.x >> 6, lane = threadIdx.x & 63;

@@ -360,11 +360,13 @@ template <typename T>
 unsigned DenseInverse::apply(mk_ctx* c, const T* b, T* x, const int* skip, const double* r, const float* xold,
                              double* partials) const {
     const unsigned g = unsigned((n + 3) / 4);
-#define MK_GEMV(CP, DOTS)                                                                                               \
-    hipLaunchKernelGGL((k_dense_gemv<T, CP, DOTS>), dim3(g), dim3(256), 0, c->stream, n, ld, (const double*)inv.p, b, x, skip, \
-                       r, xold, partials)
-    if (cplx) { if (r) MK_GEMV(true, true); else MK_GEMV(true, false); }
-    else { if (r) MK_GEMV(false, true); else MK_GEMV(false, false); }
+#define MK_GEMV(CP, DOTS)                                                                                              \
+    hipLaunchKernelGGL((k_dense_gemv<T, CP, DOTS>), dim3(g), dim3(256), 0, c->stream, n, ld, (const double*)inv.p, b, \
+                       x, skip, r, xold, partials)
+    constexpr bool dots = std::is_same<T, float>::value;  // only the FP32 V-cycle is asked for them
+    MK_CHECK(dots || !r, MK_ERR_UNSUPPORTED, "dense product: dots in FP32 only");
+    if (cplx) { if (r) MK_GEMV(true, dots); else MK_GEMV(true, false); }
+    else { if (r) MK_GEMV(false, dots); else MK_GEMV(false, false); }
 #undef MK_GEMV
     return g;
 }

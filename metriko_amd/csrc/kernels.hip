@@ -5,10 +5,9 @@
 // a wavefront is one contiguous, coalesced 64-lane access.  Rows may be sorted by
 // length inside windows of sigma rows (perm maps a stored row to the original row).
 //
-// Reductions are deterministic: each block reduces with xor-butterfly shuffles
-// (DPP on CDNA) and LDS and writes one partial per block; the kernel that needs the total, or a
-// one-block kernel in between, sums the partials in a fixed order.  Reruns are therefore
-// bit-identical.
+// Reductions are deterministic: each block reduces with DPP row shifts and broadcasts inside its
+// wavefronts and LDS between them and writes one partial; the kernel that needs the total, or a one-block
+// kernel in between, sums the partials in a fixed order.  Reruns are therefore bit-identical.
 #include <algorithm>
 #include <chrono>
 #include <memory>
@@ -1197,9 +1196,13 @@ unsigned spmv2_launch(mk_ctx* c, const mk_op* A, int m1, const T* u, const T* v,
     const SellDev<T> D = sell_dev<T>(A, val, A->block, &g);
     MK_CHECK(!r || g <= kMaxParts, MK_ERR_ARG, "operator too large for the reduction buffer");
     SpmvTimer tm(c, sizeof(T) == 8 ? A->bytes64 : A->bytes32, A, name, sizeof(T) == 4);
-#define MK_SPMV2(CP, DOTS)                                                                                                 MK_TLAUNCH(tm, 0, (sell_spmv2<T, CP, DOTS>), dim3(g), dim3(A->block), 0, c->stream, D, m1, u, v, y, skip, r, yold, partials)
-    if (A->cplx) { if (r) MK_SPMV2(true, true); else MK_SPMV2(true, false); }
-    else { if (r) MK_SPMV2(false, true); else MK_SPMV2(false, false); }
+#define MK_SPMV2(CP, DOTS)                                                                                        \
+    MK_TLAUNCH(tm, 0, (sell_spmv2<T, CP, DOTS>), dim3(g), dim3(A->block), 0, c->stream, D, m1, u, v, y, skip, r, \
+               yold, partials)
+    constexpr bool dots = std::is_same<T, float>::value;  // only the FP32 V-cycle is asked for them
+    MK_CHECK(dots || !r, MK_ERR_UNSUPPORTED, "two-source product: dots in FP32 only");
+    if (A->cplx) { if (r) MK_SPMV2(true, dots); else MK_SPMV2(true, false); }
+    else { if (r) MK_SPMV2(false, dots); else MK_SPMV2(false, false); }
 #undef MK_SPMV2
     MK_HIP(hipGetLastError());
     return g;
@@ -1408,14 +1411,18 @@ static CgResult cg_run(mk_ctx* c, const mk_op* A, const T* val, const T* dinv, c
             const int nin = fold && k ? int(gn) : 0;
             {
                 SpmvTimer tm(c, bytes, A, "cg_spmv", sizeof(T) == 4);
-#define MK_STEP1(CP, JAC)                                                                                                    MK_TLAUNCH(tm, 0, (cg_step1<T, CP, JAC>), dim3(gr), dim3(A->block), 0, c->stream, D, (const T*)z, (const T*)pa, pb, q, st,                part, nin)
+#define MK_STEP1(CP, JAC)                                                                                               \
+    MK_TLAUNCH(tm, 0, (cg_step1<T, CP, JAC>), dim3(gr), dim3(A->block), 0, c->stream, D, (const T*)z, (const T*)pa, pb, \
+               q, st, part, nin)
                 if (A->cplx) { if (mg) MK_STEP1(true, false); else MK_STEP1(true, true); }
                 else { if (mg) MK_STEP1(false, false); else MK_STEP1(false, true); }
 #undef MK_STEP1
             }
             if (!fold) hipLaunchKernelGGL(cg_alpha_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gr));
             const int npq = fold ? int(gr) : 0;
-#define MK_STEP2(CP, JAC)                                                                                                hipLaunchKernelGGL((cg_step2<T, CP, JAC>), dim3(gn), dim3(256), 0, c->stream, n, x, r, z, (const T*)pb, (const T*)q,                        dinv, st, part, npq)
+#define MK_STEP2(CP, JAC)                                                                                       \
+    hipLaunchKernelGGL((cg_step2<T, CP, JAC>), dim3(gn), dim3(256), 0, c->stream, n, x, r, z, (const T*)pb, \
+                       (const T*)q, dinv, st, part, npq)
             if (A->cplx) { if (mg) MK_STEP2(true, false); else MK_STEP2(true, true); }
             else { if (mg) MK_STEP2(false, false); else MK_STEP2(false, true); }
 #undef MK_STEP2

@@ -1344,9 +1344,6 @@ extern "C" mk_status mk_mg_host_pcg(int n, const int64_t* ptr, const int32_t* co
     }
 }
 
-namespace {
-}  // namespace
-
 Mg* mg_build_real(mk_ctx* c, int n, const int64_t* ptr, const int* col, const double* val, const mk_solve_opts& o,
                   const std::vector<double>* nullvec, int nnull, std::vector<int>* order_out) {
     Csr<double> A(n, n);
