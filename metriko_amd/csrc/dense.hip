@@ -272,7 +272,8 @@ __global__ void __launch_bounds__(256) k_dense_gemv(int n, int ld, const double*
 // one of the K splits per wavefront (4 column tiles x 4 splits at 64 columns, 1 x 16 at 16 and 8),
 // on the FP64 matrix cores; the splits are added in order through LDS.  A lane reads the
 // neighbours k, k + 1 of its row as 16 bytes and uses them in two products.  The one-thread-per-
-// entry loop this replaces took 65 us at n = 280 and 97 us at n = 400 with 64 columns.
+// entry loop this replaces took 65 us at n = 280 and 97 us at n = 400 with 64 columns; this takes 14.4 us
+// at n = 399 and 38 to 44 at n = 2,368 (45 MB; 148 blocks, so 108 of the 256 compute units are idle).
 template <typename T, int MW>
 __global__ void __launch_bounds__(1024) k_dense_block(int n, int ld, const double* __restrict__ inv,
                                                       const T* __restrict__ B, T* __restrict__ X, const int* skip) {

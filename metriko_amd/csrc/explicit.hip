@@ -7,11 +7,11 @@
 // (a 40,820-face field: 4.0 -> 26.6 entries, its second level 11.7 -> 92.9), but a small level pays per
 // kernel, 3 to 6 us each whatever its size, and not per byte.
 //
-// Where the line lies (a solve with the level smoothed -> explicit): 4,900 rows of 5 0.96 -> 0.67 ms;
-// 62,307 complex rows of 5 and their 10,369 in FP64 1.50 -> 0.97 ms; a field of 40,820 faces 44 -> 26 ms;
-// 72,974 rows of 9 (33 MB) below 655,743 5.1 -> 4.85 ms; but 220,152 complex rows of 10.7 (240 MB)
-// below a 1,310,720-face field 447 -> 542 ms, so M is kept to what stays in the Infinity Cache beside
-// the solve's vectors.
+// Where the line lies (a solve with such levels smoothed -> explicit): 4,900 rows of 5 0.82 -> 0.52 ms;
+// 62,307 complex rows of 5 and their 10,369 in FP64 1.36 -> 0.89 ms; a field of 40,820 faces 42 -> 23 ms;
+// 72,974 rows of 9 (33 MB) and less below 655,743 5.7 -> 4.8 ms; but 220,152 complex rows of 10.7 (240 MB)
+// below a 1,310,720-face field 437 -> 538 ms, so M is kept to what stays in the Infinity Cache beside
+// the solve's vectors.  (20,567 x 37 columns use the smoother either way.)
 //
 // The products are row-wise SpGEMMs, one wavefront per row with a hash table of the row in LDS: the
 // entries of the left row are taken in order, the lanes spread over the right row (whose columns are

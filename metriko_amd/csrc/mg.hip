@@ -885,12 +885,14 @@ HostHier<T> build_host(Csr<T> A, double theta, int finest_max, int coarse_max, b
 // coarse_max: a level of at most this many unknowns is solved by its dense inverse (DenseInverse)
 // instead of being smoothed and coarsened further, the finest level too (then the hierarchy is that
 // inverse), unless an order is asked for: a one-level hierarchy has none, so the finest level is
-// then taken only up to finest_ordered.  Where the line lies: on small levels a smoothing or transfer
-// kernel takes 4 to 5 us whatever its size, six of them per level and cycle; the inverse's product
-// takes 2.3 us at 1,584 complex unknowns, 4.8 us at 1,498 below a 40,820-face field (its levels of
-// 1,498 and 174 took 29 us) and 18.5 us at 2,059 (68 MB, read from HBM; its levels of 2,059 and 216
-// took 30 us); real: 46 MB at 2,400.  At 4,000 real unknowns a solve of 301,702 x 64 columns became
-// slower (46.0 -> 57.7 ms).
+// then taken only up to finest_ordered.  Where the line lies: a level costs two or six launches of 4 to
+// 6 us a cycle whatever its size, its inverse one that reads 8 n^2 bytes (16 complex).  Complex limits of
+// 1,200, 1,600, 2,100 and 3,000: a field on 1,584 faces 12.2, 5.7, 5.8 and 5.8 ms, one on 40,820 (level of
+// 1,498) 30.8, 23.5, 23.5 and 23.3, one on 1,310,720 (level of 2,059: 68 MB, 19.8 us, against 15.3 for
+// its two products and the next level's inverse) 429, 431, 436 and 436.  Real limits of 1,200, 1,600,
+// 2,400, 3,200 and 4,000: sized uv and its gradient 4.9, 2.8, 2.7, 2.7 and 2.8 ms, 20,567 x 37 columns 4.7,
+// 5.5, 4.5, 4.6 and 5.0, 302,102 x 64 within 1.5 %.  Between 1,600 and 3,000 no size measured lost more
+// than it won.
 template <typename T>
 Mg* build_impl(mk_ctx* c, Csr<T>&& A0, const mk_solve_opts& o, double theta, int coarse_max, int finest_ordered,
                const std::vector<T>* nullvec = nullptr, int nnull = 0, std::vector<int>* order_out = nullptr) {
