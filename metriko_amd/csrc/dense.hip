@@ -52,11 +52,11 @@ __global__ void __launch_bounds__(256) k_dense_fill(int n, int ld, const int64_t
 
 // Step k0 of the elimination, one block per kTile columns: D = A_kk^-1 (formed by every block for
 // itself), the pivot rows R = D A_k,: (R_kk = D) and a copy C of the pivot columns.  Pivots up to `null`
-// times their diagonal count as zero.
+// times their diagonal count as zero; *small is set where one above that is at most `low` times it.
 template <bool CPLX>
-__global__ void __launch_bounds__(256) k_gj_panel(int ld, int k0, double null, const double* __restrict__ A,
+__global__ void __launch_bounds__(256) k_gj_panel(int ld, int k0, double null, double low, const double* __restrict__ A,
                                                   const double* __restrict__ diag, double* __restrict__ R,
-                                                  double* __restrict__ C) {
+                                                  double* __restrict__ C, int* __restrict__ small) {
     constexpr int W = CPLX ? 2 : 1;
     __shared__ double M[W][kNb][kNb + 1];
     __shared__ double T[W][kNb][kTile + 4];
@@ -93,6 +93,7 @@ __global__ void __launch_bounds__(256) k_gj_panel(int ld, int k0, double null, c
             // zero), which solves every consistent system of a singular operator.  A clearly negative
             // one (an indefinite operator): a tiny pivot, as the host's Cholesky takes.
             const double ip = piv > null * d ? 1.0 / piv : piv >= -null * d ? 0.0 : 1.0 / fmax(1e-300, d * 1e-14 + 1e-300);
+            if (blockIdx.x == 0 && t == 0 && piv > null * d && piv <= low * d) *small = 1;
             const double xr = rowp[buf][0][cj] * ip, xi = CPLX ? rowp[buf][W - 1][cj] * ip : 0.0;
 #pragma unroll
             for (int q = 0; q < kNb / 8; q++) {
@@ -330,7 +331,8 @@ __global__ void __launch_bounds__(1024) k_dense_block(int n, int ld, const doubl
 
 }  // namespace
 
-DenseInverse::DenseInverse(mk_ctx* c, bool cplx_, int n_, const int64_t* ptr, const int* col, const double* val)
+DenseInverse::DenseInverse(mk_ctx* c, bool cplx_, int n_, const int64_t* ptr, const int* col, const double* val,
+                           bool fp32_null)
     : n(n_), ld((n_ + kTile - 1) / kTile * kTile), cplx(cplx_) {
     const size_t w = cplx ? 2 : 1, nz = size_t(ptr[n]);
     DevBuf<int64_t> dp;
@@ -344,14 +346,16 @@ DenseInverse::DenseInverse(mk_ctx* c, bool cplx_, int n_, const int64_t* ptr, co
     // A pivot is its diagonal less squares that sum to at most it: n eps of it is rounding (measured 0.05
     // to 0.2 n eps on singular grids of 240 to 2,352 unknowns); a Galerkin operator's entries carry the
     // rounding of their own sums of tens of products.
-    const double null = 32.0 * double(n) * 0x1p-52;
+    const double low = double(n) * 0x1p-23, null = fp32_null ? low : 32.0 * double(n) * 0x1p-52;
+    DevBuf<int> small(1);
+    MK_HIP(hipMemsetAsync(small.p, 0, sizeof(int), c->stream));
     auto run = [&](auto cp) {
         constexpr bool CP = decltype(cp)::value;
         hipLaunchKernelGGL((k_dense_fill<CP>), dim3(unsigned(ld)), dim3(256), 0, c->stream, n, ld,
                            (const int64_t*)dp.p, (const int*)dc.p, (const double*)dv.p, inv.p, diag.p);
         for (int k0 = 0; k0 < n; k0 += kNb) {
-            hipLaunchKernelGGL((k_gj_panel<CP>), dim3(nt), dim3(256), 0, c->stream, ld, k0, null, (const double*)inv.p,
-                               (const double*)diag.p, R.p, C.p);
+            hipLaunchKernelGGL((k_gj_panel<CP>), dim3(nt), dim3(256), 0, c->stream, ld, k0, null, low, (const double*)inv.p,
+                               (const double*)diag.p, R.p, C.p, small.p);
             hipLaunchKernelGGL((k_gj_update<CP>), dim3(nt, nt), dim3(256), 0, c->stream, ld, k0, inv.p,
                                (const double*)R.p, (const double*)C.p);
         }
@@ -359,7 +363,9 @@ DenseInverse::DenseInverse(mk_ctx* c, bool cplx_, int n_, const int64_t* ptr, co
     if (cplx) run(std::true_type{});
     else run(std::false_type{});
     MK_HIP(hipGetLastError());
+    MK_HIP(hipMemcpyAsync(c->pin, small.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     MK_HIP(hipStreamSynchronize(c->stream));  // the temporaries are freed on return
+    near_null = *static_cast<const int*>(c->pin) != 0;
 }
 
 template <typename T>

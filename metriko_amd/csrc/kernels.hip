@@ -1270,8 +1270,12 @@ void add32to64_scaled(mk_ctx* c, size_t len, const float* d, const double* s_dev
 }
 
 // Generic PCG on the device.
-static inline void mg_apply(mk_ctx* c, Mg* g, const double* b, double* x, const int* skip) { mg_apply64(c, g, b, x, skip); }
-static inline void mg_apply(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip) { mg_apply32(c, g, b, x, skip); }
+static inline void mg_apply(mk_ctx* c, Mg* g, const double* b, double* x, const int* skip, bool) {
+    mg_apply64(c, g, b, x, skip);
+}
+static inline void mg_apply(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip, bool drop) {
+    mg_apply32(c, g, b, x, skip, drop);
+}
 
 // Runs body(batch) on the context stream: eagerly, or -- when graphs are on and timing is off -- by
 // replaying a hipGraph captured from the same call the first time this key is seen.  It must only launch kernels on
@@ -1376,7 +1380,7 @@ static CgResult drive(mk_ctx* c, int hint, int maxiter, int check_every, L&& lau
 // PCG on r (the initial residual); b for its norm.  resid as in drive().
 template <typename T, typename R>
 static CgResult cg_run(mk_ctx* c, const mk_op* A, const T* val, const T* dinv, const T* b, T* x, T* r, T* z, T* p, T* p2,
-                       T* q, double rel_tol, int hint, int maxiter, int check_every, double bytes, Mg* mg, R&& resid) {
+                       T* q, double rel_tol, int hint, int maxiter, int check_every, double bytes, Mg* mg, bool drop, R&& resid) {
     const int n = A->n;
     const size_t len = size_t(n) * (A->cplx ? 2 : 1);
     const unsigned g = blocks_for(n);
@@ -1384,7 +1388,7 @@ static CgResult cg_run(mk_ctx* c, const mk_op* A, const T* val, const T* dinv, c
     CgState* st = c->state.p;
     const unsigned gn = fgrid(size_t(n));
     if (mg) {
-        mg_apply(c, mg, r, z, nullptr);
+        mg_apply(c, mg, r, z, nullptr, drop);
         if (A->cplx)
             hipLaunchKernelGGL((cg_init_z<T, true>), dim3(gn), dim3(256), 0, c->stream, n, r, b, z, p, c->partials.p);
         else
@@ -1428,7 +1432,7 @@ static CgResult cg_run(mk_ctx* c, const mk_op* A, const T* val, const T* dinv, c
 #undef MK_STEP2
             if (mg) {
                 hipLaunchKernelGGL(cg_rr_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gn));
-                mg_apply(c, mg, r, z, &st->done);
+                mg_apply(c, mg, r, z, &st->done, drop);
                 if (A->cplx)
                     hipLaunchKernelGGL((cg_beta<T, true>), dim3(gn), dim3(256), 0, c->stream, n, r, z, (const CgState*)st,
                                        part);
@@ -1452,7 +1456,7 @@ static CgResult cg_run(mk_ctx* c, const mk_op* A, const T* val, const T* dinv, c
         }
         run_batches(batch, check_every, [&](int m) {
             run_batch(c, A, mg, {uintptr_t(sizeof(T)), uintptr_t(val), uintptr_t(x), uintptr_t(r), uintptr_t(z), uintptr_t(p),
-                                 uintptr_t(p2), uintptr_t(q)},
+                                 uintptr_t(p2), uintptr_t(q), uintptr_t(drop)},
                       m, [&](int k) { iterations(k, p, p2); });
             if (m & 1) std::swap(p, p2);
         });
@@ -1474,19 +1478,19 @@ CgResult cg64(mk_ctx* c, const mk_op* A, const double* b, double* x, double rel_
     w.r.ensure(len); w.z.ensure(len); w.p.ensure(len); w.p2.ensure(len); w.q.ensure(len);
     spmv64(c, A, x, w.r.p, b, SPMV_RESID_NORED, nullptr, nullptr);
     return cg_run<double>(c, A, A->val64.p, jacobi ? A->dinv64.p : nullptr, b, x, w.r.p, w.z.p, w.p.p, w.p2.p, w.q.p, rel_tol,
-                          hint, maxiter, check_every, A->bytes64, mg, true_residual(c, A, b, x));
+                          hint, maxiter, check_every, A->bytes64, mg, false, true_residual(c, A, b, x));
 }
 
-// x = A^-1 b from zero in FP32
+// x = A^-1 b from zero in FP32 (drop: see mg_drop_fp32_null)
 CgResult cg32(mk_ctx* c, const mk_op* A, const float* b, float* x, double rel_tol, int maxiter, bool jacobi,
-              int check_every, Mg* mg) {
+              int check_every, Mg* mg, bool drop) {
     Work& w = work(c);
     const size_t len = size_t(A->n) * (A->cplx ? 2 : 1);
     w.r32.ensure(len); w.z32.ensure(len); w.p32.ensure(len); w.p2_32.ensure(len); w.q32.ensure(len);
     MK_HIP(hipMemsetAsync(x, 0, len * sizeof(float), c->stream));
     MK_HIP(hipMemcpyAsync(w.r32.p, b, len * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
     return cg_run<float>(c, A, A->val32.p, jacobi ? A->dinv32.p : nullptr, b, x, w.r32.p, w.z32.p, w.p32.p, w.p2_32.p, w.q32.p,
-                         rel_tol, 0, maxiter, check_every, A->bytes32, mg, [] { return false; });
+                         rel_tol, 0, maxiter, check_every, A->bytes32, mg, drop, [] { return false; });
 }
 
 // FP64 flexible PCG whose multigrid V-cycle runs in FP32 (vectors converted at its ends).
@@ -1611,6 +1615,7 @@ SolveResult solve_spd(mk_ctx* c, const mk_op* A, const double* b, double* x, con
     }
     double prev = HUGE_VAL;
     int stagn = 0;
+    bool drop = false;
     // the FP32 work vectors used by cg32 are r32,z32,p32,q32; the normalised rhs lives in x32's twin
     DevBuf<float>& rhs32 = w.x32;
     DevBuf<float>& d32 = w.d32;
@@ -1630,7 +1635,14 @@ SolveResult solve_spd(mk_ctx* c, const mk_op* A, const double* b, double* x, con
         prev = rel;
         cvt64to32_scaled(c, len, w.t.p, rr, rhs32.p);
         const double itol = std::max(o.inner_tol, 0.5 * goal / rel);
-        CgResult cr = cg32(c, A, rhs32.p, d32.p, std::min(itol, 0.5), o.maxiter - res.iters, jac, o.check_every, mg);
+        CgResult cr = cg32(c, A, rhs32.p, d32.p, std::min(itol, 0.5), o.maxiter - res.iters, jac, o.check_every, mg, drop);
+        // An operator that is singular in FP32 breaks down along the direction that the hierarchy's coarsest
+        // inverse, formed in FP64, still resolves: the corrections go on without it.
+        if ((cr.status == MK_ERR_NOT_SPD || cr.status == MK_ERR_NAN) && mg && !drop && mg_drop_fp32_null(c, mg)) {
+            res.iters += cr.iters;
+            drop = true;
+            cr = cg32(c, A, rhs32.p, d32.p, std::min(itol, 0.5), o.maxiter - res.iters, jac, o.check_every, mg, drop);
+        }
         res.iters += cr.iters;
         res.refinements++;
         if (cr.status == MK_ERR_NOT_SPD || cr.status == MK_ERR_NAN) { res.status = cr.status; break; }

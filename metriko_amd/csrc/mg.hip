@@ -48,6 +48,11 @@ struct Mg {
     bool cplx = false;
     std::vector<MgLevel> lv;
     DenseInverse coarse;  // of the coarsest operator
+    // the same without its near-null directions, and the operator to form it from (coarse.near_null only)
+    DenseInverse coarse_drop;
+    std::vector<int64_t> cptr;
+    std::vector<int> ccol;
+    std::vector<double> cval;
     int deg = 2;
     double setup_ms = 0.0;
     int64_t nnz_total = 0;
@@ -973,6 +978,12 @@ Mg* build_impl(mk_ctx* c, Csr<T>&& A0, const mk_solve_opts& o, double theta, int
         const Csr<T>& Ac = H.A.back();
         g->coarse = DenseInverse(c, g->cplx, Ac.nr, Ac.ptr.data(), Ac.col.data(),
                                  reinterpret_cast<const double*>(Ac.val.data()));
+        if (g->coarse.near_null) {
+            const auto* v = reinterpret_cast<const double*>(Ac.val.data());
+            g->cptr.assign(Ac.ptr.begin(), Ac.ptr.end());
+            g->ccol.assign(Ac.col.begin(), Ac.col.end());
+            g->cval.assign(v, v + Ac.val.size() * (g->cplx ? 2 : 1));
+        }
         if (verbose) std::fprintf(stderr, "[mg]   coarsest inverse %.0f ms\n", since_up());
         // the finest level works on the caller's b and x, the coarsest needs no other vectors
         for (size_t l = 0; l < g->lv.size(); l++) {
@@ -1098,17 +1109,17 @@ void chebyshev(mk_ctx* c, const Mg* g, MgLevel& L, const T* b, T* x, bool zero_s
 // r, xold, partials (the finest level only): the dots of mg_apply32_dots, formed by the last kernel of
 // a level that is one product or the dense inverse; returns their partials (0: not formed)
 template <typename T>
-unsigned vcycle(mk_ctx* c, Mg* g, int l, const T* b, T* x, const int* skip, const double* r_ = nullptr,
-                const float* xold = nullptr, double* partials = nullptr) {
+unsigned vcycle(mk_ctx* c, Mg* g, int l, const T* b, T* x, const int* skip, const DenseInverse& coarse,
+                const double* r_ = nullptr, const float* xold = nullptr, double* partials = nullptr) {
     MgLevel& L = g->lv[size_t(l)];
     if (l + 1 == int(g->lv.size())) {
-        const unsigned np = g->coarse.apply<T>(c, b, x, skip, r_, xold, partials);
+        const unsigned np = coarse.apply<T>(c, b, x, skip, r_, xold, partials);
         return r_ ? np : 0;
     }
     MgLevel& Cn = g->lv[size_t(l) + 1];
     if (L.M) {
         spmv_launch<T>(c, L.W, Sel<T>::val(L.W), b, Sel<T>::b(Cn), nullptr, SPMV_PLAIN, nullptr, Sel<T>::bytes(L.W), skip);
-        vcycle<T>(c, g, l + 1, Sel<T>::b(Cn), Sel<T>::x(Cn), skip);
+        vcycle<T>(c, g, l + 1, Sel<T>::b(Cn), Sel<T>::x(Cn), skip, coarse);
         const unsigned np = spmv2_launch<T>(c, L.M, L.n, b, Sel<T>::x(Cn), x, skip, "cheb_level", r_, xold, partials);
         return r_ ? np : 0;
     }
@@ -1121,7 +1132,7 @@ unsigned vcycle(mk_ctx* c, Mg* g, int l, const T* b, T* x, const int* skip, cons
         spmv_launch<T>(c, L.R, Sel<T>::val(L.R), r, Sel<T>::b(Cn), nullptr, SPMV_PLAIN, nullptr, Sel<T>::bytes(L.R),
                        skip);
     }
-    vcycle<T>(c, g, l + 1, Sel<T>::b(Cn), Sel<T>::x(Cn), skip);
+    vcycle<T>(c, g, l + 1, Sel<T>::b(Cn), Sel<T>::x(Cn), skip, coarse);
     spmv_launch<T>(c, L.P, Sel<T>::val(L.P), Sel<T>::x(Cn), x, nullptr, SPMV_ACCUM, nullptr, Sel<T>::bytes(L.P), skip);
     chebyshev<T>(c, g, L, b, x, false, skip);
     return 0;
@@ -1373,11 +1384,18 @@ Mg* mg_build_complex(mk_ctx* c, int n, const int64_t* ptr, const int* col, const
     }
     return build_impl<cd>(c, std::move(A), o, tune().theta_cplx, tune().dense_cplx, tune().coarse_cplx);
 }
-void mg_apply64(mk_ctx* c, Mg* g, const double* b, double* x, const int* skip) { vcycle<double>(c, g, 0, b, x, skip); }
-void mg_apply32(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip) { vcycle<float>(c, g, 0, b, x, skip); }
+void mg_apply64(mk_ctx* c, Mg* g, const double* b, double* x, const int* skip) { vcycle<double>(c, g, 0, b, x, skip, g->coarse); }
+void mg_apply32(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip, bool drop) {
+    vcycle<float>(c, g, 0, b, x, skip, drop ? g->coarse_drop : g->coarse);
+}
+bool mg_drop_fp32_null(mk_ctx* c, Mg* g) {
+    if (g->coarse.near_null && g->coarse_drop.n == 0)
+        g->coarse_drop = DenseInverse(c, g->cplx, g->coarse.n, g->cptr.data(), g->ccol.data(), g->cval.data(), true);
+    return g->coarse.near_null;
+}
 unsigned mg_apply32_dots(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip, const double* r, const float* xold,
                          double* partials) {
-    return vcycle<float>(c, g, 0, b, x, skip, r, xold, partials);
+    return vcycle<float>(c, g, 0, b, x, skip, g->coarse, r, xold, partials);
 }
 template <typename T>
 void mg_apply_block(mk_ctx* c, Mg* g, int mw, const T* b, T* x, const int* skip) {

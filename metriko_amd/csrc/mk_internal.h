@@ -166,10 +166,14 @@ struct BlockResult {
 struct DenseInverse {
     int n = 0, ld = 0;
     bool cplx = false;
+    // A direction the inverse keeps is below FP32 rounding (a pivot of at most n 2^-23 of its diagonal)
+    bool near_null = false;
     DevBuf<double> inv;
     DenseInverse() = default;
-    // from CSR arrays on the host (complex: values interleaved)
-    DenseInverse(mk_ctx* c, bool cplx, int n, const int64_t* ptr, const int* col, const double* val);
+    // From CSR arrays on the host (complex: values interleaved).  Unknowns whose pivot is FP64 rounding are
+    // left out (fp32_null: those whose pivot is FP32 rounding).
+    DenseInverse(mk_ctx* c, bool cplx, int n, const int64_t* ptr, const int* col, const double* val,
+                 bool fp32_null = false);
     // x = A^-1 b; with r, also per-block partials of r.x and r.xold (rows 0 and 1, kMaxParts apart).
     // Returns the number of blocks.
     template <typename T>
@@ -194,7 +198,11 @@ Mg* mg_build_real(mk_ctx* c, int n, const int64_t* ptr, const int* col, const do
                   const std::vector<double>* nullvec = nullptr, int nnull = 0, std::vector<int>* order_out = nullptr);
 Mg* mg_build_complex(mk_ctx* c, int n, const int64_t* ptr, const int* col, const double* val, const mk_solve_opts& o);
 void mg_apply64(mk_ctx* c, Mg* g, const double* b, double* x, const int* skip);
-void mg_apply32(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip);
+// drop: with the coarsest inverse of mg_drop_fp32_null
+void mg_apply32(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip, bool drop);
+// The coarsest operator's inverse without the directions that FP32 vectors cannot hold (below n 2^-23 of
+// its diagonal), formed on the first call; false: there are none.
+bool mg_drop_fp32_null(mk_ctx* c, Mg* g);
 // mg_apply32 whose last kernel also leaves the per-block partials of r.x and r.xold (FP64 vectors, rows 0
 // and 1 of partials) where that kernel can: returns their number, 0 when the caller has to form them
 unsigned mg_apply32_dots(mk_ctx* c, Mg* g, const float* b, float* x, const int* skip, const double* r, const float* xold,

@@ -1,5 +1,6 @@
-"""Consistent systems of singular operators (a grid without boundary values): the dense inverse of the
-coarsest level leaves out the unknown whose pivot is rounding."""
+"""Consistent systems of singular and nearly singular operators (a grid without boundary values, shifted by up
+to 1e-12): the dense inverse of the coarsest level leaves out the unknown whose pivot is rounding, and an
+FP32 Krylov solve that breaks down goes on without the direction that only FP64 resolves."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -30,7 +31,7 @@ def _system(nx, ny, cplx, shift, parts=1):
 
 # one-level (dense), two-level with an explicit finest level, three levels
 @pytest.mark.parametrize("precision", [mk.PREC_FP64, mk.PREC_MIXED, mk.PREC_MIXED_MG])
-@pytest.mark.parametrize("shift", [0.0])
+@pytest.mark.parametrize("shift", [0.0, 1e-12])
 @pytest.mark.parametrize("cplx", [False, True])
 @pytest.mark.parametrize("nx,ny,parts", [(15, 16, 1), (30, 31, 1), (45, 44, 1), (20, 21, 4), (49, 50, 1), (60, 61, 1),
                                          (30, 31, 5), (95, 94, 1), (150, 151, 1)])
