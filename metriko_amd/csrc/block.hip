@@ -723,6 +723,8 @@ __global__ void k_set_bstate(BState* st, double tol2) {
     st->stepped = 0;
 }
 
+__global__ void k_tell_bstate(const BState* st, int* started) { tell_start(started, st->all_done); }
+
 // Launches bk_step; returns the number of partials it leaves per column.
 template <int MW, typename ZT>
 static int block_step(mk_ctx* c, const mk_op* A, const ZT* Z, double* P, double* Q, double* X, BState* st, double* part) {
@@ -772,6 +774,7 @@ static BlockResult block_pcg_mw(mk_ctx* c, const mk_op* A, Mg* mg, const double*
     hipLaunchKernelGGL((bk_init1<MW, ZT>), dim3(g), dim3(256), 0, c->stream, len, (const double*)R.p,
                        (const ZT*)zc, P.p, Q.p, part.p);
     hipLaunchKernelGGL((bk_init1_fin<MW>), dim3(MW), dim3(256), 0, c->stream, st.p, (const double*)part.p, ng);
+    hipLaunchKernelGGL(k_tell_bstate, dim3(1), dim3(1), 0, c->stream, (const BState*)st.p, arm_start(c));
     MK_HIP(hipGetLastError());
     static_assert(sizeof(BState) <= mk_ctx::kPinBytes, "BState does not fit the readback memory");
     const BState& h = *static_cast<const BState*>(c->pin);
@@ -784,6 +787,8 @@ static BlockResult block_pcg_mw(mk_ctx* c, const mk_op* A, Mg* mg, const double*
     for (;;) {
         const int batch = std::max(0, std::min(plan, maxiter - iters));
         for (int k = 0; k < batch; k++) {
+            // blocks whose columns all start converged (zeros) stop here
+            if (prev_iters < 0 && k == BatchPlanner::before_start(batch, false) && start_converged(c)) break;
             const int np = block_step<MW, ZT>(c, A, zc, P.p, Q.p, X, st.p, part.p);
             std::swap(zc, zo);
             hipLaunchKernelGGL((bk_alpha_fin<MW>), dim3(MW), dim3(256), 0, c->stream, st.p, (const double*)part.p, np);

@@ -468,7 +468,7 @@ mk_status mk_init(mk_ctx** out, int device) {
         c->partials.alloc(mk::kMaxParts * mk::kMaxK);
         c->state.alloc(1);
         c->scal.alloc(64);
-        MK_HIP(hipHostMalloc(&c->pin, mk_ctx::kPinBytes, hipHostMallocDefault));
+        MK_HIP(hipHostMalloc(&c->pin, mk_ctx::kPinBytes + 64, hipHostMallocDefault));
         MK_HIP(hipMemsetAsync(c->scal.p, 0, 64 * sizeof(double), c->stream));
         MK_HIP(hipStreamSynchronize(c->stream));
         const char* t = std::getenv("METRIKO_TIME_SPMV");

@@ -365,7 +365,7 @@ __global__ void __launch_bounds__(256) cg_init_z(int n, const T* __restrict__ r,
 // rz, rr, bb of the first residual -> the state of a new solve (z from an external preconditioner,
 // check_z, must make rz positive)
 __global__ void __launch_bounds__(1024) cg_init_fin(CgState* st, const double* __restrict__ partials, int nparts,
-                                                    double tol2, int check_z) {
+                                                    double tol2, int check_z, int* started) {
     double tot[3];
     partials_sum<3>(partials, nparts, tot);
     if (threadIdx.x == 0) {
@@ -380,6 +380,7 @@ __global__ void __launch_bounds__(1024) cg_init_fin(CgState* st, const double* _
         st->done = (tot[1] <= tol2 * tot[2]) ? 1 : 0;
         if (!(tot[0] == tot[0]) || !(tot[1] == tot[1])) { st->status = MK_ERR_NAN; st->done = 1; }
         if (check_z && !st->done && !(tot[0] > 0.0)) { st->status = MK_ERR_NOT_SPD; st->done = 1; }
+        tell_start(started, st->done);
     }
 }
 
@@ -616,7 +617,7 @@ __global__ void __launch_bounds__(256) cgm_init(size_t len, const double* __rest
     partials_write<2>(v, partials);
 }
 __global__ void __launch_bounds__(1024) cgm_init_fin(CgState* st, const double* __restrict__ partials, int nparts,
-                                                   double tol2) {
+                                                   double tol2, int* started) {
     double tot[2];
     partials_sum<2>(partials, nparts, tot);
     if (threadIdx.x == 0) {
@@ -630,6 +631,7 @@ __global__ void __launch_bounds__(1024) cgm_init_fin(CgState* st, const double* 
         st->status = MK_OK;
         st->done = (tot[0] <= tol2 * tot[1]) ? 1 : 0;
         if (!(tot[0] == tot[0])) { st->status = MK_ERR_NAN; st->done = 1; }
+        tell_start(started, st->done);
     }
 }
 
@@ -1355,13 +1357,19 @@ static void run_batches(int m, int interval, F&& batch) {
 // the true residual of x into the state behind a batch that is expected to be the last, so that a
 // solve that ends where its operator's last one did costs one round trip to the host.
 template <typename L, typename R>
-static CgResult drive(mk_ctx* c, int hint, int maxiter, int check_every, L&& launch, R&& resid) {
+static CgResult drive(mk_ctx* c, int hint, int maxiter, int check_every, bool captured, L&& launch, R&& resid) {
     BatchPlanner plan(c->time_spmv ? 1 : check_every);
     CgState* h = static_cast<CgState*>(c->pin);
     static_assert(sizeof(CgState) <= mk_ctx::kPinBytes, "CgState does not fit the readback memory");
     int launched = 0, batch = plan.first(hint);
     for (;;) {
         batch = std::min(batch, maxiter - launched);
+        if (launched == 0 && batch > 2) {
+            const int p = BatchPlanner::before_start(batch, captured);
+            launch(p);
+            launched += p;
+            batch = start_converged(c) ? 0 : batch - p;
+        }
         if (batch > 0) { launch(batch); launched += batch; }
         const bool checked = plan.last && !c->time_spmv && resid();
         MK_HIP(hipGetLastError());
@@ -1402,7 +1410,7 @@ static CgResult cg_run(mk_ctx* c, const mk_op* A, const T* val, const T* dinv, c
                                c->partials.p);
     }
     hipLaunchKernelGGL(cg_init_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)c->partials.p, int(gn),
-                       rel_tol * rel_tol, mg ? 1 : 0);
+                       rel_tol * rel_tol, mg ? 1 : 0, arm_start(c));
     MK_HIP(hipGetLastError());
     unsigned gs = 0;
     const SellDev<T> D = sell_dev<T>(A, val, A->block, &gs);
@@ -1448,7 +1456,7 @@ static CgResult cg_run(mk_ctx* c, const mk_op* A, const T* val, const T* dinv, c
             else hipLaunchKernelGGL((cg_beta_fin<true>), dim3(1), nt, 0, c->stream, st, (const double*)part, int(gn));
         }
     };
-    return drive(c, hint, maxiter, check_every, [&](int batch) {
+    return drive(c, hint, maxiter, check_every, mg != nullptr, [&](int batch) {
         if (!mg) {
             iterations(batch, p, p2);
             if (batch & 1) std::swap(p, p2);
@@ -1508,7 +1516,7 @@ CgResult cg64_mg32(mk_ctx* c, const mk_op* A, const double* b, double* x, double
     hipLaunchKernelGGL(cgm_init, dim3(gl), dim3(256), 0, c->stream, len, (const double*)w.r.p, b, w.r32.p, w.p.p, w.q.p,
                        zo, c->partials.p);
     hipLaunchKernelGGL(cgm_init_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)c->partials.p, int(gl),
-                       rel_tol * rel_tol);
+                       rel_tol * rel_tol, arm_start(c));
     double* part = c->partials.p;
     // the V-cycle on r32 and the two dots beta needs, in its last kernel where that can; returns
     // their partials
@@ -1545,7 +1553,7 @@ CgResult cg64_mg32(mk_ctx* c, const mk_op* A, const double* b, double* x, double
         hipLaunchKernelGGL(cgm_update_fin, dim3(1), dim3(1024), 0, c->stream, st, (const double*)part, int(gl));
         precondition(zn, z);
     };
-    return drive(c, hint, maxiter, check_every, [&](int batch) {
+    return drive(c, hint, maxiter, check_every, true, [&](int batch) {
         run_batches(batch, check_every, [&](int m) {
             run_batch(c, A, mg, {uintptr_t(4), uintptr_t(A->val64.p), uintptr_t(x), uintptr_t(w.r.p),
                                  uintptr_t(w.r32.p), uintptr_t(zc), uintptr_t(zo), uintptr_t(w.p.p),

@@ -100,14 +100,23 @@ struct CgState {
 // each still costs its launches (about a third of a multigrid PCG iteration on a large system, more
 // than half on a small one), and every check costs a
 // round trip to the host of about 20 us.  The first batch takes as many iterations as the
-// operator's last solve needed (kFirst without one), at most the interval; after that the count is
-// predicted: the residual's geometric decrease per iteration since the previous check,
+// operator's last solve needed (kFirst without one), at most the interval, most of them only once the
+// start's kernel has told the host that the start does not meet the tolerance (before_start: a solve
+// whose start does queued 10 iterations for nothing, 0.18 -> 0.26 ms at 22,500 unknowns; 0.15 now);
+// after that the count is predicted: the residual's geometric decrease per iteration since the previous check,
 // extrapolated to the target (rounded up).  While it says two intervals or more, half of it is
 // launched (up to kAhead intervals).  An iteration stops where it would stop with any batching, so
 // results do not depend on the prediction.  The solvers use interval 1 in kernel-timing mode, so
 // the per-kernel averages hold no launch past convergence.
 struct BatchPlanner {
     static constexpr int kFirst = 4, kAhead = 8;
+    // Iterations of a first batch of m that are queued before the host knows whether the start already meets
+    // the tolerance (then the others are not): two, or, of the power-of-two pieces of a captured batch, the
+    // smallest one (half of a single one).
+    static int before_start(int m, bool captured) {
+        const int p = m & -m;
+        return !captured || m <= 2 ? std::min(m, 2) : p == m ? m / 2 : p;
+    }
     int interval;
     int prev_it = -1;
     double prev_rr = 0.0;
@@ -250,6 +259,9 @@ struct mk_ctx {
     mk::DevBuf<double> scal;   // general device scalars
     void* pin = nullptr;       // page-locked host memory the solvers' states are read back into
     static constexpr size_t kPinBytes = 8192;
+    // behind it: whether the running solve's start meets the tolerance (-1: not known yet), which the
+    // kernel that finds out stores there
+    int* started() const { return reinterpret_cast<int*>(static_cast<char*>(pin) + kPinBytes); }
     // SpMV timing (events around each SpMV launch when enabled), attributed per
     // "operator label:kernel:precision" key
     bool time_spmv = false;

@@ -5,6 +5,7 @@
 #include <string>
 #include <hip/hip_ext.h>
 #include "mk_internal.h"
+#include <chrono>
 
 namespace mk {
 
@@ -90,6 +91,11 @@ __device__ __forceinline__ void partials_sum(const double* __restrict__ partials
         for (int k = 0; k < K; k++) tot[k] += partials[k * kMaxParts + i];
     }
     block_sum<K, 1>(tot);
+}
+
+// Tells the host whether the start meets the tolerance (mk_ctx::started: page-locked memory).
+__device__ __forceinline__ void tell_start(int* started, int done) {
+    __hip_atomic_store(started, done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The blocks of a launch go round-robin over the 8 XCDs, each with its own L2.  xcd_block maps
@@ -315,6 +321,23 @@ __device__ __forceinline__ bool spmv_row_g(const SellDev<T>& A, const G& g, int 
     return spmv_row_gp<T, CPLX>(A, g, vb, row, ar, ai, none);
 }
 
+
+// The word the start's kernel stores its finding in, not known yet (the stream is idle or has read the last
+// solve's: every solve ends with a readback).
+static inline int* arm_start(mk_ctx* c) {
+    __atomic_store_n(c->started(), -1, __ATOMIC_RELAXED);
+    return c->started();
+}
+// Whether the start meets the tolerance, waited for while the first iterations run; false also when that
+// takes longer than kStartWait.
+static inline bool start_converged(mk_ctx* c) {
+    constexpr auto kStartWait = std::chrono::microseconds(300);
+    const auto t0 = std::chrono::steady_clock::now();
+    int v;
+    while ((v = __atomic_load_n(c->started(), __ATOMIC_RELAXED)) < 0)
+        if (std::chrono::steady_clock::now() - t0 > kStartWait) return false;
+    return v != 0;
+}
 
 static inline unsigned blocks_for(size_t len, int bs = 256) { return unsigned((len + bs - 1) / bs); }
 // grid of the grid-stride reduction kernels: few enough blocks that the per-block arrival
