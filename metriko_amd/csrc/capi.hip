@@ -495,6 +495,7 @@ mk_status mk_finalize(mk_ctx* c) {
     c->partials.release();
     c->state.release();
     c->scal.release();
+    c->scratch.clear();
     if (c->pin) (void)hipHostFree(c->pin);
     c->pin = nullptr;
     if (c->stream) (void)hipStreamDestroy(c->stream);

@@ -16,7 +16,14 @@
 // The products are row-wise SpGEMMs, one wavefront per row with a hash table of the row in LDS: the
 // entries of the left row are taken in order, the lanes spread over the right row (whose columns are
 // distinct), so every sum has a fixed order; the finished row is written in column order.  Rows of
-// more than kMaxRow entries are reported and the level is smoothed instead.
+// more than kMaxRow entries are reported and the level is smoothed instead.  Counting uses a table of
+// kHash slots, filling one of kSmall where every row fits: a quarter of the clearing, collecting and LDS
+// (16 KB a block instead of 64, so ten blocks per compute unit instead of two): 62,307 complex rows of
+// 5, four products of up to 33 entries a row, 500 -> 110 us each.
+//
+// A first solve pays for all of this, so the temporaries are carved out of scratch that the context keeps
+// (allocating and freeing them took 3 of the 8.6 ms that 102,845 rows of 9 cost before): a first solve
+// of that operator 26.0 -> 20.9 ms, 21.1 with the level smoothed.
 #include "mk_internal.h"
 #include "sell.h"
 
@@ -24,8 +31,10 @@ namespace mk {
 
 namespace {
 
-constexpr int kHash = 1024;        // slots per row
+constexpr int kHash = 1024;           // slots per row
 constexpr int kMaxRow = kHash - 128;  // entries a row may have; a step adds at most 64 more
+constexpr int kSmall = 256;           // slots per row where no row has more than kSmallRow entries
+constexpr int kSmallRow = 192;
 
 struct CsrDev {
     const int64_t* ptr = nullptr;  // null: absent
@@ -46,11 +55,14 @@ struct SpProduct {
     const double* cs = nullptr;
 };
 
-__device__ __forceinline__ unsigned hash_of(int c) { return (unsigned(c) * 2654435761u) >> 22; }  // 10 bits
-static_assert(kHash == 1 << 10, "hash_of yields 10 bits");
+// the slot of a column in a table of H (a power of two) slots
+template <int H>
+__device__ __forceinline__ unsigned hash_of(int c) {
+    return (unsigned(c) * 2654435761u) >> (32 - __builtin_ctz(H));
+}
 
-// One row's table: keys, values (FILL) and the number of keys, of one wavefront.
-template <bool CPLX, bool FILL>
+// One row's table of H slots: keys, values (FILL) and the number of keys, of one wavefront.
+template <bool CPLX, bool FILL, int H>
 struct RowTable {
     static constexpr int W = CPLX ? 2 : 1;
     int* key;
@@ -58,9 +70,9 @@ struct RowTable {
     int* count;
     // value (vr, vi) at column c; lanes of one call hold distinct columns
     __device__ __forceinline__ void add(int c, double vr, double vi) const {
-        unsigned h = hash_of(c);
+        unsigned h = hash_of<H>(c);
         int old;
-        while ((old = atomicCAS(&key[h], -1, c)) != -1 && old != c) h = (h + 1) & (kHash - 1);
+        while ((old = atomicCAS(&key[h], -1, c)) != -1 && old != c) h = (h + 1) & (H - 1);
         if (old == -1) atomicAdd(count, 1);
         if constexpr (FILL) {
             if (old == -1) {
@@ -72,12 +84,13 @@ struct RowTable {
             }
         }
     }
-    // factor (fr, fi) times entries [b, e) of a CSR row; false when the row is too long
+    // factor (fr, fi) times entries [b, e) of a CSR row; false when the row is too long (counting only: a
+    // row that is filled fits)
     __device__ __forceinline__ bool add_row(const CsrDev& M, int64_t b, int64_t e, double fr, double fi, int lane) const {
         for (int64_t k0 = b; k0 < e; k0 += 64) {
             // one wavefront: its LDS operations are in order, so the count is up to date and leaves
             // room for 64 more keys
-            if (*static_cast<volatile int*>(count) > kMaxRow) return false;
+            if (!FILL && *static_cast<volatile int*>(count) > kMaxRow) return false;
             const int64_t k = k0 + lane;
             if (k < e) {
                 double vr = 0.0, vi = 0.0;
@@ -102,20 +115,20 @@ struct RowTable {
 
 // FILL = false: cnt[i] = entries of row i (overflow set when it has too many).  FILL = true: row i
 // in column order at optr[i] + (ooff ? ooff[i] : 0), columns shifted by cshift.
-template <bool CPLX, bool FILL>
+template <bool CPLX, bool FILL, int H>
 __global__ void __launch_bounds__(256) k_spgemm(SpProduct S, int* __restrict__ cnt, int* __restrict__ overflow,
                                                 const int64_t* __restrict__ optr, const int* __restrict__ ooff, int cshift,
                                                 int* __restrict__ ocol, double* __restrict__ oval) {
     constexpr int W = CPLX ? 2 : 1;
-    __shared__ int s_key[4][kHash];
-    __shared__ double s_val[FILL ? 4 : 1][FILL ? kHash * W : 1];
-    __shared__ int s_list[FILL ? 4 : 1][FILL ? kHash : 1];
+    __shared__ int s_key[4][H];
+    __shared__ double s_val[FILL ? 4 : 1][FILL ? H * W : 1];
+    __shared__ int s_list[FILL ? 4 : 1][FILL ? H : 1];
     __shared__ int s_count[4];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const int i = blockIdx.x * 4 + wid;
     if (i >= S.n) return;  // uniform inside the wavefront; nothing below synchronises the block
-    const RowTable<CPLX, FILL> t{s_key[wid], s_val[FILL ? wid : 0], &s_count[wid]};
-    for (int h = lane; h < kHash; h += 64) t.key[h] = -1;
+    const RowTable<CPLX, FILL, H> t{s_key[wid], s_val[FILL ? wid : 0], &s_count[wid]};
+    for (int h = lane; h < H; h += 64) t.key[h] = -1;
     if (lane == 0) s_count[wid] = 0;
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     bool ok = true;
@@ -142,7 +155,7 @@ __global__ void __launch_bounds__(256) k_spgemm(SpProduct S, int* __restrict__ c
         // occupied slots, then every key's rank among them
         int* list = s_list[wid];
         int base = 0;
-        for (int h = lane; h < kHash; h += 64) {
+        for (int h = lane; h < H; h += 64) {
             const bool used = t.key[h] >= 0;
             const unsigned long long b = __ballot(used);
             if (used) list[base + __popcll(b & ((1ull << lane) - 1))] = h;
@@ -161,25 +174,64 @@ __global__ void __launch_bounds__(256) k_spgemm(SpProduct S, int* __restrict__ c
     }
 }
 
-// ptr[0 .. n] = exclusive prefix sums of a (+ b): one block, each thread a contiguous share
+// ptr[0 .. n] = exclusive prefix sums of a (+ b), maxima[0], maxima[1] = the largest of a and of b: one block,
+// a tile of 4,096 rows at a time, four neighbouring rows a thread.  (With a contiguous share of the
+// whole per thread 62,307 rows took 209 us, this 55.)
 __global__ void __launch_bounds__(1024) k_scan(int n, const int* __restrict__ a, const int* __restrict__ b,
-                                               int64_t* __restrict__ ptr) {
-    __shared__ int64_t part[1024];
-    const int t = threadIdx.x, per = (n + 1023) / 1024;
-    const int i0 = min(n, t * per), i1 = min(n, i0 + per);
-    int64_t s = 0;
-    for (int i = i0; i < i1; i++) s += a[i] + (b ? b[i] : 0);
-    part[t] = s;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        const int64_t v = t >= off ? part[t - off] : 0;
+                                               int64_t* __restrict__ ptr, int* __restrict__ maxima) {
+    __shared__ int wsum[2][16];
+    __shared__ int smax[2][16];
+    const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+    int64_t base = 0;
+    int ma = 0, mb = 0;
+    int buf = 0;
+    for (int i0 = 0; i0 < n; i0 += 4096, buf ^= 1) {
+        int v[4], s = 0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int i = i0 + 4 * t + q;
+            const int x = i < n ? a[i] : 0, y = b && i < n ? b[i] : 0;
+            ma = max(ma, x);
+            mb = max(mb, y);
+            v[q] = x + y;
+            s += v[q];
+        }
+        int inc = s;  // inclusive sums over the wavefront (a tile holds fewer than 2^31 entries)
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int u = __shfl_up(inc, off, 64);
+            if (lane >= off) inc += u;
+        }
+        if (lane == 63) wsum[buf][wid] = inc;
         __syncthreads();
-        part[t] += v;
-        __syncthreads();
+        int before = 0, all = 0;
+#pragma unroll
+        for (int w = 0; w < 16; w++) {
+            if (w < wid) before += wsum[buf][w];
+            all += wsum[buf][w];
+        }
+        int64_t o = base + before + inc - s;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int i = i0 + 4 * t + q;
+            if (i < n) ptr[i] = o;
+            o += v[q];
+        }
+        base += all;
     }
-    s = t ? part[t - 1] : 0;
-    for (int i = i0; i < i1; i++) { ptr[i] = s; s += a[i] + (b ? b[i] : 0); }
-    if (t == 1023) ptr[n] = part[1023];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        ma = max(ma, __shfl_xor(ma, off, 64));
+        mb = max(mb, __shfl_xor(mb, off, 64));
+    }
+    if (lane == 0) { smax[0][wid] = ma; smax[1][wid] = mb; }
+    __syncthreads();
+    if (t == 0) {
+        for (int w = 1; w < 16; w++) { ma = max(ma, smax[0][w]); mb = max(mb, smax[1][w]); }
+        ptr[n] = base;
+        maxima[0] = ma;
+        maxima[1] = mb;
+    }
 }
 
 // y = diag(d) x (rows != 0) or x diag(d), on the values of a CSR matrix: one wavefront per row
@@ -204,61 +256,111 @@ __global__ void k_round32(size_t n, const double* __restrict__ x, float* __restr
 }
 inline unsigned nb(size_t n) { return unsigned((n + 255) / 256); }
 
-// a CSR matrix on the device
+// Temporaries of one set-up, carved out of the context's scratch chunks in order.  The context keeps up to
+// kKeep of them for the next set-up (its stream runs the two one after the other) until it ends.
+struct Scratch {
+    static constexpr size_t kChunk = size_t(32) << 20, kKeep = size_t(256) << 20;
+    mk_ctx* c;
+    size_t k = 0, off = 0;
+    explicit Scratch(mk_ctx* c_) : c(c_) {}
+    Scratch(const Scratch&) = delete;
+    ~Scratch() {
+        size_t held = 0;
+        for (size_t q = 0; q < c->scratch.size();) {
+            if (held + c->scratch[q].n <= kKeep) held += c->scratch[q++].n;
+            else c->scratch.erase(c->scratch.begin() + std::ptrdiff_t(q));
+        }
+    }
+    template <typename T>
+    T* get(size_t count) {
+        const size_t bytes = (std::max<size_t>(count, 1) * sizeof(T) + 255) / 256 * 256;
+        while (k < c->scratch.size() && off + bytes > c->scratch[k].n) { k++; off = 0; }
+        if (k == c->scratch.size()) c->scratch.emplace_back(std::max(bytes, kChunk));
+        T* p = reinterpret_cast<T*>(c->scratch[k].p + off);
+        off += bytes;
+        return p;
+    }
+};
+
+// a CSR matrix on the device that the caller keeps
 struct DevCsr {
     DevBuf<int64_t> ptr;
     DevBuf<int> col;
     DevBuf<double> val;
-    CsrDev view() const { return {ptr.p, col.p, val.p}; }
 };
+// entries of a product and of its longest row; nz < 0: a row was too long
+struct Size { int64_t nz; int longest, longest_b; };
 
 struct Builder {
     mk_ctx* c;
     bool cplx;
-    DevBuf<int> overflow;
-    Builder(mk_ctx* c_, bool cplx_) : c(c_), cplx(cplx_), overflow(1) {
-        MK_HIP(hipMemsetAsync(overflow.p, 0, sizeof(int), c->stream));
+    Scratch& tmp;
+    int* overflow;
+    Builder(mk_ctx* c_, bool cplx_, Scratch& t) : c(c_), cplx(cplx_), tmp(t), overflow(t.get<int>(1)) {
+        MK_HIP(hipMemsetAsync(overflow, 0, sizeof(int), c->stream));
     }
-    DevCsr upload(const HostCsr& A) const {
-        DevCsr d;
-        const size_t nz = size_t(A.ptr[A.rows]);
-        d.ptr.upload(A.ptr, size_t(A.rows) + 1, c->stream);
-        d.col.upload(A.col, std::max<size_t>(nz, 1), c->stream);
-        d.val.upload(A.val, std::max<size_t>(nz, 1) * (cplx ? 2 : 1), c->stream);
+    template <typename T>
+    const T* upload(const T* h, size_t n) const {
+        T* d = tmp.get<T>(n);
+        if (n) MK_HIP(hipMemcpyAsync(d, h, n * sizeof(T), hipMemcpyHostToDevice, c->stream));
         return d;
     }
-    void count(const SpProduct& S, DevBuf<int>& cnt) const {
-        cnt.alloc(size_t(std::max(S.n, 1)));
-        const dim3 g(unsigned((S.n + 3) / 4));
-        if (cplx) hipLaunchKernelGGL((k_spgemm<true, false>), g, dim3(256), 0, c->stream, S, cnt.p, overflow.p, nullptr, nullptr, 0, nullptr, nullptr);
-        else hipLaunchKernelGGL((k_spgemm<false, false>), g, dim3(256), 0, c->stream, S, cnt.p, overflow.p, nullptr, nullptr, 0, nullptr, nullptr);
-        MK_HIP(hipGetLastError());
+    CsrDev upload(const HostCsr& A) const {
+        const size_t nz = size_t(A.ptr[A.rows]);
+        return {upload(A.ptr, size_t(A.rows) + 1), upload(A.col, nz), upload(A.val, nz * (cplx ? 2 : 1))};
     }
-    // row pointers from the counts; their total, or -1 when a row was too long
-    int64_t scan(int n, const DevBuf<int>& a, const int* b, DevBuf<int64_t>& ptr) const {
-        ptr.alloc(size_t(n) + 1);
-        hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, c->stream, n, (const int*)a.p, b, ptr.p);
+    int* count(const SpProduct& S) const {
+        int* cnt = tmp.get<int>(size_t(S.n));
+        const dim3 g(unsigned((S.n + 3) / 4));
+#define MK_COUNT(CP)                                                                                                \
+    hipLaunchKernelGGL((k_spgemm<CP, false, kHash>), g, dim3(256), 0, c->stream, S, cnt, overflow, nullptr, nullptr, \
+                       0, nullptr, nullptr)
+        if (cplx) MK_COUNT(true);
+        else MK_COUNT(false);
+#undef MK_COUNT
+        MK_HIP(hipGetLastError());
+        return cnt;
+    }
+    // row pointers from the counts a (+ b)
+    Size scan(int n, const int* a, const int* b, int64_t* ptr) const {
+        int* found = tmp.get<int>(2);
+        hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, c->stream, n, a, b, ptr, found);
         int64_t* h = static_cast<int64_t*>(c->pin);
-        MK_HIP(hipMemcpyAsync(h, ptr.p + n, sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
-        MK_HIP(hipMemcpyAsync(h + 1, overflow.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+        int* hi = reinterpret_cast<int*>(h + 1);
+        MK_HIP(hipMemcpyAsync(h, ptr + n, sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
+        MK_HIP(hipMemcpyAsync(hi, found, 2 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+        MK_HIP(hipMemcpyAsync(hi + 2, overflow, sizeof(int), hipMemcpyDeviceToHost, c->stream));
         MK_HIP(hipStreamSynchronize(c->stream));
-        return *reinterpret_cast<const int*>(h + 1) ? -1 : h[0];
+        return {hi[2] ? -1 : *h, hi[0], hi[1]};
     }
-    void fill(const SpProduct& S, const int64_t* optr, const int* ooff, int cshift, int* ocol, double* oval) const {
+    // longest: the longest row's entries
+    void fill(const SpProduct& S, int longest, const int64_t* optr, const int* ooff, int cshift, int* ocol,
+              double* oval) const {
         const dim3 g(unsigned((S.n + 3) / 4));
-        if (cplx) hipLaunchKernelGGL((k_spgemm<true, true>), g, dim3(256), 0, c->stream, S, nullptr, nullptr, optr, ooff, cshift, ocol, oval);
-        else hipLaunchKernelGGL((k_spgemm<false, true>), g, dim3(256), 0, c->stream, S, nullptr, nullptr, optr, ooff, cshift, ocol, oval);
+#define MK_FILL(CP, H)                                                                                            \
+    hipLaunchKernelGGL((k_spgemm<CP, true, H>), g, dim3(256), 0, c->stream, S, nullptr, nullptr, optr, ooff, cshift, \
+                       ocol, oval)
+        const bool small = longest <= kSmallRow;
+        if (cplx) { if (small) MK_FILL(true, kSmall); else MK_FILL(true, kHash); }
+        else { if (small) MK_FILL(false, kSmall); else MK_FILL(false, kHash); }
+#undef MK_FILL
         MK_HIP(hipGetLastError());
     }
-    bool product(const SpProduct& S, DevCsr& out) const {
-        DevBuf<int> cnt;
-        count(S, cnt);
-        const int64_t nz = scan(S.n, cnt, nullptr, out.ptr);
-        if (nz < 0) return false;
+    // false: a row was too long
+    bool product(const SpProduct& S, CsrDev& out) const {
+        const int* cnt = count(S);
+        int64_t* ptr = tmp.get<int64_t>(size_t(S.n) + 1);
+        const Size z = scan(S.n, cnt, nullptr, ptr);
+        if (z.nz < 0) return false;
+        int* col = tmp.get<int>(size_t(z.nz));
+        double* val = tmp.get<double>(size_t(z.nz) * (cplx ? 2 : 1));
+        fill(S, z.longest, ptr, nullptr, 0, col, val);
+        out = {ptr, col, val};
+        return true;
+    }
+    void alloc(DevCsr& out, int64_t nz) const {
         out.col.alloc(size_t(std::max<int64_t>(nz, 1)));
         out.val.alloc(size_t(std::max<int64_t>(nz, 1)) * (cplx ? 2 : 1));
-        fill(S, out.ptr.p, nullptr, 0, out.col.p, out.val.p);
-        return true;
     }
     // an operator of medium rows only, taking over its CSR arrays
     mk_op* op(int rows, int cols, int64_t nz, DevBuf<int64_t>&& ptr, DevBuf<int>&& col, DevBuf<double>&& val, int block) const {
@@ -299,43 +401,49 @@ struct Builder {
 
 bool explicit_level(mk_ctx* c, bool cplx, const HostCsr& hA, const HostCsr& hP, const HostCsr& hR, const double* dinv,
                     double alpha, double beta, double max_bytes, int block, mk_op** W, mk_op** M) {
-    const Builder b(c, cplx);
+    Scratch tmp(c);
+    const Builder b(c, cplx, tmp);
     const int n = hA.rows, nc = hR.rows;
-    const DevCsr A = b.upload(hA), P = b.upload(hP), R = b.upload(hR);
-    DevBuf<double> D, vB(A.val.n), vG(A.val.n);
-    D.upload(dinv, size_t(n), c->stream);
-    const CsrDev a = A.view(), B{a.ptr, a.col, vB.p}, G{a.ptr, a.col, vG.p};  // B = D^-1 A, G = A D^-1
+    const CsrDev a = b.upload(hA), P = b.upload(hP), R = b.upload(hR);
+    const double* D = b.upload(dinv, size_t(n));
+    // B = D^-1 A, G = A D^-1
+    const size_t len = size_t(hA.ptr[n]) * (cplx ? 2 : 1);
+    double *vB = tmp.get<double>(len), *vG = tmp.get<double>(len);
+    const CsrDev B{a.ptr, a.col, vB}, G{a.ptr, a.col, vG};
     const dim3 g(unsigned((n + 3) / 4));
     for (int rows = 0; rows < 2; rows++) {
-        double* out = rows ? vB.p : vG.p;
-        if (cplx) hipLaunchKernelGGL((k_scale<true>), g, dim3(256), 0, c->stream, n, a, (const double*)D.p, rows, out);
-        else hipLaunchKernelGGL((k_scale<false>), g, dim3(256), 0, c->stream, n, a, (const double*)D.p, rows, out);
+        double* out = rows ? vB : vG;
+        if (cplx) hipLaunchKernelGGL((k_scale<true>), g, dim3(256), 0, c->stream, n, a, D, rows, out);
+        else hipLaunchKernelGGL((k_scale<false>), g, dim3(256), 0, c->stream, n, a, D, rows, out);
     }
     MK_HIP(hipGetLastError());
-    DevCsr X, Wc, Q, U;
+    CsrDev X, Q, U;
     // T = (2 alpha I - (2 beta + alpha^2) B + 2 alpha beta B^2 - beta^2 B^3) D^-1, by Horner;
     // V = (I - alpha B + beta B^2) P; M = [T | V]
     if (!b.product({n, -beta * beta, B, B, 2.0 * alpha * beta, B, 0.0, {}, -(2.0 * beta + alpha * alpha)}, Q)) return false;
-    if (!b.product({n, 1.0, B, P.view()}, U)) return false;
-    const SpProduct T{n, 1.0, B, Q.view(), 0.0, {}, 0.0, {}, 2.0 * alpha, D.p};
-    const SpProduct V{n, beta, B, U.view(), -alpha, U.view(), 1.0, P.view()};
-    DevBuf<int> cT, cV;
-    b.count(T, cT);
-    b.count(V, cV);
-    DevCsr Mc;
-    const int64_t nz = b.scan(n, cT, cV.p, Mc.ptr);
-    if (nz < 0 || double(nz) * (cplx ? 12.0 : 8.0) > max_bytes) return false;
+    if (!b.product({n, 1.0, B, P}, U)) return false;
+    const SpProduct T{n, 1.0, B, Q, 0.0, {}, 0.0, {}, 2.0 * alpha, D};
+    const SpProduct V{n, beta, B, U, -alpha, U, 1.0, P};
+    const int *cT = b.count(T), *cV = b.count(V);
+    DevCsr Wc, Mc;
+    Mc.ptr.alloc(size_t(n) + 1);
+    const Size m = b.scan(n, cT, cV, Mc.ptr.p);
+    if (m.nz < 0 || double(m.nz) * (cplx ? 12.0 : 8.0) > max_bytes) return false;
     // W = R (I - alpha G + beta G^2)
-    if (!b.product({nc, 1.0, R.view(), G}, X)) return false;
-    if (!b.product({nc, beta, X.view(), G, -alpha, X.view(), 1.0, R.view()}, Wc)) return false;
-    Mc.col.alloc(size_t(std::max<int64_t>(nz, 1)));
-    Mc.val.alloc(size_t(std::max<int64_t>(nz, 1)) * (cplx ? 2 : 1));
-    b.fill(T, Mc.ptr.p, nullptr, 0, Mc.col.p, Mc.val.p);
-    b.fill(V, Mc.ptr.p, cT.p, n, Mc.col.p, Mc.val.p);
-    const int64_t wz = int64_t(Wc.col.n);
-    *W = b.op(nc, n, wz, std::move(Wc.ptr), std::move(Wc.col), std::move(Wc.val), block);
-    *M = b.op(n, n + nc, nz, std::move(Mc.ptr), std::move(Mc.col), std::move(Mc.val), block);
-    MK_HIP(hipStreamSynchronize(c->stream));  // the temporaries are freed on return
+    if (!b.product({nc, 1.0, R, G}, X)) return false;
+    const SpProduct Wp{nc, beta, X, G, -alpha, X, 1.0, R};
+    const int* cW = b.count(Wp);
+    Wc.ptr.alloc(size_t(nc) + 1);
+    const Size w = b.scan(nc, cW, nullptr, Wc.ptr.p);
+    if (w.nz < 0) return false;
+    b.alloc(Wc, w.nz);
+    b.alloc(Mc, m.nz);
+    b.fill(Wp, w.longest, Wc.ptr.p, nullptr, 0, Wc.col.p, Wc.val.p);
+    b.fill(T, m.longest, Mc.ptr.p, nullptr, 0, Mc.col.p, Mc.val.p);
+    b.fill(V, m.longest_b, Mc.ptr.p, cT, n, Mc.col.p, Mc.val.p);
+    *W = b.op(nc, n, w.nz, std::move(Wc.ptr), std::move(Wc.col), std::move(Wc.val), block);
+    *M = b.op(n, n + nc, m.nz, std::move(Mc.ptr), std::move(Mc.col), std::move(Mc.val), block);
+    MK_HIP(hipStreamSynchronize(c->stream));  // the host arrays and the scratch may go
     return true;
 }
 

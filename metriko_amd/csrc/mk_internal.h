@@ -257,6 +257,7 @@ struct mk_ctx {
     mk::DevBuf<double> partials;
     mk::DevBuf<mk::CgState> state;
     mk::DevBuf<double> scal;   // general device scalars
+    std::vector<mk::DevBuf<char>> scratch;  // kept chunks of set-up temporaries (explicit.hip: at most 256 MiB)
     void* pin = nullptr;       // page-locked host memory the solvers' states are read back into
     static constexpr size_t kPinBytes = 8192;
     // behind it: whether the running solve's start meets the tolerance (-1: not known yet), which the

@@ -136,3 +136,36 @@ def test_which_finest_levels_are_explicit(gpu_ctx, what, explicit):
             gpu_ctx.set_timing(False)
         assert (f"op_mg0_M:cheb_level:{tag}" in keys) == explicit, keys
         assert any(k.startswith("op_mg0:cheb") and k.endswith(tag) for k in keys) != explicit, keys
+
+
+def _band(n, w):
+    """Half-width w: T has 6 w + 1 entries a row (three steps), four strong couplings on either side."""
+    v = {d: -0.1 if d <= 4 else -0.1 / (w - 4) for d in range(1, w + 1)}
+    S = sp.diags([np.full(n - abs(d), v[abs(d)]) for d in range(-w, w + 1) if d], [d for d in range(-w, w + 1) if d])
+    return sp.csr_matrix(S - sp.diags(np.asarray(S.sum(axis=1)).ravel()) + 0.05 * sp.identity(n))
+
+
+# rows of 169, 187 | 193, 361 and 841: on both sides of the small table (192) and up to the largest
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("w", [28, 31, 32, 60, 140])
+def test_v_cycle_of_the_tables(gpu_ctx, w, cplx):
+    n = 2999
+    rng = np.random.default_rng(w)
+    A = _band(n, w)
+    b = rng.standard_normal(n) + (1j * rng.standard_normal(n) if cplx else 0.0)
+    if cplx:
+        G = sp.diags(np.exp(2j * np.pi * rng.random(n)))
+        A = sp.csr_matrix(G @ A @ G.getH())
+    op = gpu_ctx.op_complex(A) if cplx else gpu_ctx.op_real(A)
+    z, _, levels, _ = mk.mg_host_pcg(A, b, maxit=0)
+    for precision, tol, tag in ((mk.PREC_FP64, 1e-12, "fp64"), (mk.PREC_MIXED_MG, 1e-5, "fp32")):
+        try:
+            gpu_ctx.set_timing(True)
+            gpu_ctx.timing_report(reset=True)
+            x, dev_levels = _first_step(gpu_ctx, op, b, mk.opts(precision=precision, maxiter=1))
+            keys = {k["key"] for k in gpu_ctx.timing_report(reset=True)}
+        finally:
+            gpu_ctx.set_timing(False)
+        assert levels == dev_levels == 2 and f"op_mg0_M:cheb_level:{tag}" in keys
+        c = np.vdot(z, x) / np.vdot(z, z)
+        assert np.linalg.norm(x - c * z) <= tol * np.linalg.norm(x), precision
